@@ -70,19 +70,9 @@ __device__ __forceinline__ uint64_t morton63(float x, float y, float z) {
     return spread_bits21((uint64_t)x) * 4u + spread_bits21((uint64_t)y) * 2u + spread_bits21((uint64_t)z);
 }
 
-// Leaf boxes (build_bvh.cu:212-219, :452-460), the triangle ids in input order and, for the
-// fitted modes, the centroids the Morton codes are computed from (build_bvh.cu:26-71).
-// The reference's scene box is the union of all leaf boxes with the reduction's initial
-// value AABB<T>() = [-MAX, +MAX] (build_bvh.cu:243-244, :505-506; aabb.cu:25-33); min/max
-// against +-MAX leave that initial value unchanged whatever the boxes are, so the scene box
-// is [-MAX, +MAX], every normalised centroid is ~0.5 * 2^-1023 or smaller and every code is
-// 0: the stable sort then keeps the input order, and the compat mode writes no codes.
-template <typename T, bool MOTION, bool FIT>
-__global__ void k_leaf_boxes(const T *__restrict__ t0, const T *__restrict__ t1, int64_t total,
-                             int64_t n, T *__restrict__ boxes, T *__restrict__ cent,
-                             int32_t *__restrict__ ids) {
-    int64_t gi = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (gi >= total) return;
+// The box of triangle gi (build_bvh.cu:212-219, :452-460): of t0, or of t0 and t1 (MOTION).
+template <typename T, bool MOTION>
+__device__ __forceinline__ Box<T> leaf_box(const T *__restrict__ t0, const T *__restrict__ t1, int64_t gi, V3<T> *cent) {
     const T *a = t0 + 9 * gi;
     V3<T> a0 = ld3(a), a1 = ld3(a + 3), a2 = ld3(a + 6);
     Box<T> bx = tri_box(a0, a1, a2);
@@ -94,12 +84,30 @@ __global__ void k_leaf_boxes(const T *__restrict__ t0, const T *__restrict__ t1,
         V3<T> c2 = mk((b0.x + b1.x + b2.x) / (T)3.0, (b0.y + b1.y + b2.y) / (T)3.0, (b0.z + b1.z + b2.z) / (T)3.0);
         c = mk((c.x + c2.x) / (T)2.0, (c.y + c2.y) / (T)2.0, (c.z + c2.z) / (T)2.0);
     }
+    if (cent) *cent = c;
+    return bx;
+}
+
+// Fitted modes: leaf boxes, the triangle ids in input order and the centroids the Morton
+// codes are computed from (build_bvh.cu:26-71).
+// The reference's scene box is the union of all leaf boxes with the reduction's initial
+// value AABB<T>() = [-MAX, +MAX] (build_bvh.cu:243-244, :505-506; aabb.cu:25-33); min/max
+// against +-MAX leave that initial value unchanged whatever the boxes are, so the scene box
+// is [-MAX, +MAX], every normalised centroid is ~0.5 * 2^-1023 or smaller and every code is
+// 0: the stable sort then keeps the input order, and the compat mode needs neither codes nor
+// a sort (k_index_leaves).
+template <typename T, bool MOTION>
+__global__ void k_leaf_boxes(const T *__restrict__ t0, const T *__restrict__ t1, int64_t total,
+                             int64_t n, T *__restrict__ boxes, T *__restrict__ cent,
+                             int32_t *__restrict__ ids) {
+    int64_t gi = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (gi >= total) return;
+    V3<T> c;
+    const Box<T> bx = leaf_box<T, MOTION>(t0, t1, gi, &c);
     T *o = boxes + 6 * gi;
     o[0] = bx.mn.x; o[1] = bx.mn.y; o[2] = bx.mn.z; o[3] = bx.mx.x; o[4] = bx.mx.y; o[5] = bx.mx.z;
-    if (FIT) {
-        T *q = cent + 3 * gi;
-        q[0] = c.x; q[1] = c.y; q[2] = c.z;
-    }
+    T *q = cent + 3 * gi;
+    q[0] = c.x; q[1] = c.y; q[2] = c.z;
     ids[gi] = (int32_t)(gi % n);
 }
 
@@ -263,7 +271,6 @@ __global__ __launch_bounds__(kSortThreads) void k_sort_scatter(const K *__restri
 // ---- Karras radix tree ----------------------------------------------------------------------
 // bvh.cu:70-89 LongestCommonPrefix: -1 outside [0, n-1]; equal codes extend the prefix with
 // the ids' common prefix (32 + clz(id_i ^ id_j) for 32-bit keys, 64 + ... for 64-bit ones).
-// codes == NULL: every code is 0 (the reference's scene box), only the ids decide.
 template <typename K> __device__ __forceinline__ int clz_key(K x);
 template <> __device__ __forceinline__ int clz_key<uint32_t>(uint32_t x) { return __clz((int)x); }
 template <> __device__ __forceinline__ int clz_key<uint64_t>(uint64_t x) { return __clzll((long long)x); }
@@ -271,10 +278,8 @@ template <> __device__ __forceinline__ int clz_key<uint64_t>(uint64_t x) { retur
 template <typename K>
 __device__ __forceinline__ int lcp_delta(const K *codes, const int32_t *ids, int64_t n, int64_t i, int64_t j) {
     if (j < 0 || j > n - 1) return -1;
-    if (codes) {
-        const K a = codes[i], c = codes[j];
-        if (a != c) return clz_key<K>(a ^ c);
-    }
+    const K a = codes[i], c = codes[j];
+    if (a != c) return clz_key<K>(a ^ c);
     return 8 * (int)sizeof(K) + __clz((int)((uint32_t)ids[i] ^ (uint32_t)ids[j]));
 }
 
@@ -287,7 +292,7 @@ __global__ void k_karras(const K *__restrict__ codes_all, const int32_t *__restr
     const int b = blockIdx.y;
     const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= n - 1) return;
-    const K *codes = codes_all ? codes_all + (int64_t)b * n : nullptr;
+    const K *codes = codes_all + (int64_t)b * n;
     const int32_t *ids = ids_all + (int64_t)b * n;
     int64_t *tree = tree_all + (int64_t)b * (2 * n - 1) * 4;
     int2 *range = range_all + (int64_t)b * (n - 1);
@@ -319,63 +324,212 @@ __global__ void k_karras(const K *__restrict__ codes_all, const int32_t *__restr
     range[i] = make_int2((int)lo, (int)hi);
 }
 
-// Node boxes (build_bvh.cu:145-209 computes them by an atomic bottom-up climb).  Every
+// ---- node boxes -----------------------------------------------------------------------------
+// The reference computes them by an atomic bottom-up climb (build_bvh.cu:145-209).  Every
 // internal node of the Karras tree covers a contiguous range [lo, hi] of sorted leaf
-// positions, so its box is the union of the leaf boxes of that range.  Min / max are exact
-// and order-independent, so any grouping gives the climb's result; here the union is read
-// off a hierarchy of chunk boxes (64, 64^2, ... leaves), with no atomics or fences.
+// positions, so its box is the union of the leaf boxes of that range; min / max are exact and
+// order-independent, so any grouping gives the climb's result, with no atomics or fences.
+// Positions are grouped in chunks of 64, one per lane of a wave, whose unions come from lane
+// exchanges.  (One thread per chunk, walking its 64 boxes one after the other, was bound by
+// the latency of that chain: 12-22 us per level, and as much again for the nodes' own walks.)
 constexpr int kChunkBits = 6;
 constexpr int kChunk = 1 << kChunkBits;
 constexpr int kChunkLevels = 5;      // 64^5 = 2^30 > 2^28 leaves
 
-// Leaf rows (build_bvh.cu:309-378 layout): the box of triangle ids[p] and (-1, -1, id).
+template <typename T> struct BoxReg { T v[6]; };   // min xyz, max xyz
+
+template <typename T> __device__ __forceinline__ BoxReg<T> load_box(const T *p) {
+    BoxReg<T> r;
+#pragma unroll
+    for (int k = 0; k < 6; ++k) r.v[k] = p[k];
+    return r;
+}
+template <typename T> __device__ __forceinline__ void store_box(T *p, const BoxReg<T> &r) {
+#pragma unroll
+    for (int k = 0; k < 6; ++k) p[k] = r.v[k];
+}
+template <typename T> __device__ __forceinline__ void box_join(BoxReg<T> &a, const BoxReg<T> &b) {
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+        a.v[k] = tmin(a.v[k], b.v[k]);
+        a.v[k + 3] = tmax(a.v[k + 3], b.v[k + 3]);
+    }
+}
+// the union over lanes l and l ^ d
+template <typename T> __device__ __forceinline__ void box_join_xor(BoxReg<T> &a, int d) {
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+        a.v[k] = tmin(a.v[k], __shfl_xor(a.v[k], d, 64));
+        a.v[k + 3] = tmax(a.v[k + 3], __shfl_xor(a.v[k + 3], d, 64));
+    }
+}
+
+// The compat tree is the radix tree over leaf indices (every code is 0).  Node i covers the
+// aligned block of 2^k leaves that starts at i (i even, k = trailing zeros of i) or ends at i
+// (i odd, k = trailing zeros of i + 1), cut off at n; node 0 covers everything.  That is
+// Karras' Algorithm 1 (k_karras below) with delta(i, j) = 32 + clz(i ^ j) solved in closed
+// form: the direction and range follow from i's neighbours, and the split is at the highest
+// differing bit of the range's ends.
+__device__ __forceinline__ int index_node_level(int64_t i) { return __ffsll((long long)((i & 1) ? i + 1 : i)) - 1; }
+
+__device__ __forceinline__ void index_node_row(int64_t i, int64_t n, int64_t &left, int64_t &right) {
+    int64_t lo = 0, hi = n - 1;
+    if (i > 0) {
+        const int64_t len = (int64_t)1 << index_node_level(i);
+        lo = (i & 1) ? i + 1 - len : i;
+        hi = (i & 1) ? i : (i + len <= n ? i + len - 1 : n - 1);
+    }
+    const int bit = 63 - __clzll((long long)(lo ^ hi));
+    const int64_t split = ((hi >> bit) << bit) - 1;
+    left = lo == split ? n - 1 + split : split;
+    right = hi == split + 1 ? n - 1 + split + 1 : split + 1;
+}
+
+// Writes the boxes of the nodes that end at this level: `box` is the union over lane's leaf
+// or chunk, unit `c` of `count` units of 2^shift leaves each; a unit's node is the one whose
+// aligned block starts at its first leaf (c even) or ends at its last (c odd).  Lanes past
+// the end hold a copy of the last unit's box, which changes no union.  Returns the union of
+// the wave's 64 units.
 template <typename T>
-__global__ void k_leaf_rows(const T *__restrict__ boxes_all, const int32_t *__restrict__ ids_all, int64_t n,
-                            T *__restrict__ bboxes_all, int64_t *__restrict__ tree_all) {
+__device__ __forceinline__ BoxReg<T> index_nodes_of_wave(BoxReg<T> box, int64_t c, int64_t count, int shift, int64_t n, T *bb) {
+    const int64_t i = (c & 1) ? ((c + 1) << shift) - 1 : c << shift;
+    // unit 0's node is the root, which the top level writes
+    const int k = c > 0 ? index_node_level(c) : kChunkBits + 1;
+    const bool mine = c < count && i < n - 1;
+    BoxReg<T> out = box;
+#pragma unroll
+    for (int l = 1; l <= kChunkBits; ++l) {
+        box_join_xor(box, 1 << (l - 1));
+        if (k == l) out = box;
+    }
+    if (mine && c == 0 && count <= kChunk) store_box(bb, box);
+    else if (mine && k <= kChunkBits) store_box(bb + 6 * i, out);
+    return box;
+}
+
+// Compat mode, first level: leaf boxes, leaf rows, the tree's internal rows (wire layout of
+// build_bvh.cu:309-378), the boxes of all nodes of up to 64 leaves and each chunk's box, one
+// wave per chunk, in one launch.  Bound by its reads and writes (226 B per fp64 triangle with
+// motion); it stands in for five launches (boxes, tree, rows, chunks, nodes) that took 60-110
+// us per build, nearly all of it latency, from 450 to 130k triangles.
+template <typename T, bool MOTION>
+__global__ __launch_bounds__(256) void k_index_leaves(const T *__restrict__ t0, const T *__restrict__ t1, int64_t n,
+                                                      T *__restrict__ bboxes_all, int64_t *__restrict__ tree_all,
+                                                      T *__restrict__ chunk_all, int64_t chunk_stride) {
     const int b = blockIdx.y;
     const int64_t p = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (p >= n) return;
+    if ((p & ~(int64_t)(kChunk - 1)) >= n) return;      // the whole wave is past the end
     const int64_t rows = 2 * n - 1;
-    const T *boxes = boxes_all + (int64_t)b * n * 6;
     T *bb = bboxes_all + (int64_t)b * rows * 6;
     int64_t *tree = tree_all + (int64_t)b * rows * 4;
-    const int64_t row = n - 1 + p;
-    const int32_t id = ids_all[(int64_t)b * n + p];
-#pragma unroll
-    for (int k = 0; k < 6; ++k) bb[6 * row + k] = boxes[6 * (int64_t)id + k];
-    if (n == 1) tree[4 * row + 0] = -1;
-    tree[4 * row + 1] = -1;
-    tree[4 * row + 2] = -1;
-    tree[4 * row + 3] = id;
+    const Box<T> bx = leaf_box<T, MOTION>(t0, t1, (int64_t)b * n + (p < n ? p : n - 1), (V3<T> *)nullptr);
+    const BoxReg<T> box{{bx.mn.x, bx.mn.y, bx.mn.z, bx.mx.x, bx.mx.y, bx.mx.z}};
+    if (p < n) {
+        const int64_t row = n - 1 + p;
+        store_box(bb + 6 * row, box);
+        if (n == 1) tree[4 * row] = -1;
+        tree[4 * row + 1] = -1;
+        tree[4 * row + 2] = -1;
+        tree[4 * row + 3] = p;
+    }
+    if (p < n - 1) {
+        int64_t left, right;
+        index_node_row(p, n, left, right);
+        if (p == 0) tree[0] = -1;
+        tree[4 * p + 1] = left;
+        tree[4 * p + 2] = right;
+        tree[4 * p + 3] = -1;
+        tree[4 * left] = p;
+        tree[4 * right] = p;
+    }
+    if (n == 1) return;
+    const BoxReg<T> all = index_nodes_of_wave(box, p, n, 0, n, bb);
+    if (chunk_all && (threadIdx.x & 63) == 0) store_box(chunk_all + (int64_t)b * chunk_stride + 6 * (p >> kChunkBits), all);
 }
 
-template <typename T> __device__ __forceinline__ void box_union_into(T *acc, const T *src) {
-    acc[0] = tmin(acc[0], src[0]);
-    acc[1] = tmin(acc[1], src[1]);
-    acc[2] = tmin(acc[2], src[2]);
-    acc[3] = tmax(acc[3], src[3]);
-    acc[4] = tmax(acc[4], src[4]);
-    acc[5] = tmax(acc[5], src[5]);
-}
-
-// chunk level L box c = union of the (at most 64) level L-1 boxes 64c .. 64c+63; level 0 is
-// the leaf rows of bboxes.
+// Compat mode, further levels: `count` units of 2^shift leaves, one per lane.
 template <typename T>
-__global__ void k_chunk_boxes(const T *__restrict__ src_all, int64_t src_stride, int64_t src_count, T *__restrict__ dst_all,
-                              int64_t dst_stride, int64_t dst_count) {
+__global__ __launch_bounds__(256) void k_index_nodes(const T *__restrict__ src_all, int64_t src_stride, int64_t count, int shift, int64_t n,
+                                                     T *__restrict__ bboxes_all, T *__restrict__ dst_all, int64_t dst_stride) {
     const int b = blockIdx.y;
     const int64_t c = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (c >= dst_count) return;
-    const T *src = src_all + (int64_t)b * src_stride;
-    T acc[6];
-    const int64_t first = c << kChunkBits;
-    const int64_t last = first + kChunk < src_count ? first + kChunk : src_count;
+    if ((c & ~(int64_t)(kChunk - 1)) >= count) return;
+    const BoxReg<T> box = load_box(src_all + (int64_t)b * src_stride + 6 * (c < count ? c : count - 1));
+    const BoxReg<T> all = index_nodes_of_wave(box, c, count, shift, n, bboxes_all + (int64_t)b * (2 * n - 1) * 6);
+    if (dst_all && (threadIdx.x & 63) == 0) store_box(dst_all + (int64_t)b * dst_stride + 6 * (c >> kChunkBits), all);
+}
+
+// Fitted modes: leaf rows in sorted order (the box of triangle ids[p] and (-1, -1, id)), each
+// chunk's box and the boxes of the nodes whose range lies within a chunk, one wave per chunk.
+// For those, level l of a table in LDS holds the unions over [p, p + 2^l), one coordinate at a
+// time; a range is the union of the two table entries that cover it.
+template <typename T>
+__global__ __launch_bounds__(256) void k_sorted_leaves(const T *__restrict__ boxes_all, const int32_t *__restrict__ ids_all, int64_t n,
+                                                       const int2 *__restrict__ range_all, T *__restrict__ bboxes_all,
+                                                       int64_t *__restrict__ tree_all, T *__restrict__ chunk_all, int64_t chunk_stride) {
+    __shared__ T s_tab[256 / kChunk][kChunkBits][kChunk];
+    const int b = blockIdx.y, lane = threadIdx.x & 63;
+    const int64_t p = (int64_t)blockIdx.x * blockDim.x + threadIdx.x, first = p - lane;
+    if (first >= n) return;
+    const int64_t rows = 2 * n - 1, at = p < n ? p : n - 1;
+    T *bb = bboxes_all + (int64_t)b * rows * 6;
+    int64_t *tree = tree_all + (int64_t)b * rows * 4;
+    T(*tab)[kChunk] = s_tab[threadIdx.x >> 6];
+    const int32_t id = ids_all[(int64_t)b * n + at];
+    const BoxReg<T> box = load_box(boxes_all + ((int64_t)b * n + id) * 6);
+    if (p < n) {
+        const int64_t row = n - 1 + p;
+        store_box(bb + 6 * row, box);
+        if (n == 1) tree[4 * row] = -1;
+        tree[4 * row + 1] = -1;
+        tree[4 * row + 2] = -1;
+        tree[4 * row + 3] = id;
+    }
+    int lo = 0, hi = 0;
+    bool mine = false;
+    if (p < n - 1) {
+        const int2 r = range_all[(int64_t)b * (n - 1) + p];
+        mine = r.x >= first && r.y < first + kChunk;
+        if (mine) { lo = (int)(r.x - first); hi = (int)(r.y - first); }
+    }
+    const int level = 31 - __clz(hi - lo + 1);      // 2^level <= length; at most 6: the whole chunk
+    const int l = level < kChunkBits ? level : kChunkBits - 1;
+    BoxReg<T> out, all;
 #pragma unroll
-    for (int k = 0; k < 6; ++k) acc[k] = src[6 * first + k];
-    for (int64_t j = first + 1; j < last; ++j) box_union_into(acc, src + 6 * j);
-    T *dst = dst_all + (int64_t)b * dst_stride + 6 * c;
+    for (int k = 0; k < 6; ++k) {
+        T v = box.v[k];
 #pragma unroll
-    for (int k = 0; k < 6; ++k) dst[k] = acc[k];
+        for (int j = 0; j < kChunkBits; ++j) {
+            tab[j][lane] = v;
+            const T w = __shfl_down(v, 1 << j, 64);      // past the wave's end: the lane's own value
+            v = k < 3 ? tmin(v, w) : tmax(v, w);
+        }
+        all.v[k] = v;                                    // lane 0: the union of all 64
+        // one wave's LDS accesses are served in order; this keeps the compiler to it
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+        const T u = tab[l][lo], w = tab[l][hi + 1 - (1 << l)];
+        out.v[k] = k < 3 ? tmin(u, w) : tmax(u, w);
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    }
+    if (mine) store_box(bb + 6 * p, out);
+    if (chunk_all && lane == 0) store_box(chunk_all + (int64_t)b * chunk_stride + 6 * (p >> kChunkBits), all);
+}
+
+// chunk level L box c = union of the (at most 64) level L-1 boxes 64c .. 64c+63, one per lane.
+template <typename T>
+__global__ __launch_bounds__(256) void k_chunk_boxes(const T *__restrict__ src_all, int64_t src_stride, int64_t src_count,
+                                                     T *__restrict__ dst_all, int64_t dst_stride) {
+    const int b = blockIdx.y;
+    const int64_t c = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if ((c & ~(int64_t)(kChunk - 1)) >= src_count) return;
+    BoxReg<T> box = load_box(src_all + (int64_t)b * src_stride + 6 * (c < src_count ? c : src_count - 1));
+#pragma unroll
+    for (int d = 1; d < kChunk; d <<= 1) box_join_xor(box, d);
+    if ((threadIdx.x & 63) == 0) store_box(dst_all + (int64_t)b * dst_stride + 6 * (c >> kChunkBits), box);
 }
 
 struct ChunkLevels {
@@ -384,35 +538,41 @@ struct ChunkLevels {
     int levels;                          // chunk levels in use
 };
 
+// Fitted modes: the nodes whose range crosses a chunk boundary (a few percent), each by its
+// whole wave: at every level the units at both ends that no unit of the next level covers
+// (at most 63 each, one per lane), until the rest lies within 64 units.
 template <typename T>
-__global__ void k_node_boxes(const int2 *__restrict__ range_all, int64_t n, ChunkLevels lv, T *__restrict__ bboxes_all) {
-    const int b = blockIdx.y;
+__global__ __launch_bounds__(256) void k_cross_nodes(const int2 *__restrict__ range_all, int64_t n, ChunkLevels lv, T *__restrict__ bboxes_all) {
+    const int b = blockIdx.y, lane = threadIdx.x & 63;
     const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n - 1) return;
-    const int2 r = range_all[(int64_t)b * (n - 1) + i];
-    int64_t p = r.x;
-    const int64_t end = (int64_t)r.y + 1;
-    T acc[6];
-    bool first = true;
-    while (p < end) {
-        // the largest aligned chunk that starts at p and ends inside the range
-        int L = 0;
-        while (L < lv.levels && (p & ((int64_t)kChunk << (kChunkBits * L)) - 1) == 0 &&
-               p + ((int64_t)kChunk << (kChunkBits * L)) <= end)
-            ++L;
-        const T *src = (const T *)lv.box[L] + (int64_t)b * lv.stride[L] + 6 * (p >> (kChunkBits * L));
-        if (first) {
-#pragma unroll
-            for (int k = 0; k < 6; ++k) acc[k] = src[k];
-            first = false;
-        } else {
-            box_union_into(acc, src);
+    int2 r = make_int2(0, 0);
+    if (i < n - 1) r = range_all[(int64_t)b * (n - 1) + i];
+    unsigned long long todo = __ballot((r.x >> kChunkBits) != (r.y >> kChunkBits));
+    T *bb = bboxes_all + (int64_t)b * (2 * n - 1) * 6;
+    while (todo) {
+        const int who = __ffsll((long long)todo) - 1;
+        todo &= todo - 1;
+        int64_t lo = __shfl(r.x, who, 64), hi = __shfl(r.y, who, 64);
+        const int64_t node = i - lane + who;
+        BoxReg<T> acc = load_box((const T *)lv.box[0] + (int64_t)b * lv.stride[0] + 6 * lo);
+        for (int L = 0; lo <= hi; ++L) {
+            const T *src = (const T *)lv.box[L] + (int64_t)b * lv.stride[L];
+            if (L == lv.levels || hi - lo < kChunk) {
+                // lanes past the end take the last unit again
+                for (int64_t u = lo; u <= hi; u += kChunk) box_join(acc, load_box(src + 6 * (u + lane <= hi ? u + lane : hi)));
+                break;
+            }
+            const int64_t up = (lo + kChunk - 1) >> kChunkBits, down = ((hi + 1) >> kChunkBits) - 1;   // whole units above
+            const int64_t head = (up << kChunkBits) - 1, tail = (down + 1) << kChunkBits;             // units lo..head, tail..hi
+            if (lo <= head) box_join(acc, load_box(src + 6 * (lo + lane <= head ? lo + lane : head)));
+            if (tail <= hi) box_join(acc, load_box(src + 6 * (tail + lane <= hi ? tail + lane : hi)));
+            lo = up;
+            hi = down;
         }
-        p += (int64_t)1 << (kChunkBits * L);
-    }
-    T *o = bboxes_all + (int64_t)b * (2 * n - 1) * 6 + 6 * i;
 #pragma unroll
-    for (int k = 0; k < 6; ++k) o[k] = acc[k];
+        for (int d = 1; d < 64; d <<= 1) box_join_xor(acc, d);
+        if (lane == 0) store_box(bb + 6 * node, acc);
+    }
 }
 
 // Stable LSD radix sort of B rows of n (key, id) pairs, 8 bits per pass over the key's width;
@@ -441,15 +601,15 @@ static ccc_status build(ccc_context *ctx, const T *t0, const T *t1, int64_t B, i
     const int nb = (int)((n + kSortTile - 1) / kSortTile);
     const bool fit = morton != CCC_MORTON_COMPAT;
     const size_t ksz = morton == CCC_MORTON_63 ? 8 : 4;
-    T *boxes = ws.get_as<T>(total * 6);
-    int32_t *va = ws.get_as<int32_t>(total);
+    T *boxes = fit ? ws.get_as<T>(total * 6) : nullptr;
+    int32_t *va = fit ? ws.get_as<int32_t>(total) : nullptr;
     T *cent = fit ? ws.get_as<T>(total * 3) : nullptr;
     T *part = fit ? ws.get_as<T>((size_t)B * kSceneBlocks * 6) : nullptr;
     void *ka = fit ? ws.get(total * ksz) : nullptr;
     void *kb = fit ? ws.get(total * ksz) : nullptr;
     int32_t *vb = fit ? ws.get_as<int32_t>(total) : nullptr;
     uint32_t *hist = fit ? ws.get_as<uint32_t>((size_t)B * 256 * nb) : nullptr;
-    int2 *range = ws.get_as<int2>((size_t)B * (n > 1 ? n - 1 : 1));
+    int2 *range = fit ? ws.get_as<int2>((size_t)B * (n > 1 ? n - 1 : 1)) : nullptr;
     ChunkLevels lv{};
     lv.box[0] = bboxes + (size_t)6 * (n - 1);
     lv.stride[0] = (2 * n - 1) * 6;
@@ -461,17 +621,34 @@ static ccc_status build(ccc_context *ctx, const T *t0, const T *t1, int64_t B, i
         lv.stride[lv.levels] = count * 6;
     }
     if (ws.failed()) return CCC_ERR_NO_MEMORY;
+    T *chunk1 = lv.levels > 0 ? (T *)lv.box[1] : nullptr;
 
-    tm.begin("bvh_leaf_boxes");
-#define CCC_LEAF(M, F) hipLaunchKernelGGL((k_leaf_boxes<T, M, F>), dim3(grid_for(total, 256)), dim3(256), 0, s, t0, t1, total, n, boxes, cent, va)
-    if (t1) { if (fit) CCC_LEAF(true, true); else CCC_LEAF(true, false); }
-    else { if (fit) CCC_LEAF(false, true); else CCC_LEAF(false, false); }
-#undef CCC_LEAF
+    if (!fit) {
+        // every code is 0 and the stable sort keeps the input order: the index tree
+        tm.begin("bvh_leaves");
+        if (t1) hipLaunchKernelGGL((k_index_leaves<T, true>), dim3(grid_for(n, 256), B), dim3(256), 0, s, t0, t1, n, bboxes, tree, chunk1, lv.stride[1]);
+        else hipLaunchKernelGGL((k_index_leaves<T, false>), dim3(grid_for(n, 256), B), dim3(256), 0, s, t0, t1, n, bboxes, tree, chunk1, lv.stride[1]);
+        tm.end();
+        CCC_LAUNCH_CHECK("k_index_leaves");
+        tm.begin("bvh_refit");
+        int64_t units = n;
+        for (int L = 1; L <= lv.levels; ++L) {
+            units = (units + kChunk - 1) / kChunk;
+            T *dst = L < lv.levels ? (T *)lv.box[L + 1] : nullptr;
+            hipLaunchKernelGGL((k_index_nodes<T>), dim3(grid_for(units, 256), B), dim3(256), 0, s, (const T *)lv.box[L], lv.stride[L], units,
+                               kChunkBits * L, n, bboxes, dst, L < lv.levels ? lv.stride[L + 1] : 0);
+        }
+        tm.end();
+        CCC_LAUNCH_CHECK("node boxes");
+        return CCC_OK;
+    }
+
+    tm.begin("bvh_leaves");
+    if (t1) hipLaunchKernelGGL((k_leaf_boxes<T, true>), dim3(grid_for(total, 256)), dim3(256), 0, s, t0, t1, total, n, boxes, cent, va);
+    else hipLaunchKernelGGL((k_leaf_boxes<T, false>), dim3(grid_for(total, 256)), dim3(256), 0, s, t0, t1, total, n, boxes, cent, va);
     tm.end();
     CCC_LAUNCH_CHECK("k_leaf_boxes");
-
-    // compat: every code is 0 and the stable sort keeps the input order (no codes, no sort)
-    if (fit) {
+    {
         tm.begin("bvh_sort");
         const unsigned gparts = (unsigned)std::min<int64_t>(kSceneBlocks, (n + 255) / 256);
         hipLaunchKernelGGL((k_scene_partial<T>), dim3(gparts, B), dim3(256), 0, s, boxes, n, part);
@@ -501,17 +678,14 @@ static ccc_status build(ccc_context *ctx, const T *t0, const T *t1, int64_t B, i
         CCC_LAUNCH_CHECK("k_karras");
     }
     tm.begin("bvh_refit");
-    hipLaunchKernelGGL((k_leaf_rows<T>), dim3(grid_for(n, 256), B), dim3(256), 0, s, boxes, va, n, bboxes, tree);
-    {
-        int64_t src_count = n;
-        for (int L = 1; L <= lv.levels; ++L) {
-            const int64_t dst_count = (src_count + kChunk - 1) / kChunk;
-            hipLaunchKernelGGL((k_chunk_boxes<T>), dim3(grid_for(dst_count, 256), B), dim3(256), 0, s, (const T *)lv.box[L - 1],
-                               lv.stride[L - 1], src_count, (T *)lv.box[L], lv.stride[L], dst_count);
-            src_count = dst_count;
-        }
+    hipLaunchKernelGGL((k_sorted_leaves<T>), dim3(grid_for(n, 256), B), dim3(256), 0, s, boxes, va, n, range, bboxes, tree, chunk1, lv.stride[1]);
+    int64_t src_count = n;
+    for (int L = 2; L <= lv.levels; ++L) {
+        src_count = (src_count + kChunk - 1) / kChunk;
+        hipLaunchKernelGGL((k_chunk_boxes<T>), dim3(grid_for(src_count, 256), B), dim3(256), 0, s, (const T *)lv.box[L - 1],
+                           lv.stride[L - 1], src_count, (T *)lv.box[L], lv.stride[L]);
     }
-    if (n > 1) hipLaunchKernelGGL((k_node_boxes<T>), dim3(grid_for(n - 1, 256), B), dim3(256), 0, s, range, n, lv, bboxes);
+    if (lv.levels > 0) hipLaunchKernelGGL((k_cross_nodes<T>), dim3(grid_for(n - 1, 256), B), dim3(256), 0, s, range, n, lv, bboxes);
     tm.end();
     CCC_LAUNCH_CHECK("node boxes");
     return CCC_OK;
@@ -533,9 +707,12 @@ size_t build_bvh_arena_bytes(int64_t B, int64_t n, int32_t dtype, int morton) {
     const bool fit = morton != CCC_MORTON_COMPAT;
     const size_t ksz = morton == CCC_MORTON_63 ? 8 : 4;
     const int nb = (int)((n + kSortTile - 1) / kSortTile);
-    size_t tot = r(esz * total * 6) + r(4 * total);
-    if (fit) tot += r(esz * total * 3) + r(esz * B * kSceneBlocks * 6) + 2 * r(ksz * total) + r(4 * total) + r(4 * (size_t)B * 256 * nb);
-    tot += r(sizeof(int2) * B * (n > 1 ? n - 1 : 1));
+    size_t tot = 0;
+    if (fit) {
+        tot += r(esz * total * 6) + r(4 * total) + r(esz * total * 3) + r(esz * B * kSceneBlocks * 6) + 2 * r(ksz * total) + r(4 * total) +
+               r(4 * (size_t)B * 256 * nb);
+        tot += r(sizeof(int2) * B * (n > 1 ? n - 1 : 1));
+    }
     int64_t count = n;
     for (int levels = 0; levels < kChunkLevels && count > kChunk; ++levels) {
         count = (count + kChunk - 1) / kChunk;

@@ -1387,19 +1387,25 @@ __global__ __launch_bounds__(kCcdThreads, MODE == MODE_IMPULSE ? (DET ? 3 : 4) :
     const int ntiles = (int)((M + NT - 1) / NT);
     const int tper = (ntiles + kXcds - 1) / kXcds, tstep = (int)gridDim.x / kXcds;
     const int tbase = (int)(blockIdx.x % kXcds) * tper;
+    // Each block takes one contiguous run of tiles: its collisions share corners, and the
+    // blocks running beside it are far away in the list, so that their atomics fall on other
+    // corners (tiles dealt out one by one: 129.6 instead of 104 ms per step of the 130k cloth,
+    // 8.5 instead of 6.8 of the garment scene, in the order that k_pairs writes its pairs).
+    const int trun = (tper + tstep - 1) / tstep;
+    const int tfirst = (int)blockIdx.x / kXcds * trun, tlast = tfirst + trun < tper ? tfirst + trun : tper;
     auto item_of = [&](int k) -> uint32_t {
         const int64_t i = (int64_t)(tbase + k) * NT + tid;
-        return (k < tper && tbase + k < ntiles && i < M) ? items[i] : kNoItem;
+        return (k < tlast && tbase + k < ntiles && i < M) ? items[i] : kNoItem;
     };
     // the next tile's item waits as its pair (registers) and its type (LDS, 15: no item), so
     // that it holds no more registers than the packed item through phases C and D
     __shared__ unsigned char s_ntype[NT];
     __shared__ int64_t s_myitem[NT];
-    uint32_t next_item = item_of(blockIdx.x / kXcds);
+    uint32_t next_item = item_of(tfirst);
     int2 next_pair = make_int2(0, 0);
     if (next_item != kNoItem) next_pair = pairs[next_item >> 4];
     s_ntype[tid] = (unsigned char)(next_item & 15u);
-    for (int tk = (int)blockIdx.x / kXcds; tk < tper && tbase + tk < ntiles; tk += tstep) {
+    for (int tk = tfirst; tk < tlast && tbase + tk < ntiles; ++tk) {
         // ---- A: coefficients and branch of the lane's item
         const int ntype = s_ntype[tid];
         const int64_t it = ntype != 15 ? pack_item(next_pair.x, next_pair.y, ntype) : (int64_t)-1;
@@ -1417,7 +1423,7 @@ __global__ __launch_bounds__(kCcdThreads, MODE == MODE_IMPULSE ? (DET ? 3 : 4) :
             code = cubic_prepare(cf[0], cf[1], cf[2], cf[3], st);
         }
         s_myitem[tid] = it;     // read back for the root list, not held through the solver
-        next_item = item_of(tk + tstep);
+        next_item = item_of(tk + 1);
         // ---- B: the lane's roots in [0, 1], in the order found, to the root list
         T r0, r1, r2;
         const int nk = cubic_roots<T>(code, st, r0, r1, r2);

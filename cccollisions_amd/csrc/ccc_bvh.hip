@@ -332,58 +332,7 @@ __global__ void k_karras(const K *__restrict__ codes_all, const int32_t *__restr
 // Positions are grouped in chunks of 64, one per lane of a wave, whose unions come from lane
 // exchanges.  (One thread per chunk, walking its 64 boxes one after the other, was bound by
 // the latency of that chain: 12-22 us per level, and as much again for the nodes' own walks.)
-constexpr int kChunkBits = 6;
-constexpr int kChunk = 1 << kChunkBits;
 constexpr int kChunkLevels = 5;      // 64^5 = 2^30 > 2^28 leaves
-
-template <typename T> struct BoxReg { T v[6]; };   // min xyz, max xyz
-
-template <typename T> __device__ __forceinline__ BoxReg<T> load_box(const T *p) {
-    BoxReg<T> r;
-#pragma unroll
-    for (int k = 0; k < 6; ++k) r.v[k] = p[k];
-    return r;
-}
-template <typename T> __device__ __forceinline__ void store_box(T *p, const BoxReg<T> &r) {
-#pragma unroll
-    for (int k = 0; k < 6; ++k) p[k] = r.v[k];
-}
-template <typename T> __device__ __forceinline__ void box_join(BoxReg<T> &a, const BoxReg<T> &b) {
-#pragma unroll
-    for (int k = 0; k < 3; ++k) {
-        a.v[k] = tmin(a.v[k], b.v[k]);
-        a.v[k + 3] = tmax(a.v[k + 3], b.v[k + 3]);
-    }
-}
-// the union over lanes l and l ^ d
-template <typename T> __device__ __forceinline__ void box_join_xor(BoxReg<T> &a, int d) {
-#pragma unroll
-    for (int k = 0; k < 3; ++k) {
-        a.v[k] = tmin(a.v[k], __shfl_xor(a.v[k], d, 64));
-        a.v[k + 3] = tmax(a.v[k + 3], __shfl_xor(a.v[k + 3], d, 64));
-    }
-}
-
-// The compat tree is the radix tree over leaf indices (every code is 0).  Node i covers the
-// aligned block of 2^k leaves that starts at i (i even, k = trailing zeros of i) or ends at i
-// (i odd, k = trailing zeros of i + 1), cut off at n; node 0 covers everything.  That is
-// Karras' Algorithm 1 (k_karras below) with delta(i, j) = 32 + clz(i ^ j) solved in closed
-// form: the direction and range follow from i's neighbours, and the split is at the highest
-// differing bit of the range's ends.
-__device__ __forceinline__ int index_node_level(int64_t i) { return __ffsll((long long)((i & 1) ? i + 1 : i)) - 1; }
-
-__device__ __forceinline__ void index_node_row(int64_t i, int64_t n, int64_t &left, int64_t &right) {
-    int64_t lo = 0, hi = n - 1;
-    if (i > 0) {
-        const int64_t len = (int64_t)1 << index_node_level(i);
-        lo = (i & 1) ? i + 1 - len : i;
-        hi = (i & 1) ? i : (i + len <= n ? i + len - 1 : n - 1);
-    }
-    const int bit = 63 - __clzll((long long)(lo ^ hi));
-    const int64_t split = ((hi >> bit) << bit) - 1;
-    left = lo == split ? n - 1 + split : split;
-    right = hi == split + 1 ? n - 1 + split + 1 : split + 1;
-}
 
 // Writes the boxes of the nodes that end at this level: `box` is the union over lane's leaf
 // or chunk, unit `c` of `count` units of 2^shift leaves each; a unit's node is the one whose
@@ -505,15 +454,10 @@ __global__ __launch_bounds__(256) void k_sorted_leaves(const T *__restrict__ box
             v = k < 3 ? tmin(v, w) : tmax(v, w);
         }
         all.v[k] = v;                                    // lane 0: the union of all 64
-        // one wave's LDS accesses are served in order; this keeps the compiler to it
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-        __builtin_amdgcn_wave_barrier();
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+        wave_sync();
         const T u = tab[l][lo], w = tab[l][hi + 1 - (1 << l)];
         out.v[k] = k < 3 ? tmin(u, w) : tmax(u, w);
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-        __builtin_amdgcn_wave_barrier();
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+        wave_sync();
     }
     if (mine) store_box(bb + 6 * p, out);
     if (chunk_all && lane == 0) store_box(chunk_all + (int64_t)b * chunk_stride + 6 * (p >> kChunkBits), all);

@@ -72,6 +72,35 @@ template <typename T> __device__ __forceinline__ Box<T> tri_box(V3<T> a, V3<T> b
                   mk(tmax(a.x, tmax(b.x, c.x)), tmax(a.y, tmax(b.y, c.y)), tmax(a.z, tmax(b.z, c.z)))};
 }
 
+// Boxes held as six values, for loads, stores and unions over the lanes of a wave.
+template <typename T> struct BoxReg { T v[6]; };   // min xyz, max xyz
+
+template <typename T> __device__ __forceinline__ BoxReg<T> load_box(const T *p) {
+    BoxReg<T> r;
+#pragma unroll
+    for (int k = 0; k < 6; ++k) r.v[k] = p[k];
+    return r;
+}
+template <typename T> __device__ __forceinline__ void store_box(T *p, const BoxReg<T> &r) {
+#pragma unroll
+    for (int k = 0; k < 6; ++k) p[k] = r.v[k];
+}
+template <typename T> __device__ __forceinline__ void box_join(BoxReg<T> &a, const BoxReg<T> &b) {
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+        a.v[k] = tmin(a.v[k], b.v[k]);
+        a.v[k + 3] = tmax(a.v[k + 3], b.v[k + 3]);
+    }
+}
+// the union over lanes l and l ^ d
+template <typename T> __device__ __forceinline__ void box_join_xor(BoxReg<T> &a, int d) {
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+        a.v[k] = tmin(a.v[k], __shfl_xor(a.v[k], d, 64));
+        a.v[k + 3] = tmax(a.v[k + 3], __shfl_xor(a.v[k + 3], d, 64));
+    }
+}
+
 // figures.cu:527-544 shareVertex: exact coincidence of any t0 vertices.
 template <typename T> __device__ __forceinline__ bool share_vertex(const V3<T> *a, const V3<T> *b) {
     bool s = false;

@@ -146,7 +146,29 @@ inline unsigned grid_for(int64_t items, int block) {
 // Device error bits reported by kernels.
 // DEV_UNORDERED is informational: the tree's subtrees do not cover contiguous, ordered
 // leaf ranges (or are deeper than 64), so the rightmost leaves come from the climb.
-enum : unsigned { DEV_BAD_TREE = 1u, DEV_STACK = 2u, DEV_UNORDERED = 4u };
+// DEV_FOREIGN: the tree is not the index tree that bvh / bvh_motion build by default.
+enum : unsigned { DEV_BAD_TREE = 1u, DEV_STACK = 2u, DEV_UNORDERED = 4u, DEV_FOREIGN = 8u };
+
+// The compat tree is the radix tree over leaf indices (every Morton code is 0).  Node i covers
+// the aligned block of 2^k leaves that starts at i (i even, k = trailing zeros of i) or ends
+// at i (i odd, k = trailing zeros of i + 1), cut off at n; node 0 covers everything.  That is
+// Karras' Algorithm 1 (k_karras) with delta(i, j) = 32 + clz(i ^ j) solved in closed form: the
+// direction and range follow from i's neighbours, and the split is at the highest differing
+// bit of the range's ends.
+__device__ __forceinline__ int index_node_level(int64_t i) { return __ffsll((long long)((i & 1) ? i + 1 : i)) - 1; }
+
+__device__ __forceinline__ void index_node_row(int64_t i, int64_t n, int64_t &left, int64_t &right) {
+    int64_t lo = 0, hi = n - 1;
+    if (i > 0) {
+        const int64_t len = (int64_t)1 << index_node_level(i);
+        lo = (i & 1) ? i + 1 - len : i;
+        hi = (i & 1) ? i : (i + len <= n ? i + len - 1 : n - 1);
+    }
+    const int bit = 63 - __clzll((long long)(lo ^ hi));
+    const int64_t split = ((hi >> bit) << bit) - 1;
+    left = lo == split ? n - 1 + split : split;
+    right = hi == split + 1 ? n - 1 + split + 1 : split + 1;
+}
 
 // Per-batch-element counters kept on the device during a call.
 struct alignas(64) DevCounters {
@@ -185,7 +207,7 @@ struct ResidentPass {
     int64_t cap_pairs;
     int64_t chunk;
     int ccd_blocks_per_cu;       // grid cap of k_ccd (0: 128)
-    bool stack_deep;             // traverse with the deep stack from the start
+    const int64_t *leaf_ids;     // the tree when its leaves are in another order than the triangles (fitted), else NULL
     long long *det_acc;
     void *dv, *dx;
     int32_t *cnt;
@@ -195,9 +217,19 @@ ccc_status resident_pass(ccc_context *ctx, const ResidentPass &p, void *arena, s
 size_t resident_pass_arena_bytes(ccc_context *ctx, const ResidentPass &p);
 constexpr int kDetWordsPerCorner = 24;
 
-// Fill kernels (used instead of hipMemsetAsync so that the calls stay capturable).
-ccc_status fill_u64(void *p, int64_t count, uint64_t value, hipStream_t s);
-ccc_status fill_u32(void *p, int64_t count, uint32_t value, hipStream_t s);
+// Buffers a call fills before it starts (a kernel instead of hipMemsetAsync, so that the
+// calls stay capturable): `words` 32-bit words of the repeated 64-bit `value`.
+struct FillRegion {
+    void *p;
+    int64_t words;
+    uint64_t value;
+};
+struct FillRegions {
+    FillRegion r[8];
+    int count = 0;
+    void add(void *p, int64_t bytes, uint64_t value) { r[count++] = FillRegion{p, bytes / 4, value}; }
+};
+ccc_status fill_regions(const FillRegions &r, hipStream_t s);
 
 // BVH over B soups of n triangles each (t1 = NULL: static boxes) into the wire format, with
 // Morton mode `morton` (CCC_MORTON_*); arguments already validated, the device already
@@ -208,6 +240,12 @@ ccc_status build_bvh_device(ccc_context *ctx, const void *t0, const void *t1, in
 size_t build_bvh_arena_bytes(int64_t B, int64_t n, int32_t dtype, int morton);
 
 }  // namespace ccc
+
+// Leaf positions are grouped in chunks of 64, one per lane of a wave.
+namespace ccc {
+constexpr int kChunkBits = 6;
+constexpr int kChunk = 1 << kChunkBits;
+}
 
 // ---- wave primitives (wave64) ---------------------------------------------------------
 namespace ccc {
@@ -241,4 +279,15 @@ __device__ __forceinline__ unsigned long long wave_reserve(unsigned long long *c
     base = readfirstlane_u64(base);
     return base + below;
 }
+
+// Orders the wave's LDS accesses before this point against those after it.  The lanes of a
+// wavefront run in lockstep and the LDS serves one wave's accesses in issue order, so no
+// instruction is needed: the fences and the barrier only keep the compiler from moving
+// memory accesses across the point.
+__device__ __forceinline__ void wave_sync() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
 }  // namespace ccc

@@ -184,6 +184,7 @@ __global__ void k_order_check(const int64_t *__restrict__ tree_all, int64_t n, c
 }
 
 // Climb for the remaining trees: the second thread to reach a node combines its children.
+// The counters are k_check_tree's claims, one per leaf id and each 1 in a valid tree.
 __global__ void k_rightmost(const int64_t *__restrict__ tree_all, int64_t n, int *__restrict__ counters_all,
                             int *__restrict__ rm_all, DevCounters *__restrict__ ctr) {
     const int b = blockIdx.y;
@@ -192,14 +193,14 @@ __global__ void k_rightmost(const int64_t *__restrict__ tree_all, int64_t n, int
     if ((ctr[b].flags & DEV_BAD_TREE) || !(ctr[b].flags & DEV_UNORDERED)) return;
     const int64_t rows = 2 * n - 1;
     const int64_t *tree = tree_all + (int64_t)b * rows * 4;
-    int *counters = counters_all + (int64_t)b * (n - 1);
+    int *counters = counters_all + (int64_t)b * n;
     int *rm = rm_all + (int64_t)b * (n - 1);
     int64_t cur = tree[4 * (n - 1 + pos)];
     for (int64_t step = 0; cur >= 0; ++step) {
         if (step > n) { atomicOr(&ctr[b].flags, DEV_BAD_TREE); return; }
         __threadfence();
         const int old = __hip_atomic_fetch_add(&counters[cur], 1, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT);
-        if (old == 0) return;
+        if (old == 1) return;
         __threadfence();
         const int64_t l = tree[4 * cur + 1], r = tree[4 * cur + 2];
         const int a = l >= n - 1 ? (int)(l - (n - 1)) : __hip_atomic_load(&rm[l], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -680,6 +681,347 @@ __global__ __launch_bounds__(kTravThreads) void k_traverse(const T *__restrict__
     }
 }
 
+// ---- candidate pairs of an index tree -------------------------------------------------------
+// A traversal reports the pairs (p, l) of leaf positions, l > p, whose exact boxes overlap
+// (collisions_static.cu:10-120, collisions_continuous.cu:127-230, :1079-1100); which tree it
+// walks does not matter as long as node boxes contain their leaves'.  For the trees whose
+// leaves are in index or Morton order (the index tree, and the resident simulation's fitted
+// trees), positions are therefore grouped in chunks of 64 instead: a wave takes a group of
+// queries, tests the group's union box against 64 chunks at a time (one per lane), the leaves
+// of each hit chunk against it (one per lane), and the leaves that are left against the
+// queries.  There is no per-lane walk and no stack: the walk (k_traverse) spent 560 lane
+// instructions per pair that it found, on dependent node reads.  Traversal per pass, walk ->
+// chunks: 130k cloth (5.9e7 pairs) 1,770 -> 390 us, packed 12 meshes (1.4e8 pairs) 9,300 ->
+// 1,000 us, shuffled 32k 500 -> 63 us, garment 122k 220 -> 130 us, 33k f32 144 -> 38 us.
+
+// The answer of k_prep's tree check, one 256-byte line per batch element: every wave of
+// k_pairs reads it, so it lies apart from the counters that they reserve pairs on.
+constexpr int kForeignStep = 64;
+
+constexpr int kPairQ = 16;        // queries per wave of k_pairs, each held by 64 / kPairQ lanes
+
+// The union of a group's kPairQ boxes as two boxes: those of the queries up to and after the
+// place where splitting the sequence gives the smallest extents, when that is much smaller
+// than the union of all.  Consecutive triangles are neighbours except where a row of the mesh
+// or one of its parts ends; the union over such a place spans everything between, and the few
+// waves that hold one would take many times as long as the others (with single boxes 400 us
+// instead of 144 on the 122k garment scene, 1,075 instead of 395 on the 130k cloth).
+template <typename T> __device__ __forceinline__ float box_extent(const BoxReg<T> &a) {
+    return (float)(a.v[3] - a.v[0]) + (float)(a.v[4] - a.v[1]) + (float)(a.v[5] - a.v[2]);
+}
+template <typename T> __device__ __forceinline__ void split_union(const BoxReg<T> &q, int qi, BoxReg<T> &ua, BoxReg<T> &ub) {
+    BoxReg<T> pre = q, suf = q;      // of the queries 0..qi and qi..kPairQ - 1
+#pragma unroll
+    for (int d = 1; d < kPairQ; d <<= 1) {
+        // a lane without a source gets its own value back: joining it changes nothing
+#pragma unroll
+        for (int k = 0; k < 3; ++k) {
+            pre.v[k] = tmin(pre.v[k], __shfl_up(pre.v[k], d, kPairQ));
+            pre.v[k + 3] = tmax(pre.v[k + 3], __shfl_up(pre.v[k + 3], d, kPairQ));
+            suf.v[k] = tmin(suf.v[k], __shfl_down(suf.v[k], d, kPairQ));
+            suf.v[k + 3] = tmax(suf.v[k + 3], __shfl_down(suf.v[k + 3], d, kPairQ));
+        }
+    }
+    const float whole = __shfl(box_extent(pre), kPairQ - 1, kPairQ);
+    float cost = box_extent(pre) + __shfl_down(box_extent(suf), 1, kPairQ);
+    if (!(cost <= 3.0e38f) || qi == kPairQ - 1) cost = 3.0e38f;      // no split here (NaN included)
+    float best = cost;
+#pragma unroll
+    for (int d = 1; d < kPairQ; d <<= 1) best = fminf(best, __shfl_xor(best, d, kPairQ));
+    const int at = best < 0.75f * whole ? __ffsll((long long)__ballot(cost == best)) - 1 : kPairQ - 1;
+    const int from = at == kPairQ - 1 ? 0 : at + 1;
+#pragma unroll
+    for (int k = 0; k < 6; ++k) {
+        ua.v[k] = __shfl(pre.v[k], at, kPairQ);
+        ub.v[k] = __shfl(suf.v[k], from, kPairQ);
+    }
+}
+
+// First launch of a query: (1) does the tree equal the index tree?  Any other tree sets
+// `foreign` and goes through the checked general path; (2) the box of each chunk of 64 leaf
+// positions and the two unions of each query group; (3) the vertex records (when tv is given).
+// Blocks of 256 threads, partitioned by blockIdx.x: rows, leaves, corners.
+template <typename T>
+__global__ __launch_bounds__(256) void k_prep(const T *__restrict__ bb_all, const int64_t *__restrict__ tree_all, int64_t n, unsigned row_blocks,
+                                              unsigned leaf_blocks, T *__restrict__ chunk_all, T *__restrict__ group_all,
+                                              const T *__restrict__ t0_all,
+                                              const T *__restrict__ t1_all, T *__restrict__ tv_all, unsigned *__restrict__ foreign) {
+    const int b = blockIdx.y;
+    const int64_t rows = 2 * n - 1;
+    if (blockIdx.x < row_blocks) {
+        const int64_t r = (int64_t)blockIdx.x * 256 + threadIdx.x;
+        if (r >= rows) return;
+        const int64_t *tree = tree_all + (int64_t)b * rows * 4;
+        const int64_t l = tree[4 * r + 1], rr = tree[4 * r + 2];
+        bool ok = r != 0 || tree[0] == -1;
+        if (r < n - 1) {
+            int64_t left, right;
+            index_node_row(r, n, left, right);
+            ok = ok && l == left && rr == right && tree[4 * left] == r && tree[4 * right] == r;
+        } else {
+            ok = ok && l == -1 && rr == -1 && tree[4 * r + 3] == r - (n - 1);
+        }
+        if (!ok) foreign[kForeignStep * b] = 1u;
+    } else if (blockIdx.x < row_blocks + leaf_blocks) {
+        const int64_t p = (int64_t)(blockIdx.x - row_blocks) * 256 + threadIdx.x;
+        if ((p & ~(int64_t)(kChunk - 1)) >= n) return;
+        const int64_t nc = (n + kChunk - 1) >> kChunkBits;
+        const BoxReg<T> leaf = load_box(bb_all + ((int64_t)b * rows + (n - 1) + (p < n ? p : n - 1)) * 6);
+        BoxReg<T> box = leaf;
+#pragma unroll
+        for (int d = 1; d < kChunk; d <<= 1) box_join_xor(box, d);
+        if ((threadIdx.x & 63) == 0) store_box(chunk_all + ((int64_t)b * nc + (p >> kChunkBits)) * 6, box);
+        // the two unions of each query group
+        const int qi = threadIdx.x & (kPairQ - 1);
+        BoxReg<T> ua, ub;
+        split_union(leaf, qi, ua, ub);
+        if (qi == 0) {
+            T *g = group_all + ((int64_t)b * nc * (kChunk / kPairQ) + p / kPairQ) * 12;
+            store_box(g, ua);
+            store_box(g + 6, ub);
+        }
+    } else {
+        const int64_t i = (int64_t)(blockIdx.x - row_blocks - leaf_blocks) * 256 + threadIdx.x;
+        if (i >= 3 * n) return;
+        const T *a = t0_all + ((int64_t)b * 3 * n + i) * 3, *c = t1_all + ((int64_t)b * 3 * n + i) * 3;
+        VRec<T> r;
+        r.a[0] = a[0]; r.a[1] = a[1]; r.a[2] = a[2];
+        r.a[3] = c[0] - a[0]; r.a[4] = c[1] - a[1]; r.a[5] = c[2] - a[2];
+        reinterpret_cast<VRec<T> *>(tv_all)[(int64_t)b * 3 * n + i] = r;
+    }
+}
+
+// Boxes of 64 chunks each, for meshes of more than kSuperFrom chunks.
+template <typename T>
+__global__ __launch_bounds__(256) void k_super_boxes(const T *__restrict__ chunk_all, int64_t nc, T *__restrict__ super_all) {
+    const int b = blockIdx.y;
+    const int64_t c = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    if ((c & ~(int64_t)(kChunk - 1)) >= nc) return;
+    BoxReg<T> box = load_box(chunk_all + ((int64_t)b * nc + (c < nc ? c : nc - 1)) * 6);
+#pragma unroll
+    for (int d = 1; d < kChunk; d <<= 1) box_join_xor(box, d);
+    if ((threadIdx.x & 63) == 0) store_box(super_all + ((int64_t)b * ((nc + kChunk - 1) >> kChunkBits) + (c >> kChunkBits)) * 6, box);
+}
+// Testing every chunk costs each query chunk nc / 64 wave steps: up to 64 steps (262k
+// triangles) that is far less than its leaf tests.
+constexpr int64_t kSuperFrom = 4096;
+
+constexpr int kPairEnt = 512;    // (leaf, query mask) entries per wave before a flush
+constexpr int kPairWaves = 8;     // waves per block; their last entries share one reservation
+constexpr int kPairSub = 64 / kPairQ;
+
+// The reference's checkOverlap(q, other, thr) term by term (aabb.cu:101-111), with the other
+// box already moved by the threshold.  Rounding is monotone, so a box that contains another's
+// passes whenever that one does.
+template <typename T> __device__ __forceinline__ bool box_hits(const BoxReg<T> &q, const BoxReg<T> &o) {
+    return (q.v[0] <= o.v[3]) & (q.v[3] >= o.v[0]) & (q.v[1] <= o.v[4]) & (q.v[4] >= o.v[1]) & (q.v[2] <= o.v[5]) & (q.v[5] >= o.v[2]);
+}
+// A box moved outward by the threshold, as checkOverlap moves it (aabb.cu:101-111).
+template <typename T> __device__ __forceinline__ void box_grow(BoxReg<T> &o, T thr) {
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+        o.v[k] = o.v[k] - thr;
+        o.v[k + 3] = o.v[k + 3] + thr;
+    }
+}
+
+// One wave per (group of kPairQ queries, split): split s of `splits` takes every splits-th
+// chunk, so that small meshes fill the chip too.  The chunks that the group's union box meets
+// are visited one after the other (the next one's boxes already on their way); the leaves that
+// it meets gather in a list in LDS, from which each step takes four, one per 16 lanes, against
+// the 16 queries.  16 queries rather than 64: consecutive triangles are a strip of the mesh,
+// and a shorter strip's union box meets fewer leaves (1.7e8 leaf tests against 5.1e8 on the
+// 130k cloth, of which 5.9e7 are pairs).  A step is about 14 vector instructions and 26 LDS
+// cycles for 64 tests.  Results are kept as (leaf, mask of the queries) until kPairEnt - 64
+// entries are there; then one reservation and one run of coalesced stores writes the pairs,
+// grouped by leaf.  A reservation is a returning atomic on one device address (6-12 ns each,
+// whatever the number of waves), so there are few of them.
+// Tried and slower: 64 queries against leaf boxes read by scalar loads, and against boxes
+// broadcast from LDS one leaf at a time (1,570 and 1,150 us on the 130k cloth, both bound by
+// the latency of that one read per leaf).
+// leaf_ids: the tree (its id column) when position and triangle id differ, else NULL.
+template <typename T, bool PARTIAL>
+__global__ __launch_bounds__(64 * kPairWaves) void k_pairs(const T *__restrict__ bb_all, const int64_t *__restrict__ leaf_ids, int64_t n, T thr,
+                                                           const T *__restrict__ chunk_all, const T *__restrict__ super_all,
+                                                           const T *__restrict__ group_all, int splits,
+                                                           const uint8_t *__restrict__ to_check_all, const int32_t *__restrict__ mesh_end,
+                                                           int2 *__restrict__ pairs_all, int64_t cap, const unsigned *__restrict__ foreign_all,
+                                                           DevCounters *__restrict__ ctr_all) {
+    struct alignas(16) SBox { BoxReg<T> box; };
+    constexpr int kList = kChunk + kPairSub;      // a visit's leaves and fewer than a step's left over
+    __shared__ SBox s_boxes[kPairWaves][kList];
+    __shared__ int s_leafs[kPairWaves][kList];             // position
+    __shared__ int s_idss[kPairWaves][PARTIAL ? kList : 1];    // id | (to_check << 31)
+    __shared__ uint32_t s_ents[kPairWaves][kPairEnt];          // (position - ebase) << kPairQ | mask of the queries
+    __shared__ unsigned long long s_base[kPairWaves];
+    const int b = blockIdx.y, lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int qi = lane & (kPairQ - 1), sub = lane / kPairQ;
+    SBox *s_box = s_boxes[w];
+    int *s_leaf = s_leafs[w], *s_id = s_idss[w];
+    uint32_t *s_ent = s_ents[w];
+    DevCounters *ctr = ctr_all + b;
+    if (foreign_all && foreign_all[kForeignStep * b]) {
+        if (blockIdx.x == 0 && threadIdx.x == 0) atomicOr(&ctr->flags, DEV_FOREIGN);
+        return;
+    }
+    const int64_t rows = 2 * n - 1;
+    const unsigned nq = (unsigned)((n + kPairQ - 1) / kPairQ), task = blockIdx.x * kPairWaves + w;
+    const unsigned qg = task % nq, split = task / nq;      // split >= splits: an idle wave
+    const int64_t nc = (n + kChunk - 1) >> kChunkBits;
+    const T *bb = bb_all + ((int64_t)b * rows + (n - 1)) * 6;          // leaf rows
+    const int64_t *ids = leaf_ids ? leaf_ids + ((int64_t)b * rows + (n - 1)) * 4 + 3 : nullptr;
+    const T *chunks = chunk_all + (int64_t)b * nc * 6;
+    const T *supers = super_all ? super_all + (int64_t)b * ((nc + kChunk - 1) >> kChunkBits) * 6 : nullptr;
+    int2 *pairs = pairs_all + (int64_t)b * cap;
+    const uint8_t *to_check = PARTIAL ? to_check_all + (int64_t)b * n : nullptr;
+
+    const int last = (int)n - 1, p0 = (int)qg * kPairQ, p = p0 + qi, pc = p < last ? p : last;
+    bool active = p <= last && split < (unsigned)splits;
+    if (PARTIAL) active = active && to_check[pc] != 0;
+    const bool any = __any(active);
+    const BoxReg<T> q = load_box(bb + 6 * (int64_t)pc);
+    const int qid = ids ? (int)ids[4 * (int64_t)pc] : pc;
+    // the group's unions are the same for the whole wave: scalar loads, scalar operands
+    using ConstT = const __attribute__((address_space(4))) T;
+    ConstT *group = (ConstT *)(uintptr_t)(group_all + ((int64_t)b * nc * (kChunk / kPairQ) + qg) * 12);
+    BoxReg<T> ua, ub;
+#pragma unroll
+    for (int k = 0; k < 6; ++k) {
+        ua.v[k] = group[k];
+        ub.v[k] = group[6 + k];
+    }
+    auto meets = [&](const BoxReg<T> &o) { return box_hits(ua, o) | box_hits(ub, o); };
+    // packed meshes: leaves from lim on belong to later meshes (lim does not decrease with p)
+    const int lim = mesh_end ? mesh_end[pc] : (int)n;
+    const int lend = mesh_end ? mesh_end[p0 + kPairQ - 1 < last ? p0 + kPairQ - 1 : last] : (int)n;
+    const int64_t cend = any ? ((int64_t)lend + kChunk - 1) >> kChunkBits : 0;
+    const int64_t first = PARTIAL ? 0 : (int64_t)(p0 >> kChunkBits);
+    int nent = 0, cnt = 0, ebase = 0;
+    unsigned total = 0;
+
+    // one step: the leaf of a list entry against this lane's query
+    auto test = [&](const BoxReg<T> &o, int l, int id, bool valid) {
+        bool h = valid & active & box_hits(q, o);
+        if (PARTIAL) h = h & ((id >= 0) | (qid < (id & 0x7fffffff)));   // collisions_continuous.cu:1090: the lower id of two checked ones
+        else h = h & (l > p);
+        if (mesh_end) h = h & (l < lim);
+        const unsigned long long m = __ballot(h);
+        total += (unsigned)__popcll(m);
+        if (qi == 0) s_ent[nent + sub] = ((uint32_t)(l - ebase) << kPairQ) | ((uint32_t)(m >> (sub * kPairQ)) & ((1u << kPairQ) - 1));
+        nent += kPairSub;
+    };
+    auto step = [&](int e, bool valid) { test(s_box[e].box, s_leaf[e], PARTIAL ? s_id[e] : 0, valid); };
+    // two steps, all their reads in flight together
+    auto step2 = [&](int e) {
+        const BoxReg<T> o0 = s_box[e].box, o1 = s_box[e - kPairSub].box;
+        const int l0 = s_leaf[e], l1 = s_leaf[e - kPairSub], i0 = PARTIAL ? s_id[e] : 0, i1 = PARTIAL ? s_id[e - kPairSub] : 0;
+        test(o0, l0, i0, true);
+        test(o1, l1, i1, true);
+    };
+    // writes the entries' pairs from slot `base` on, four entries at a time
+    auto emit = [&](unsigned long long base) {
+#pragma unroll 2
+        for (int e = 0; e < nent; e += kPairSub) {
+            const uint32_t en = s_ent[e + sub];
+            const bool on = ((en >> qi) & 1u) != 0u;
+            const unsigned long long m = __ballot(on), d = base + lanes_below(m);
+            if (on && d < (unsigned long long)cap) {
+                const int l = ebase + (int)(en >> kPairQ), lid = ids ? (int)ids[4 * (int64_t)l] : l;
+                pairs[d] = make_int2(min(qid, lid), max(qid, lid));
+            }
+            base += (unsigned long long)__popcll(m);
+        }
+    };
+    auto flush = [&]() {
+        wave_sync();
+        unsigned long long base = 0;
+        if (lane == 0) base = atomicAdd(&ctr->cand, (unsigned long long)total);
+        emit(readfirstlane_u64(base));
+        wave_sync();
+        nent = 0;
+        total = 0;
+    };
+    // the leaves left over, fewer than a step's
+    auto finish_list = [&]() {
+        if (cnt > 0) step(sub < cnt ? sub : 0, sub < cnt);
+        cnt = 0;
+    };
+
+    for (int64_t c0 = splits == 1 ? first & ~(int64_t)(kChunk - 1) : first; c0 < cend; c0 += (int64_t)kChunk * splits) {
+        if (supers && splits == 1) {
+            BoxReg<T> sb = load_box(supers + 6 * (c0 >> kChunkBits));
+            box_grow(sb, thr);
+            if (!meets(sb)) continue;
+        }
+        const int64_t mine = c0 + split + (int64_t)lane * splits;
+        BoxReg<T> cb = load_box(chunks + 6 * (mine < cend ? mine : cend - 1));
+        box_grow(cb, thr);
+        unsigned long long hit = __ballot(mine >= first && mine < cend && meets(cb));
+        // the boxes of the next chunk are loaded while this one's leaves are tested
+        auto next_leaf = [&](BoxReg<T> &box) -> int {
+            const int k = __ffsll((long long)hit) - 1;
+            hit &= hit - 1;
+            const int l = (int)((c0 + split + (int64_t)k * splits) << kChunkBits) + lane;
+            box = load_box(bb + 6 * (int64_t)(l < last ? l : last));
+            return l;
+        };
+        BoxReg<T> nb;
+        int nl = -1;
+        if (hit) nl = next_leaf(nb);
+        while (nl >= 0) {
+            BoxReg<T> lb = nb;
+            const int l = nl;
+            nl = -1;
+            if (hit) nl = next_leaf(nb);
+            box_grow(lb, thr);
+            const bool on = l <= last && (PARTIAL || l > p0) && meets(lb);
+            const unsigned long long left = __ballot(on);
+            if (!left) continue;
+            const int l0 = __builtin_amdgcn_readfirstlane(l - lane);
+            if (l0 + kChunk - ebase > 1 << (32 - kPairQ)) {
+                // entries hold positions relative to ebase in 16 bits
+                finish_list();
+                if (nent) flush();
+                ebase = l0;
+            }
+            if (on) {
+                const int e = cnt + (int)lanes_below(left);
+                s_box[e].box = lb;
+                s_leaf[e] = l;
+                if (PARTIAL) {
+                    const int id = ids ? (int)ids[4 * (int64_t)l] : l;
+                    s_id[e] = id | (to_check[id] ? (int)0x80000000 : 0);
+                }
+            }
+            cnt += (int)__popcll(left);
+            wave_sync();
+            for (; cnt >= 2 * kPairSub; cnt -= 2 * kPairSub) step2(cnt - kPairSub + sub);
+            if (cnt >= kPairSub) {
+                step(cnt - kPairSub + sub, true);
+                cnt -= kPairSub;
+            }
+            wave_sync();
+            if (nent > kPairEnt - kList - kPairSub) flush();
+        }
+    }
+    finish_list();
+    // the waves' last entries: one reservation for the block
+    if (lane == 0) s_base[w] = total;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        unsigned long long sum = 0;
+        for (int k = 0; k < kPairWaves; ++k) {
+            const unsigned long long t = s_base[k];
+            s_base[k] = sum;
+            sum += t;
+        }
+        const unsigned long long base = sum ? atomicAdd(&ctr->cand, sum) : 0ull;
+        for (int k = 0; k < kPairWaves; ++k) s_base[k] += base;
+    }
+    __syncthreads();
+    if (nent) emit(readfirstlane_u64(s_base[w]));
+}
+
 // ---- sub-primitive filter -----------------------------------------------------------------
 // Candidate pairs -> the pairs of sub-primitives (9 edge-edge, 6 vertex-face) whose boxes
 // overlap, with PP pairs per thread and one reservation per PP * kThreads pairs (the item
@@ -875,20 +1217,6 @@ __global__ __launch_bounds__(kThreads) void k_subprim(const int2 *__restrict__ p
 //            with atomics into dv / dx / cnt (collisions_impulses.cu:1312-1366).
 // The tetrahedron is gathered again for the filter so that it is not live across the
 // cubic solver (fewer VGPRs, more waves per SIMD).
-// Vertex records [x0 y0 z0 dx dy dz] (d = x1 - x0) per triangle corner from the t0 / t1 soups.
-template <typename T>
-__global__ void k_vertex_records(const T *__restrict__ t0_all, const T *__restrict__ t1_all, int64_t corners,
-                                 T *__restrict__ tv_all) {
-    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;   // corner of batch element blockIdx.y
-    if (i >= corners) return;
-    const int64_t b = blockIdx.y;
-    const T *a = t0_all + (b * corners + i) * 3, *c = t1_all + (b * corners + i) * 3;
-    VRec<T> r;
-    r.a[0] = a[0]; r.a[1] = a[1]; r.a[2] = a[2];
-    r.a[3] = c[0] - a[0]; r.a[4] = c[1] - a[1]; r.a[5] = c[2] - a[2];
-    reinterpret_cast<VRec<T> *>(tv_all)[b * corners + i] = r;
-}
-
 enum { MODE_COLLECT = 0, MODE_IMPULSE = 1 };
 // Threads (items) per k_ccd tile, in both modes: one wave per block, so that its phases need
 // no workgroup barrier (k_ccd per step on the 130k cloth: 4 waves per block 206 ms, 2 waves
@@ -1193,16 +1521,6 @@ template <typename P> __device__ __forceinline__ P *opaque_ptr(P *p) {
 // query triangle in LDS (so that half the corner reads leave the vector memory path) made
 // the impulse mode spill and took 196-209 ms per step instead of 177.
 constexpr int kCollectFlush = 64;
-
-// Orders the wave's LDS accesses before this point against those after it.  The lanes of a
-// wavefront run in lockstep and the LDS serves one wave's accesses in issue order, so no
-// instruction is needed: the fences and the barrier only keep the compiler from moving
-// memory accesses across the point.
-__device__ __forceinline__ void wave_sync() {
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
 
 // Waves per SIMD asked of the compiler: the deterministic table's LDS (12.3 KB) allows only
 // 3.25 waves, and at four its registers spilled (37.28 against 37.06 ms per pass at three).
@@ -1766,7 +2084,7 @@ struct Query {
     int2 *pairs_ext;        // B * cap_candidates pairs or NULL
     int64_t chunk_ext;      // pairs per narrow-phase chunk (0: the context's)
     int ccd_blocks_per_cu;  // grid cap of k_ccd in blocks per CU (0: 128)
-    bool stack_deep;        // start with the deep traversal stack
+    const int64_t *leaf_ids; // resident: the tree when its leaves are in another order than the triangles
     long long *det_acc;     // non-NULL: impulse sums in fixed-point limbs (n * 3 * 6 * 4 per element)
 };
 
@@ -1811,70 +2129,141 @@ static unsigned persistent_grid(const ccc_context *ctx, int64_t items, int64_t B
     return (unsigned)want;
 }
 
+// The path for every tree that is not the index tree (trees of other builders, fitted trees
+// given back to the stateless calls): the tree is checked, its rightmost leaves found, and
+// k_traverse walks it with a bounded stack.
+template <typename T> class GeneralTree {
+  public:
+    GeneralTree(const Query &q, Workspace &ws, const T *bb, DevCounters *ctr, hipStream_t s, KernelTimer &tm)
+        : q_(q), ws_(ws), bb_(bb), ctr_(ctr), s_(s), tm_(tm) {}
+    bool used() const { return used_; }
+    bool deep() const { return deep_; }
+    void go_deep() { deep_ = true; }
+    ccc_status prepare() {
+        used_ = true;
+        const int64_t B = q_.B, n = q_.n, rows = 2 * n - 1, nint = n > 1 ? n - 1 : 1;
+        int *claims = ws_.get_as<int>(B * n);
+        int *rm = ws_.get_as<int>(B * nint);
+        int *lo = ws_.get_as<int>(B * nint);
+        TNode *nodes = ws_.get_as<TNode>(B * nint);
+        qnodes_ = ws_.get_as<QNode>(B * nint);
+        recs_ = ws_.get_as<LeafRec>(B * n);
+        frontier_ = ws_.get_as<Frontier>(B);
+        // one block per (start point, query block); query blocks rounded to a multiple of kXcds
+        nqb_ = (int)((grid_for(n, kTravThreads) + kXcds - 1) / kXcds * kXcds);
+        qbox_ = ws_.get_as<float>(B * (int64_t)nqb_ * 6);
+        if (ws_.failed()) return CCC_ERR_NO_MEMORY;
+        FillRegions fill;
+        fill.add(claims, B * n * 4, 0ull);
+        ccc_status st = fill_regions(fill, s_);
+        if (st != CCC_OK) return st;
+        tm_.begin("tree_prep");
+        hipLaunchKernelGGL(k_check_tree, dim3(grid_for(rows, 256), B), dim3(256), 0, s_, q_.tree, n, claims, ctr_);
+        if (n > 1) {
+            hipLaunchKernelGGL(k_ranges, dim3(grid_for(n - 1, 256), B), dim3(256), 0, s_, q_.tree, n, lo, rm, ctr_);
+            hipLaunchKernelGGL(k_order_check, dim3(grid_for(n - 1, 256), B), dim3(256), 0, s_, q_.tree, n, lo, rm, ctr_);
+        }
+        hipLaunchKernelGGL(k_rightmost, dim3(grid_for(n, 256), B), dim3(256), 0, s_, q_.tree, n, claims, rm, ctr_);
+        if (n > 1) {
+            hipLaunchKernelGGL((k_nodes<T>), dim3(grid_for(n - 1, 256), B), dim3(256), 0, s_, bb_, q_.tree, rm, n, q_.thr, nodes, ctr_);
+            hipLaunchKernelGGL(k_qnodes, dim3(grid_for(n - 1, 256), B), dim3(256), 0, s_, nodes, n, qnodes_, ctr_);
+        }
+        hipLaunchKernelGGL((k_leaf_recs<T>), dim3(grid_for(n, 256), B), dim3(256), 0, s_, bb_, q_.tree, n, recs_, ctr_);
+        hipLaunchKernelGGL((k_frontier<T>), dim3(B), dim3(kFrontier), 0, s_, bb_, q_.tree, rm, lo, n, q_.thr, frontier_, ctr_);
+        hipLaunchKernelGGL((k_qblock_boxes<T>), dim3(nqb_, B), dim3(kTravThreads), 0, s_, bb_, n, nqb_, qbox_, ctr_);
+        tm_.end();
+        CCC_LAUNCH_CHECK("tree preparation");
+        return CCC_OK;
+    }
+    ccc_status traverse(int2 *pairs, int64_t capK) {
+        const dim3 g(kFrontier * (unsigned)nqb_, (unsigned)q_.B);
+        tm_.begin("traverse");
+#define CCC_TRAVERSE(P, D)                                                                                                  \
+    hipLaunchKernelGGL((k_traverse<T, P, D>), g, dim3(kTravThreads), 0, s_, bb_, q_.tree, qnodes_, recs_, q_.n, (T)q_.thr, \
+                       q_.to_check, q_.mesh_end, pairs, capK, ctr_, frontier_, qbox_)
+        if (q_.to_check) {
+            if (deep_) CCC_TRAVERSE(true, kStackDeep);
+            else CCC_TRAVERSE(true, kStackShort);
+        } else {
+            if (deep_) CCC_TRAVERSE(false, kStackDeep);
+            else CCC_TRAVERSE(false, kStackShort);
+        }
+#undef CCC_TRAVERSE
+        tm_.end();
+        CCC_LAUNCH_CHECK("k_traverse");
+        return CCC_OK;
+    }
+
+  private:
+    const Query &q_;
+    Workspace &ws_;
+    const T *bb_;
+    DevCounters *ctr_;
+    hipStream_t s_;
+    KernelTimer &tm_;
+    bool used_ = false, deep_ = false;
+    QNode *qnodes_ = nullptr;
+    LeafRec *recs_ = nullptr;
+    Frontier *frontier_ = nullptr;
+    int nqb_ = 0;
+    float *qbox_ = nullptr;
+};
+
 template <typename T>
 static ccc_status run_query(const Query &q) {
     hipStream_t s = q.s;
     const int64_t B = q.B, n = q.n, rows = 2 * n - 1;
-    const int64_t nint = n > 1 ? n - 1 : 1;
     Workspace ws(q.ctx, s, q.arena, q.arena_bytes);
     // no event objects in the allocation-free entry point (arena without resident mode)
     KernelTimer tm(q.arena && !q.nosync ? nullptr : q.ctx, s);
+    const bool moving = q.narrow == Narrow::CCD_COLLECT || q.narrow == Narrow::CCD_IMPULSE || q.narrow == Narrow::MINCOL;
+    const int64_t nc = (n + kChunk - 1) >> kChunkBits;
     DevCounters *ctr = q.ctr_ext ? q.ctr_ext : ws.get_as<DevCounters>(B);
-    int *claims = ws.get_as<int>(B * n);
-    int *climb = ws.get_as<int>(B * nint);
-    int *rm = ws.get_as<int>(B * nint);
-    int *lo = ws.get_as<int>(B * nint);
-    TNode *nodes = ws.get_as<TNode>(B * nint);
-    QNode *qnodes = ws.get_as<QNode>(B * nint);
-    LeafRec *recs = ws.get_as<LeafRec>(B * n);
-    Frontier *frontier = ws.get_as<Frontier>(B);
+    T *chunks = ws.get_as<T>(B * nc * 6);
+    T *groups = ws.get_as<T>(B * nc * (kChunk / kPairQ) * 12);
+    T *supers = nc > kSuperFrom ? ws.get_as<T>(B * ((nc + kChunk - 1) >> kChunkBits) * 6) : nullptr;
+    T *tv = moving ? ws.get_as<T>(B * n * 18) : nullptr;
+    unsigned *foreign = q.nosync ? nullptr : ws.get_as<unsigned>(B * kForeignStep);
     if (ws.failed()) return CCC_ERR_NO_MEMORY;
     ccc_status st;
-    if ((st = fill_u64(ctr, B * (int64_t)(sizeof(DevCounters) / 8), 0ull, s)) != CCC_OK) return st;
-    if ((st = fill_u32(claims, B * n, 0u, s)) != CCC_OK) return st;
-    if ((st = fill_u32(climb, B * nint, 0u, s)) != CCC_OK) return st;
 
     // outputs start at -1 (index rows, roots) or 0 (impulses)
+    FillRegions fill;
+    fill.add(ctr, B * (int64_t)sizeof(DevCounters), 0ull);
+    if (foreign) fill.add(foreign, B * kForeignStep * 4, 0ull);
+    const uint64_t minus1 = sizeof(T) == 8 ? 0xBFF0000000000000ull : 0xBF800000BF800000ull;
+    const int64_t cells = B * q.out_cap, tsz = (int64_t)sizeof(T);
     switch (q.narrow) {
-        case Narrow::SAT: st = fill_u64(q.out_rows, B * q.out_cap * 2, ~0ull, s); break;
+        case Narrow::SAT: fill.add(q.out_rows, cells * 16, ~0ull); break;
         case Narrow::TRI_EDGE:
-            st = fill_u64(q.out_rows, B * q.out_cap * (q.te_mode == TE_CANDIDATES2 ? 2 : 4), ~0ull, s);
-            if (st == CCC_OK && q.te_mode == TE_COLLISIONS) {
-                if (sizeof(T) == 8) st = fill_u64(q.out_roots, B * q.out_cap, 0xBFF0000000000000ull, s);
-                else st = fill_u32(q.out_roots, B * q.out_cap, 0xBF800000u, s);
-            }
-            if (st == CCC_OK && q.te_mode == TE_CANDIDATES2) st = fill_u32(q.masks, B * q.out_cap * 2, 0u, s);
+            fill.add(q.out_rows, cells * (q.te_mode == TE_CANDIDATES2 ? 16 : 32), ~0ull);
+            if (q.te_mode == TE_COLLISIONS) fill.add(q.out_roots, cells * tsz, minus1);
+            if (q.te_mode == TE_CANDIDATES2) fill.add(q.masks, cells * 8, 0ull);
             break;
         case Narrow::PROXIMITY:
-        case Narrow::MINCOL: st = fill_u64(q.out_rows, B * q.out_cap * 3, ~0ull, s); break;
+        case Narrow::MINCOL: fill.add(q.out_rows, cells * 24, ~0ull); break;
         case Narrow::CCD_COLLECT:
-            st = fill_u64(q.out_rows, B * q.out_cap * 3, ~0ull, s);
-            if (st == CCC_OK) {
-                if (sizeof(T) == 8) st = fill_u64(q.out_roots, B * q.out_cap, 0xBFF0000000000000ull, s);
-                else st = fill_u32(q.out_roots, B * q.out_cap, 0xBF800000u, s);
-            }
+            fill.add(q.out_rows, cells * 24, ~0ull);
+            fill.add(q.out_roots, cells * tsz, minus1);
             break;
         case Narrow::CCD_IMPULSE:
-            if (sizeof(T) == 8) { st = fill_u64(q.dv, B * n * 9, 0ull, s); if (st == CCC_OK) st = fill_u64(q.dx, B * n * 9, 0ull, s); }
-            else { st = fill_u32(q.dv, B * n * 9, 0u, s); if (st == CCC_OK) st = fill_u32(q.dx, B * n * 9, 0u, s); }
-            if (st == CCC_OK) st = fill_u32(q.cnt, B * n * 3, 0u, s);
-            if (st == CCC_OK && q.det_acc) st = fill_u64(q.det_acc, B * n * 3 * kDetWords, 0ull, s);
+            fill.add(q.dv, B * n * 9 * tsz, 0ull);
+            fill.add(q.dx, B * n * 9 * tsz, 0ull);
+            fill.add(q.cnt, B * n * 12, 0ull);
+            if (q.det_acc) fill.add(q.det_acc, B * n * 3 * kDetWords * 8, 0ull);
             break;
     }
-    if (st != CCC_OK) return st;
+    if ((st = fill_regions(fill, s)) != CCC_OK) return st;
 
     const T *bb = (const T *)q.bboxes;
     tm.begin("tree_prep");
-    hipLaunchKernelGGL(k_check_tree, dim3(grid_for(rows, 256), B), dim3(256), 0, s, q.tree, n, claims, ctr);
-    if (n > 1) {
-        hipLaunchKernelGGL(k_ranges, dim3(grid_for(n - 1, 256), B), dim3(256), 0, s, q.tree, n, lo, rm, ctr);
-        hipLaunchKernelGGL(k_order_check, dim3(grid_for(n - 1, 256), B), dim3(256), 0, s, q.tree, n, lo, rm, ctr);
+    {
+        // a resident pass's tree was built by the pass itself
+        const unsigned gr = q.nosync ? 0u : grid_for(rows, 256), gl = grid_for(n, 256), gv = moving ? grid_for(3 * n, 256) : 0u;
+        hipLaunchKernelGGL((k_prep<T>), dim3(gr + gl + gv, B), dim3(256), 0, s, bb, q.tree, n, gr, gl, chunks, groups, (const T *)q.t0,
+                           (const T *)q.t1, tv, foreign);
+        if (supers) hipLaunchKernelGGL((k_super_boxes<T>), dim3(grid_for(nc, 256), B), dim3(256), 0, s, chunks, nc, supers);
     }
-    hipLaunchKernelGGL(k_rightmost, dim3(grid_for(n, 256), B), dim3(256), 0, s, q.tree, n, climb, rm, ctr);
-    if (n > 1) hipLaunchKernelGGL((k_nodes<T>), dim3(grid_for(n - 1, 256), B), dim3(256), 0, s, bb, q.tree, rm, n, q.thr, nodes, ctr);
-    if (n > 1) hipLaunchKernelGGL(k_qnodes, dim3(grid_for(n - 1, 256), B), dim3(256), 0, s, nodes, n, qnodes, ctr);
-    hipLaunchKernelGGL((k_leaf_recs<T>), dim3(grid_for(n, 256), B), dim3(256), 0, s, bb, q.tree, n, recs, ctr);
-    hipLaunchKernelGGL((k_frontier<T>), dim3(B), dim3(kFrontier), 0, s, bb, q.tree, rm, lo, n, q.thr, frontier, ctr);
     tm.end();
     CCC_LAUNCH_CHECK("tree preparation");
 
@@ -1883,14 +2272,13 @@ static ccc_status run_query(const Query &q) {
     int64_t capK = q.cap_candidates > 0 ? q.cap_candidates : 1;
     bool warn_cand = false;
     int2 *pairs = nullptr;
-    // one block per (start point, query block); query blocks rounded to a multiple of kXcds
-    const unsigned gT = kFrontier * (unsigned)((grid_for(n, kTravThreads) + kXcds - 1) / kXcds * kXcds);
-    const int nqb = (int)(gT / kFrontier);
-    float *qbox = ws.get_as<float>(B * (int64_t)nqb * 6);
-    if (ws.failed()) return CCC_ERR_NO_MEMORY;
-    hipLaunchKernelGGL((k_qblock_boxes<T>), dim3(nqb, B), dim3(kTravThreads), 0, s, bb, n, nqb, qbox, ctr);
-    CCC_LAUNCH_CHECK("k_qblock_boxes");
-    bool deep = q.stack_deep;   // the short stack overflowed once: run with the deep one
+    // Splits per query group: 16,384 waves in all, at least three while the groups alone do not
+    // fill the chip twice over (the longest group then ends sooner), at most one per chunk.
+    // More waves cost their reservations: 33k-triangle pass (f32) 8k waves 35 us, 16k 38, 32k 55;
+    // garment scene 1 split 230 us, 2 144, 4 113; 130k cloth 1 split 410 us, 2 383, 4 409.
+    const int64_t nq = (n + kPairQ - 1) / kPairQ, groups_all = nq * B;
+    const int splits = (int)std::max<int64_t>(1, std::min<int64_t>(nc, std::max<int64_t>(16384 / groups_all, groups_all < 16384 ? 3 : 1)));
+    GeneralTree<T> general(q, ws, bb, ctr, s, tm);
     for (int attempt = 0; attempt < 2; ++attempt) {
         if (q.pairs_ext) {
             pairs = q.pairs_ext;
@@ -1899,20 +2287,20 @@ static ccc_status run_query(const Query &q) {
             pairs = ws.get_as<int2>(B * capK);
             if (ws.failed()) return CCC_ERR_NO_MEMORY;
         }
-        tm.begin("traverse");
-#define CCC_TRAVERSE(P, D)                                                                                   \
-    hipLaunchKernelGGL((k_traverse<T, P, D>), dim3(gT, B), dim3(kTravThreads), 0, s, bb, q.tree, qnodes, recs, n, \
-                       (T)q.thr, q.to_check, q.mesh_end, pairs, capK, ctr, frontier, qbox)
-        if (q.to_check) {
-            if (deep) CCC_TRAVERSE(true, kStackDeep);
-            else CCC_TRAVERSE(true, kStackShort);
+        if (general.used()) {
+            if ((st = general.traverse(pairs, capK)) != CCC_OK) return st;
         } else {
-            if (deep) CCC_TRAVERSE(false, kStackDeep);
-            else CCC_TRAVERSE(false, kStackShort);
+            tm.begin("traverse");
+            const dim3 g((unsigned)((nq * splits + kPairWaves - 1) / kPairWaves), (unsigned)B);
+            if (q.to_check)
+                hipLaunchKernelGGL((k_pairs<T, true>), g, dim3(64 * kPairWaves), 0, s, bb, q.leaf_ids, n, (T)q.thr, chunks, supers, groups, splits, q.to_check,
+                                   q.mesh_end, pairs, capK, foreign, ctr);
+            else
+                hipLaunchKernelGGL((k_pairs<T, false>), g, dim3(64 * kPairWaves), 0, s, bb, q.leaf_ids, n, (T)q.thr, chunks, supers, groups, splits, q.to_check,
+                                   q.mesh_end, pairs, capK, foreign, ctr);
+            tm.end();
+            CCC_LAUNCH_CHECK("k_pairs");
         }
-#undef CCC_TRAVERSE
-        tm.end();
-        CCC_LAUNCH_CHECK("k_traverse");
         if (q.nosync) break;          // the caller checks the counters after its step
         CCC_HIP_TRY(hipMemcpyAsync(h.data(), ctr, sizeof(DevCounters) * B, hipMemcpyDeviceToHost, s));
         CCC_HIP_TRY(hipStreamSynchronize(s));
@@ -1923,16 +2311,20 @@ static ccc_status run_query(const Query &q) {
             kmax = std::max(kmax, h[b].cand);
         }
         if (flags & DEV_BAD_TREE) { set_error("tree tensor is not a valid BVH over n leaves"); return CCC_ERR_BAD_TREE; }
-        if (flags & DEV_STACK) {
-            if (deep) { set_error("BVH deeper than the traversal stack"); return CCC_ERR_STACK; }
-            // again with the deep stack (not a capacity attempt)
-            deep = true;
-            --attempt;
+        if ((flags & DEV_STACK) && general.deep()) { set_error("BVH deeper than the traversal stack"); return CCC_ERR_STACK; }
+        if (flags & (DEV_STACK | DEV_FOREIGN)) {
+            // again with the deep stack, or by the general path (not a capacity attempt)
             for (int64_t b = 0; b < B; ++b) {
                 h[b].cand = 0;
-                h[b].flags &= ~DEV_STACK;
+                h[b].flags &= ~(DEV_STACK | DEV_FOREIGN);
             }
             CCC_HIP_TRY(hipMemcpyAsync(ctr, h.data(), sizeof(DevCounters) * B, hipMemcpyHostToDevice, s));
+            if (flags & DEV_STACK) general.go_deep();
+            else {
+                if (!q.pairs_ext) { ws.release(pairs); pairs = nullptr; }   // the list follows the tree's buffers
+                if ((st = general.prepare()) != CCC_OK) return st;
+            }
+            --attempt;
             continue;
         }
         if (kmax <= (unsigned long long)capK) break;
@@ -1968,12 +2360,8 @@ static ccc_status run_query(const Query &q) {
         tm.end();
         CCC_LAUNCH_CHECK("k_tri_edge");
     } else if (q.narrow == Narrow::MINCOL) {
-        T *tv = ws.get_as<T>(B * n * 18);
-        if (ws.failed()) return CCC_ERR_NO_MEMORY;
         const unsigned gS = persistent_grid(q.ctx, (kmax + kSubprimPairs - 1) / kSubprimPairs, B);
         tm.begin("mincol");
-        hipLaunchKernelGGL((k_vertex_records<T>), dim3(grid_for(3 * n, 256), B), dim3(256), 0, s, (const T *)q.t0,
-                           (const T *)q.t1, 3 * n, tv);
         hipLaunchKernelGGL((k_subprim<T, SUB_MINCOL, kSubprimPairs>), dim3(gS, B), dim3(kThreads), 0, s, pairs, capK,
                            (int64_t)0, capK, (const T *)tv, n, thr, q.out_rows, q.out_cap, ctr);
         tm.end();
@@ -1983,9 +2371,6 @@ static ccc_status run_query(const Query &q) {
         // chunk bounds the pairs of all batch elements together (the item buffer holds B
         // chunks), so the workspace does not grow with the batch
         int64_t chunk = pair_chunk_of(q.ctx, q.chunk_ext, kmax, B, item_bytes(q.narrow));
-        const bool ccd = q.narrow == Narrow::CCD_COLLECT || q.narrow == Narrow::CCD_IMPULSE;
-        T *tv = ccd ? ws.get_as<T>(B * n * 18) : nullptr;
-        if (ws.failed()) return CCC_ERR_NO_MEMORY;
         if (ws.arena()) {
             // the item list takes what the arena has left (results do not depend on the chunk)
             const int64_t fit = (int64_t)(ws.arena_left() / ((size_t)B * 15 * item_bytes(q.narrow)));
@@ -2006,11 +2391,6 @@ static ccc_status run_query(const Query &q) {
         const unsigned gCcdI = persistent_grid(q.ctx, capM, B, ccd_threads<MODE_IMPULSE>(),
                                                q.ccd_blocks_per_cu > 0 ? q.ccd_blocks_per_cu : 128);
         if (ws.failed()) return CCC_ERR_NO_MEMORY;
-        if (ccd) {
-            hipLaunchKernelGGL((k_vertex_records<T>), dim3(grid_for(3 * n, 256), B), dim3(256), 0, s, (const T *)q.t0,
-                               (const T *)q.t1, 3 * n, tv);
-            CCC_LAUNCH_CHECK("k_vertex_records");
-        }
         auto narrow_phase = [&]() -> ccc_status {
             for (int64_t c0 = 0; c0 < kmax; c0 += chunk) {
                 const int64_t c1 = c0 + chunk;
@@ -2078,15 +2458,13 @@ static ccc_status run_query(const Query &q) {
 // Workspace bytes of a resident CCD_IMPULSE pass (nosync, caller-owned counters and pair
 // list): the same buffers, sizes and 256-byte rounding as run_query's requests.
 static size_t resident_bytes(const Query &q) {
-    const int64_t B = q.B, n = q.n, nint = n > 1 ? n - 1 : 1;
+    const int64_t B = q.B, n = q.n, nc = (n + kChunk - 1) >> kChunkBits;
     const size_t esz = q.dtype == CCC_FLOAT64 ? 8 : 4;
     auto r = [](size_t b) { return ((b ? b : 256) + 255) & ~(size_t)255; };
     size_t tot = 0;
     if (!q.ctr_ext) tot += r(sizeof(DevCounters) * B);
-    tot += r(4 * B * n) + 3 * r(4 * B * nint);
-    tot += r(sizeof(TNode) * B * nint) + r(sizeof(QNode) * B * nint) + r(sizeof(LeafRec) * B * n) + r(sizeof(Frontier) * B);
-    const unsigned gT = kFrontier * (unsigned)((grid_for(n, kTravThreads) + kXcds - 1) / kXcds * kXcds);
-    tot += r(sizeof(float) * B * (int64_t)(gT / kFrontier) * 6);
+    tot += r(esz * B * nc * 6) + r(esz * B * nc * (kChunk / kPairQ) * 12);
+    if (nc > kSuperFrom) tot += r(esz * B * ((nc + kChunk - 1) >> kChunkBits) * 6);
     const int64_t capK = q.cap_candidates > 0 ? q.cap_candidates : 1;
     if (!q.pairs_ext) tot += r(sizeof(int2) * B * capK);
     const int64_t chunk = pair_chunk_of(q.ctx, q.chunk_ext, capK, B, item_bytes(q.narrow));
@@ -2119,7 +2497,7 @@ static Query resident_query(ccc_context *ctx, const ResidentPass &p, hipStream_t
     q.pairs_ext = p.pairs;
     q.chunk_ext = p.chunk;
     q.ccd_blocks_per_cu = p.ccd_blocks_per_cu;
-    q.stack_deep = p.stack_deep;
+    q.leaf_ids = p.leaf_ids;
     q.det_acc = p.det_acc;
     return q;
 }
@@ -2159,10 +2537,11 @@ template <typename T>
 static ccc_status from_collisions(ccc_context *ctx, const int64_t *coll, const void *roots, int64_t m, const void *t0,
                                   const void *t1, const void *masses, int64_t B, int64_t n, void *dv, void *dx, int32_t *cnt,
                                   hipStream_t s) {
-    ccc_status st;
-    if (sizeof(T) == 8) { st = fill_u64(dv, B * n * 9, 0ull, s); if (st == CCC_OK) st = fill_u64(dx, B * n * 9, 0ull, s); }
-    else { st = fill_u32(dv, B * n * 9, 0u, s); if (st == CCC_OK) st = fill_u32(dx, B * n * 9, 0u, s); }
-    if (st == CCC_OK) st = fill_u32(cnt, B * n * 3, 0u, s);
+    FillRegions fill;
+    fill.add(dv, B * n * 9 * (int64_t)sizeof(T), 0ull);
+    fill.add(dx, B * n * 9 * (int64_t)sizeof(T), 0ull);
+    fill.add(cnt, B * n * 12, 0ull);
+    const ccc_status st = fill_regions(fill, s);
     if (st != CCC_OK) return st;
     KernelTimer tm(ctx, s);
     if (m > 0) {

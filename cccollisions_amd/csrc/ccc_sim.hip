@@ -16,9 +16,8 @@
 // simulation's own, or one the caller passes, e.g. a serving slot's), the candidate list has
 // a fixed capacity and the narrow phase a fixed number of chunks.  The step can therefore be
 // captured once in a HIP graph and replayed.  After each step the host reads the per-pass
-// counters once: if a pass found more candidate pairs than the list holds, or its traversal
-// needed the deep stack, the capacity (or stack) grows and the step runs again from the
-// saved x1.
+// counters once: if a pass found more candidate pairs than the list holds, the list grows and
+// the step runs again from the saved x1.
 #include <algorithm>
 #include <chrono>
 #include <cmath>
@@ -126,7 +125,6 @@ struct ccc_sim {
     DevCounters *h_ctr = nullptr;         // pinned host copy of the per-pass counters
     void *arena = nullptr;                // own workspace (allocated at the first step that needs it)
     size_t arena_bytes = 0;
-    bool deep = false;
     // graphs, one per workspace arena the steps ran with
     hipStream_t cs = nullptr;             // capture stream
     std::map<void *, std::pair<hipGraph_t, hipGraphExec_t>> graphs;
@@ -175,7 +173,7 @@ static ResidentPass pass_of(const ccc_sim *s, int it) {
     p.cap_pairs = s->cap_pairs;
     p.chunk = s->o.pair_chunk > 0 ? s->o.pair_chunk : 0;
     p.ccd_blocks_per_cu = s->o.ccd_blocks_per_cu;
-    p.stack_deep = s->deep;
+    p.leaf_ids = s->meshes == 1 && s->o.morton != CCC_MORTON_COMPAT ? s->tree : nullptr;
     p.det_acc = s->det_acc;
     p.dv = s->dv;
     p.dx = s->dx;
@@ -294,19 +292,10 @@ static ccc_status run_step(ccc_sim *s, void *arena, size_t bytes, hipStream_t st
         const int iters = s->o.iters;
         CCC_HIP_TRY(hipMemcpyAsync(s->h_ctr, s->ctr, sizeof(DevCounters) * iters, hipMemcpyDeviceToHost, st));
         CCC_HIP_TRY(hipStreamSynchronize(st));
-        unsigned flags = 0;
         unsigned long long kmax = 0;
-        for (int i = 0; i < iters; ++i) {
-            flags |= s->h_ctr[i].flags;
-            kmax = std::max(kmax, s->h_ctr[i].cand);
-        }
-        if (flags & DEV_BAD_TREE) {
-            set_error("internal error: the step's tree is not a valid BVH");
-            return CCC_ERR_BAD_TREE;
-        }
-        const bool stack = (flags & DEV_STACK) != 0;
+        for (int i = 0; i < iters; ++i) kmax = std::max(kmax, s->h_ctr[i].cand);
         const bool over = kmax > (unsigned long long)s->cap_pairs;
-        if (!stack && !over) {
+        if (!over) {
             s->counts.assign(iters, ccc_counts{});
             for (int i = 0; i < iters; ++i) {
                 s->counts[i].candidates = (int64_t)s->h_ctr[i].cand;
@@ -316,17 +305,10 @@ static ccc_status run_step(ccc_sim *s, void *arena, size_t bytes, hipStream_t st
             }
             return CCC_OK;
         }
-        if (stack && s->deep) {
-            set_error("BVH deeper than the traversal stack");
-            return CCC_ERR_STACK;
-        }
-        // the step ran on a truncated list or a failed traversal: grow, restore x1, again
+        // the step ran on a truncated list: grow, restore x1, again
         drop_graphs(s);
-        if (stack) s->deep = true;
-        if (over) {
-            r = grow_pairs(s, (int64_t)(kmax + kmax / 4 + 1024));
-            if (r != CCC_OK) return r;
-        }
+        r = grow_pairs(s, (int64_t)(kmax + kmax / 4 + 1024));
+        if (r != CCC_OK) return r;
         r = s->dtype == CCC_FLOAT64 ? restore_x1<double>(s, st) : restore_x1<float>(s, st);
         if (r != CCC_OK) return r;
     }

@@ -1,0 +1,77 @@
+"""Candidate pairs by chunks of 64 leaf positions, at chunk edges and ragged ends: against the
+oracle's traversal, and against the general tree walk, which the same boxes take when the
+tree's internal rows are numbered differently (the pair sets must be equal)."""
+import numpy as np
+import pytest
+
+from tests import cases
+from tests.conftest import sorted_rows, valid_rows
+from tests.test_gpu_parity import _np, _renumbered_internal_tree, _t
+
+pytestmark = pytest.mark.gpu
+
+
+def _mincol(ccc, bb, tree, t0, t1, cap):
+    out = _np(ccc.find_mincol_cand(_t(bb[None]), _t(tree[None]), _t(t0[None]), _t(t1[None]), cap))[0]
+    return sorted_rows(valid_rows(out)), ccc.last_counts()[0][0]
+
+
+@pytest.mark.parametrize("dtype", [np.float64, np.float32])
+@pytest.mark.parametrize("n", [2, 3, 63, 64, 65, 127, 129, 200, 1000, 4097])
+def test_pairs_at_chunk_edges(ccc, oracle, n, dtype):
+    t0, t1, _ = cases.random_soup(n, seed=n + 1, dtype=dtype)
+    rb, rt, _, _ = oracle.bvh(t0, t1)
+    pairs, total = oracle.traverse(rb, rt, 0.0)
+    want = sorted_rows(oracle.mincol(t0, t1, pairs))
+    cap = total // n + 2
+    rows, k = _mincol(ccc, rb, rt, t0, t1, cap)
+    assert k == total
+    np.testing.assert_array_equal(rows, want)
+    if n > 3:
+        rows, k = _mincol(ccc, *_renumbered_internal_tree(rb, rt, 2), t0, t1, cap)
+        assert k == total
+        np.testing.assert_array_equal(rows, want)
+
+
+@pytest.mark.parametrize("n", [65, 300])
+def test_partial_pairs(ccc, oracle, n):
+    t0, t1, _ = cases.random_soup(n, seed=n)
+    rb, rt, _, _ = oracle.bvh(t0, t1)
+    for share in (0.0, 0.03, 0.5, 1.0):
+        check = np.random.default_rng(7).random(n) < share
+        total = len(oracle.traverse_partial(rb, rt, check))
+        counts = []
+        for bb, tree in ((rb, rt), _renumbered_internal_tree(rb, rt, 3)):
+            ccc.find_collisions_continuous_partial(_t(bb[None]), _t(tree[None]), _t(t0[None]), _t(t1[None]), _t(check[None]), 400, 400)
+            counts.append(ccc.last_counts()[0])
+        assert counts[0] == counts[1] and counts[0][0] == total
+
+
+def test_pairs_with_super_boxes(ccc, oracle):
+    """More than 4,096 chunks: groups of 64 chunks are tested first."""
+    n = 64 * 4096 + 77
+    rng = np.random.default_rng(3)
+    c = rng.random((n, 1, 3))
+    c = c[np.argsort(np.floor(c[:, 0, 0] * 40) * 1000 + c[:, 0, 1])]
+    t0 = c + 0.004 * rng.standard_normal((n, 3, 3))
+    t1 = t0 + 0.002 * rng.standard_normal((n, 3, 3))
+    rb, rt, _, _ = oracle.bvh(t0, t1)
+    pairs, total = oracle.traverse(rb, rt, 0.0)
+    assert total > n // 4
+    rows, k = _mincol(ccc, rb, rt, t0, t1, total // n + 2)
+    assert k == total
+    np.testing.assert_array_equal(rows, sorted_rows(oracle.mincol(t0, t1, pairs)))
+
+
+def test_special_boxes(ccc, oracle):
+    """NaN triangles meet nothing; infinite ones meet everything on their axis."""
+    t0, t1, _ = cases.random_soup(200, seed=8)
+    t0[5], t1[5] = np.nan, np.nan
+    t0[64:128, :, 1], t1[64:128, :, 1] = np.nan, np.nan
+    t0[150, 0] = np.inf
+    t1[151, 1] = -np.inf
+    rb, rt, _, _ = oracle.bvh(t0, t1)
+    _, total = oracle.traverse(rb, rt, 0.0)
+    for bb, tree in ((rb, rt), _renumbered_internal_tree(rb, rt, 2)):
+        _, k = _mincol(ccc, bb, tree, t0, t1, 200)
+        assert k == total

@@ -177,10 +177,20 @@ struct alignas(64) DevCounters {
     unsigned long long roots;   // V
     unsigned long long coll;    // R (total, may exceed the output capacity)
     unsigned long long items_done;  // M of the pair chunks already finished
+    unsigned long long tiles;   // item tiles of the current pair chunk (continuous narrow phase)
     unsigned int flags;         // DEV_* bits
-    unsigned int pad[5];
+    unsigned int pad[3];
 };
 static_assert(sizeof(DevCounters) == 64, "DevCounters is one 64-byte line");
+
+// Counts that nobody reads before the call ends: every block of the narrow phase adds its own
+// to one of kPartials lines, and k_fold_items sums them.  An atomic on one device address
+// takes 6-13 ns however many waves issue them: on the shared counters the 32,768 blocks of
+// k_ccd spent 0.4-0.8 ms of a pass on two of them each (all of its time on the 33k f32 pass).
+struct alignas(128) DevPartial {
+    unsigned long long items, roots, coll;
+};
+constexpr int kPartials = 64;
 
 // Device address of the allocation-free entry point's scratch array on `device` (looked up
 // once per device with that device current, then cached).

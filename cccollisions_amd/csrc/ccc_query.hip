@@ -1026,18 +1026,13 @@ __global__ __launch_bounds__(64 * kPairWaves) void k_pairs(const T *__restrict__
 // Candidate pairs -> the pairs of sub-primitives (9 edge-edge, 6 vertex-face) whose boxes
 // overlap, with PP pairs per thread and one reservation per PP * kThreads pairs (the item
 // counter is one contended device address: every reservation is a returning atomic on it).
-//   SUB_MOVING: swept boxes (collisions_continuous.cu:234-318, :340-396) -> packed items;
 //   SUB_STATIC: boxes grown by the threshold (proximity_static.cu:11-118) -> packed items;
 //   SUB_MINCOL: swept boxes, written as (x, y, type) rows (find_minimal_candidates, :321-338).
 // Items stay in pair order: pair u * kThreads + t of a tile comes after every pair
-// u' * kThreads + t' < u * kThreads + t.  SUB_MOVING writes a tile's edge-edge items first and
-// its vertex-face items after them, each in pair order, so that the narrow phase's 64-item
-// tiles hold one kind except where the kind changes (about 3% of them on the 130k cloth),
-// while a pair's items of both kinds stay close together in the list (their vertex records
-// are read again while still in the caches).  The moving masks come from the vertex records
-// (moving_mask_axes).  A tile's items are assembled in LDS (a 2-byte entry per item: pair in
-// tile and type) and written as one contiguous run.
-enum { SUB_MOVING = 0, SUB_STATIC = 1, SUB_MINCOL = 2 };
+// u' * kThreads + t' < u * kThreads + t.  A tile's items are assembled in LDS (a 2-byte entry
+// per item: pair in tile and type) and written as one contiguous run.  The moving pairs of
+// the continuous narrow phase go through k_items.
+enum { SUB_STATIC = 0, SUB_MINCOL = 1 };
 // Exclusive block-wide scan of cnt (< 16) over the NT threads in thread order, without a
 // reservation: the thread's offset; the block's sum in `total`.  Every thread calls it.
 template <int NT = kThreads>
@@ -1060,51 +1055,13 @@ __device__ __forceinline__ unsigned block_scan_excl(unsigned cnt, unsigned &tota
     return before + below;
 }
 
-// Two exclusive block-wide scans in one pass: counts a < 16 and b < 8 per thread; returns the
-// thread's offsets packed as (a offset) | (b offset) << 16 and the block's sums packed the
-// same way in `total` (a block sum stays below 2^16: at most 15 * NT).  Every thread calls it.
-template <int NT = kThreads>
-__device__ __forceinline__ unsigned block_scan_excl2(unsigned a, unsigned b, unsigned &total) {
-    static_assert(15 * NT < 65536, "packed halves do not carry");
-    __shared__ unsigned s_part[NT / 64 + 1];
-    const int w = threadIdx.x >> 6, lane = threadIdx.x & 63;
-    unsigned below = 0, mine = 0;
-#pragma unroll
-    for (int bit = 0; bit < 4; ++bit) {
-        const unsigned long long m = __ballot((a >> bit) & 1u);
-        below += lanes_below(m) << bit;
-        mine += (unsigned)__popcll(m) << bit;
-    }
-#pragma unroll
-    for (int bit = 0; bit < 3; ++bit) {
-        const unsigned long long m = __ballot((b >> bit) & 1u);
-        below += lanes_below(m) << (16 + bit);
-        mine += (unsigned)__popcll(m) << (16 + bit);
-    }
-    if (lane == 0) s_part[w] = mine;
-    __syncthreads();
-    unsigned before = 0, tot = 0;
-#pragma unroll
-    for (int q = 0; q < NT / 64; ++q) {
-        const unsigned v = s_part[q];
-        if (q < w) before += v;
-        tot += v;
-    }
-    __syncthreads();
-    total = tot;
-    return before + below;
-}
-
 template <typename T, int KIND, int PP>
 __global__ __launch_bounds__(kThreads) void k_subprim(const int2 *__restrict__ pairs_all, int64_t capK, int64_t c0, int64_t c1,
                                                       const T *__restrict__ src_all, int64_t n, T thr,
                                                       void *__restrict__ out_all, int64_t capM,
                                                       DevCounters *__restrict__ ctr_all) {
     static_assert(PP >= 1 && PP * kThreads <= 4096, "pair index and type fit 16 bits");
-    // (pair in tile) << 4 | type; SUB_MOVING: edge-edge entries from the front, vertex-face
-    // entries from the back (at most 9 and 6 per pair: the two runs never meet)
-    constexpr int kEnt = 15 * PP * kThreads;
-    constexpr bool SPLIT = KIND == SUB_MOVING;
+    constexpr int kEnt = 15 * PP * kThreads;      // (pair in tile) << 4 | type
     __shared__ unsigned short s_ent[kEnt];
     __shared__ int2 s_pair[PP * kThreads];
     __shared__ unsigned long long s_base;
@@ -1116,13 +1073,11 @@ __global__ __launch_bounds__(kThreads) void k_subprim(const int2 *__restrict__ p
     const int2 *pairs = pairs_all + (int64_t)b * capK;
     // SUB_STATIC: the t0 soup; otherwise the vertex records [x0 y0 z0 dx dy dz] per corner
     const T *src = src_all + (int64_t)b * n * (KIND == SUB_STATIC ? 9 : 18);
-    // SUB_MOVING: 32-bit items (pair index within the chunk) << 4 | type; the others 64-bit
-    int64_t *out = SPLIT ? nullptr : static_cast<int64_t *>(out_all) + (int64_t)b * capM * (KIND == SUB_MINCOL ? 3 : 1);
-    uint32_t *out32 = SPLIT ? static_cast<uint32_t *>(out_all) + (int64_t)b * capM : nullptr;
+    int64_t *out = static_cast<int64_t *>(out_all) + (int64_t)b * capM * (KIND == SUB_MINCOL ? 3 : 1);
     constexpr int kTile = PP * kThreads;
     const int64_t ntiles = K > c0 ? (K - c0 + kTile - 1) / kTile : 0;
     CCC_FOR_TILES(tile, ntiles) {
-        unsigned tot = 0, tot_vf = 0;
+        unsigned tot = 0;
 #pragma unroll
         for (int u = 0; u < PP; ++u) {
             const int64_t i = c0 + tile * kTile + u * kThreads + tid;
@@ -1141,70 +1096,137 @@ __global__ __launch_bounds__(kThreads) void k_subprim(const int2 *__restrict__ p
                     mask = moving_mask_axes(src, x, y);
                 }
             }
-            if (!SPLIT) s_pair[u * kThreads + tid] = make_int2(x, y);
-            if (SPLIT) {
-                uint32_t mee = mask & 0x1ffu, mvf = mask >> 9;
-                unsigned t;
-                const unsigned k2 = block_scan_excl2((unsigned)__popc(mee), (unsigned)__popc(mvf), t);
-                unsigned ke = tot + (k2 & 0xffffu), kv = tot_vf + (k2 >> 16);
-                tot += t & 0xffffu;
-                tot_vf += t >> 16;
-                while (mee) {
-                    const int type = __ffs(mee) - 1;
-                    mee &= mee - 1;
-                    s_ent[ke++] = (unsigned short)(((u * kThreads + tid) << 4) | type);
-                }
-                while (mvf) {
-                    const int type = 9 + __ffs(mvf) - 1;
-                    mvf &= mvf - 1;
-                    s_ent[kEnt - 1 - kv++] = (unsigned short)(((u * kThreads + tid) << 4) | type);
-                }
-            } else {
-                unsigned t;
-                unsigned k = tot + block_scan_excl((unsigned)__popc(mask), t);
-                tot += t;
-                while (mask) {
-                    const int type = __ffs(mask) - 1;
-                    mask &= mask - 1;
-                    s_ent[k++] = (unsigned short)(((u * kThreads + tid) << 4) | type);
-                }
+            s_pair[u * kThreads + tid] = make_int2(x, y);
+            unsigned t;
+            unsigned k = tot + block_scan_excl((unsigned)__popc(mask), t);
+            tot += t;
+            while (mask) {
+                const int type = __ffs(mask) - 1;
+                mask &= mask - 1;
+                s_ent[k++] = (unsigned short)(((u * kThreads + tid) << 4) | type);
             }
         }
-        if (tid == 0) {
-            const unsigned all = tot + tot_vf;
-            s_base = all ? atomicAdd(&ctr->items, (unsigned long long)all) : 0ull;
-        }
+        if (tid == 0) s_base = tot ? atomicAdd(&ctr->items, (unsigned long long)tot) : 0ull;
         __syncthreads();
         const unsigned long long base = s_base;
         const unsigned long long room = base < (unsigned long long)capM ? (unsigned long long)capM - base : 0ull;
         const unsigned lim = room < tot ? (unsigned)room : tot;
-        const uint32_t tile_pair = (uint32_t)(tile * kTile);     // < 2^28: the chunk's pairs
         for (unsigned k = tid; k < lim; k += kThreads) {
             const unsigned e = s_ent[k];
             const unsigned long long slot = base + k;
-            if (SPLIT) {
-                out32[slot] = ((tile_pair + (e >> 4)) << 4) | (e & 15u);
+            const int2 pr = s_pair[e >> 4];
+            if (KIND == SUB_MINCOL) {
+                out[3 * slot] = pr.x; out[3 * slot + 1] = pr.y; out[3 * slot + 2] = (int64_t)(e & 15u);
             } else {
-                const int2 pr = s_pair[e >> 4];
-                if (KIND == SUB_MINCOL) {
-                    out[3 * slot] = pr.x; out[3 * slot + 1] = pr.y; out[3 * slot + 2] = (int64_t)(e & 15u);
-                } else {
-                    out[slot] = pack_item(pr.x, pr.y, (int)(e & 15u));
-                }
-            }
-        }
-        if (SPLIT) {
-            // vertex-face item j of the tile follows its tot edge-edge items
-            const unsigned long long bv = base + tot;
-            const unsigned long long rv = bv < (unsigned long long)capM ? (unsigned long long)capM - bv : 0ull;
-            const unsigned limv = rv < tot_vf ? (unsigned)rv : tot_vf;
-            for (unsigned k = tid; k < limv; k += kThreads) {
-                const unsigned e = s_ent[kEnt - 1 - k];
-                out32[bv + k] = ((tile_pair + (e >> 4)) << 4) | (e & 15u);
+                out[slot] = pack_item(pr.x, pr.y, (int)(e & 15u));
             }
         }
         __syncthreads();
     }
+}
+
+// ---- items of the continuous narrow phase ---------------------------------------------------
+// Moving candidate pairs -> the sub-primitive pairs whose swept boxes overlap
+// (collisions_continuous.cu:234-318, :340-396), as 32-bit items (pair index within the chunk)
+// << 4 | type for k_ccd.
+// Each wave takes a contiguous run of pairs, 64 at a time (lane = pair), and keeps its
+// edge-edge items in its own kSegEE slots per pair and its vertex-face items in the kSegVF
+// behind them, so that k_ccd's 64-item tiles hold one kind and nothing is reserved while it
+// runs; at the end the block reserves its tiles' descriptors (first slot, a multiple of 64,
+// plus the number of items less one), which is all that k_ccd needs to find them.  A batch's
+// entries are assembled in LDS and written as whole lines.  Bound by VALU issue (about 600
+// instructions per 64 pairs, most of them comparisons): 1.11 ms per pass of the 130k cloth
+// (1.20 with blocks of 512 pairs and one reservation each), 33k f32 pass 56 -> 42 us.
+constexpr int kBatch = 64;       // pairs per wave at a time
+constexpr int kSegEE = 9, kSegVF = 6;
+constexpr int kItemBlock = 4;    // waves per block
+
+template <typename T>
+__global__ __launch_bounds__(64 * kItemBlock) void k_items(const int2 *__restrict__ pairs_all, int64_t capK, int64_t c0, int64_t c1,
+                                              const T *__restrict__ tv_all, int64_t n, uint32_t *__restrict__ list_all, int64_t capM,
+                                              unsigned slot_run, uint32_t *__restrict__ tile_all, int64_t capT,
+                                              DevPartial *__restrict__ part_all, DevCounters *__restrict__ ctr_all) {
+    // (pair in batch) << 4 | type: edge-edge entries from the front, vertex-face ones from kSegEE kBatch on
+    __shared__ unsigned short s_ents[kItemBlock][(kSegEE + kSegVF) * kBatch];
+    __shared__ unsigned s_tiles[kItemBlock];
+    const int b = blockIdx.y, lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    unsigned short *s_ent = s_ents[w];
+    const unsigned long long kc = ctr_all[b].cand;
+    int64_t K = (int64_t)(kc < (unsigned long long)capK ? kc : (unsigned long long)capK);
+    if (K > c1) K = c1;         // this launch covers the pairs [c0, c1)
+    const int64_t nbatch = K > c0 ? (K - c0 + kBatch - 1) / kBatch : 0;
+    // the XCD's contiguous share of the batches, and this wave's run of it
+    const int64_t per = (nbatch + kXcds - 1) / kXcds, step = (int64_t)gridDim.x / kXcds * kItemBlock, run = (per + step - 1) / step;
+    const int64_t base = (int64_t)(blockIdx.x % kXcds) * per, k0 = ((int64_t)(blockIdx.x / kXcds) * kItemBlock + w) * run;
+    const int64_t first = base + k0, last = base + (k0 + run < per ? k0 + run : per), stop = last < nbatch ? last : nbatch;
+    const unsigned wave = blockIdx.x * kItemBlock + w;
+    const int2 *pairs = pairs_all + (int64_t)b * capK + c0;
+    const T *tv = tv_all + (int64_t)b * n * 18;
+    // slot_run >= run: the batches per wave that the list was sized for
+    const uint32_t slot_ee = wave * ((kSegEE + kSegVF) * kBatch * slot_run), slot_vf = slot_ee + kSegEE * kBatch * slot_run;
+    uint32_t *list_ee = list_all + (int64_t)b * capM + slot_ee, *list_vf = list_all + (int64_t)b * capM + slot_vf;
+    unsigned nee = 0, nvf = 0;      // items in the two segments
+    int2 pr = make_int2(0, 0);
+    if (first < stop && first * kBatch + lane < K - c0) pr = pairs[first * kBatch + lane];
+    for (int64_t bt = first; bt < stop; ++bt) {
+        const int64_t i = bt * kBatch + lane;
+        uint32_t mask = 0;
+        if (i < K - c0) mask = moving_mask_axes(tv, pr.x, pr.y);
+        if (bt + 1 < stop && i + kBatch < K - c0) pr = pairs[i + kBatch];      // on its way for the next round
+        // the batch's entries, each kind in pair order
+        uint32_t mee = mask & 0x1ffu, mvf = mask >> 9;
+        const unsigned ce = (unsigned)__popc(mee), cv = (unsigned)__popc(mvf);
+        unsigned ke = 0, kv = 0, te = 0, tvf = 0;
+#pragma unroll
+        for (int bit = 0; bit < 4; ++bit) {
+            const unsigned long long m = __ballot((ce >> bit) & 1u);
+            ke += lanes_below(m) << bit;
+            te += (unsigned)__popcll(m) << bit;
+        }
+#pragma unroll
+        for (int bit = 0; bit < 3; ++bit) {
+            const unsigned long long m = __ballot((cv >> bit) & 1u);
+            kv += lanes_below(m) << bit;
+            tvf += (unsigned)__popcll(m) << bit;
+        }
+        while (mee) {
+            const int type = __ffs(mee) - 1;
+            mee &= mee - 1;
+            s_ent[ke++] = (unsigned short)((lane << 4) | type);
+        }
+        kv += kSegEE * kBatch;
+        while (mvf) {
+            const int type = 9 + __ffs(mvf) - 1;
+            mvf &= mvf - 1;
+            s_ent[kv++] = (unsigned short)((lane << 4) | type);
+        }
+        wave_sync();
+        const uint32_t code = (uint32_t)(bt * kBatch) << 4;      // < 2^32: the chunk holds at most 2^28 pairs
+        for (unsigned k = lane; k < te; k += 64) list_ee[nee + k] = code + s_ent[k];
+        for (unsigned k = lane; k < tvf; k += 64) list_vf[nvf + k] = code + s_ent[kSegEE * kBatch + k];
+        nee += te;
+        nvf += tvf;
+        wave_sync();
+    }
+    const unsigned tee = (nee + 63u) >> 6, tvf = (nvf + 63u) >> 6;
+    if (lane == 0) s_tiles[w] = tee + tvf;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        unsigned sum = 0;
+        for (int k = 0; k < kItemBlock; ++k) {
+            const unsigned t = s_tiles[k];
+            s_tiles[k] = sum;
+            sum += t;
+        }
+        const unsigned at = sum ? (unsigned)atomicAdd(&ctr_all[b].tiles, (unsigned long long)sum) : 0u;
+        for (int k = 0; k < kItemBlock; ++k) s_tiles[k] += at;
+    }
+    __syncthreads();
+    uint32_t *tiles = tile_all + (int64_t)b * capT + s_tiles[w];
+    for (unsigned k = lane; k < tee; k += 64) tiles[k] = slot_ee + 64 * k + (nee - 64 * k < 64u ? nee - 64 * k - 1u : 63u);
+    for (unsigned k = lane; k < tvf; k += 64) tiles[tee + k] = slot_vf + 64 * k + (nvf - 64 * k < 64u ? nvf - 64 * k - 1u : 63u);
+    if (lane == 0 && nee + nvf > 0)
+        atomicAdd(&part_all[(int64_t)b * kPartials + blockIdx.x % kPartials].items, (unsigned long long)(nee + nvf));
 }
 
 // ---- fused narrow phase --------------------------------------------------------------------
@@ -1264,8 +1286,10 @@ __device__ __forceinline__ void scatter_impulse(const MTet<T> &m, int type, T ro
 // the additions (2^21 additions per limb fit in 64 bits).  Values that cannot be held set
 // flag bits in a fourth word instead: 1 NaN, 2 +inf, 4 -inf, 8 out of range; the result
 // is then what an fp64 sum gives (NaN, or the infinity) and NaN when out of range.
-// Per triangle corner: 6 components (dv xyz, dx xyz) x 4 words.
+// Per triangle corner: 6 components (dv xyz, dx xyz) x 4 words; the upper half of the first
+// component's flag word is the corner's collision count.
 constexpr int kDetWords = kDetWordsPerCorner;
+constexpr unsigned long long kDetOne = 1ull << 32;      // one collision in that word
 constexpr double kTwo42 = 4398046511104.0, kTwo45 = 35184372088832.0, kTwo80 = 1208925819614629174706176.0;
 
 // The three limbs of v (returns 0), or its flag bit when v cannot be held.
@@ -1300,10 +1324,12 @@ __device__ __forceinline__ void det_add1(long long *a, double v) {
 // Limbs -> dv / dx of every corner: carries normalise the two low limbs into [0, 2^42),
 // then hi * 2^84 + mid * 2^42 + lo is formed in double in that order and scaled by 2^-80.
 template <typename T>
-__global__ void k_det_finalize(const long long *__restrict__ acc, int64_t corners, T *__restrict__ dv, T *__restrict__ dx) {
+__global__ void k_det_finalize(const long long *__restrict__ acc, int64_t corners, T *__restrict__ dv, T *__restrict__ dx,
+                               int *__restrict__ cnt) {
     const int64_t c = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (c >= corners) return;
     const long long *a = acc + kDetWords * c;
+    cnt[c] = (int)((unsigned long long)a[3] >> 32);
 #pragma unroll
     for (int k = 0; k < 6; ++k) {
         long long l0 = a[4 * k], l1 = a[4 * k + 1], l2 = a[4 * k + 2];
@@ -1338,6 +1364,11 @@ constexpr int kImpProbe = 16;
 constexpr int log2_exact(int v) { return v <= 1 ? 0 : 1 + log2_exact(v / 2); }
 constexpr int kImpBits = log2_exact(kImpSlots);
 
+template <typename T> struct ImpulseOut {
+    T *dv, *dx;
+    int *cnt;
+};
+
 template <typename T> struct ImpTable {
     int *key;
     int *count;
@@ -1371,7 +1402,7 @@ template <typename T> struct ImpTable {
     }
     // adds one corner's impulse and position correction; to the global arrays directly
     // when the probe window is full
-    __device__ void add(int64_t c, const V3<T> &imp, const V3<T> &imd, T *dv, T *dx, int *cnt) {
+    __device__ void add(int64_t c, const V3<T> &imp, const V3<T> &imd, const ImpulseOut<T> &to) {
         const int s = slot((int)c);
         if (s >= 0) {
             atomicAdd(&acc[6 * s + 0], imp.x);
@@ -1382,26 +1413,26 @@ template <typename T> struct ImpTable {
             atomicAdd(&acc[6 * s + 5], imd.z);
             atomicAdd(&count[s], 1);
         } else {
-            atomicAdd(dv + 3 * c + 0, imp.x);
-            atomicAdd(dv + 3 * c + 1, imp.y);
-            atomicAdd(dv + 3 * c + 2, imp.z);
-            atomicAdd(dx + 3 * c + 0, imd.x);
-            atomicAdd(dx + 3 * c + 1, imd.y);
-            atomicAdd(dx + 3 * c + 2, imd.z);
-            atomicAdd(cnt + c, 1);
+            atomicAdd(to.dv + 3 * c + 0, imp.x);
+            atomicAdd(to.dv + 3 * c + 1, imp.y);
+            atomicAdd(to.dv + 3 * c + 2, imp.z);
+            atomicAdd(to.dx + 3 * c + 0, imd.x);
+            atomicAdd(to.dx + 3 * c + 1, imd.y);
+            atomicAdd(to.dx + 3 * c + 2, imd.z);
+            atomicAdd(to.cnt + c, 1);
         }
     }
-    __device__ void drain(int tid, T *dv, T *dx, int *cnt) {
+    __device__ void drain(int tid, const ImpulseOut<T> &to) {
         for (int s = tid; s < kImpSlots; s += kCcdThreads) {
             const int k = key[s];
             if (k < 0) continue;
-            atomicAdd(dv + 3 * (int64_t)k + 0, acc[6 * s + 0]);
-            atomicAdd(dv + 3 * (int64_t)k + 1, acc[6 * s + 1]);
-            atomicAdd(dv + 3 * (int64_t)k + 2, acc[6 * s + 2]);
-            atomicAdd(dx + 3 * (int64_t)k + 0, acc[6 * s + 3]);
-            atomicAdd(dx + 3 * (int64_t)k + 1, acc[6 * s + 4]);
-            atomicAdd(dx + 3 * (int64_t)k + 2, acc[6 * s + 5]);
-            atomicAdd(cnt + k, count[s]);
+            atomicAdd(to.dv + 3 * (int64_t)k + 0, acc[6 * s + 0]);
+            atomicAdd(to.dv + 3 * (int64_t)k + 1, acc[6 * s + 1]);
+            atomicAdd(to.dv + 3 * (int64_t)k + 2, acc[6 * s + 2]);
+            atomicAdd(to.dx + 3 * (int64_t)k + 0, acc[6 * s + 3]);
+            atomicAdd(to.dx + 3 * (int64_t)k + 1, acc[6 * s + 4]);
+            atomicAdd(to.dx + 3 * (int64_t)k + 2, acc[6 * s + 5]);
+            atomicAdd(to.cnt + k, count[s]);
         }
     }
 };
@@ -1442,13 +1473,13 @@ struct DetTable {
         }
         return -1;
     }
-    __device__ void add(int64_t c, const double v[6], long long *det, int *cnt) {
+    __device__ void add(int64_t c, const double v[6], long long *det) {
         const int s = slot((int)c);
         unsigned long long *g = reinterpret_cast<unsigned long long *>(det + kDetWords * c);
         if (s < 0) {
 #pragma unroll
             for (int k = 0; k < 6; ++k) det_add1(det + kDetWords * c + 4 * k, v[k]);
-            atomicAdd(cnt + c, 1);
+            atomicAdd(g + 3, kDetOne);
             return;
         }
 #pragma unroll
@@ -1465,18 +1496,16 @@ struct DetTable {
         }
         atomicAdd(&count[s], 1);
     }
-    __device__ void drain(int tid, long long *det, int *cnt) {
-        for (int s = tid; s < kImpSlots; s += kCcdThreads) {
-            const int k = key[s];
-            if (k < 0) continue;
+    // sixteen lanes per slot: the two low limbs of the six components, then the count
+    __device__ void drain(int tid, long long *det) {
+        const int word = tid & 15;
+#pragma unroll 2
+        for (int r = 0; r < kImpSlots * 16 / kCcdThreads; ++r) {
+            const int s = r * (kCcdThreads / 16) + tid / 16, k = key[s];
+            if (k < 0 || word > 12) continue;
+            const unsigned long long v = word < 12 ? acc[12 * s + word] : kDetOne * (unsigned long long)count[s];
             unsigned long long *g = reinterpret_cast<unsigned long long *>(det + kDetWords * (int64_t)k);
-#pragma unroll
-            for (int c = 0; c < 6; ++c) {
-                const unsigned long long lo = acc[12 * s + 2 * c], mid = acc[12 * s + 2 * c + 1];
-                if (lo) atomicAdd(g + 4 * c, lo);
-                if (mid) atomicAdd(g + 4 * c + 1, mid);
-            }
-            atomicAdd(cnt + k, count[s]);
+            if (v) atomicAdd(g + (word < 12 ? 4 * (word >> 1) + (word & 1) : 3), v);
         }
     }
 };
@@ -1524,14 +1553,37 @@ constexpr int kCollectFlush = 64;
 
 // Waves per SIMD asked of the compiler: the deterministic table's LDS (12.3 KB) allows only
 // 3.25 waves, and at four its registers spilled (37.28 against 37.06 ms per pass at three).
+// k_ccd's arguments, all of them, so that late_args finds them at the start of the kernel's
+// argument memory.
+template <typename T> struct CcdArgs {
+    const uint32_t *items;      // [B][cap_items]
+    const uint32_t *tiles;      // [B][cap_tiles]: first slot | items - 1
+    const int2 *pairs;          // [B][cap_pairs], this chunk's from first_pair on
+    const T *tv;                // vertex records
+    DevCounters *ctr;
+    DevPartial *parts;
+    int64_t cap_items, cap_tiles, cap_pairs, first_pair, n;
+    // impulse mode
+    const T *masses;
+    T *dv, *dx;
+    int *cnt;
+    long long *det;
+    // collect mode
+    int64_t *coll;
+    T *roots;
+    int64_t out_cap;
+};
+// The arguments read again where they are used: what only the scatter or the output needs
+// would otherwise sit in scalar registers, or in lanes of vector registers, through the solver
+// (each spilled scalar costs a vector instruction per use, and the kernel is bound by those).
+template <typename T> __device__ __forceinline__ const __attribute__((address_space(4))) CcdArgs<T> *late_args() {
+    auto *p = (const __attribute__((address_space(4))) CcdArgs<T> *)__builtin_amdgcn_kernarg_segment_ptr();
+    asm volatile("" : "+s"(p));
+    return p;
+}
+
 template <typename T, int MODE, bool DET>
-__global__ __launch_bounds__(kCcdThreads, MODE == MODE_IMPULSE ? (DET ? 3 : 4) : 5) void k_ccd(const uint32_t *__restrict__ items_all, int64_t capM,
-                                                  const int2 *__restrict__ pairs_all, int64_t capK, int64_t c0,
-                                                  const T *__restrict__ tv_all,
-                                                  const T *__restrict__ masses_all, int64_t n,
-                                                  int64_t *__restrict__ coll_all, T *__restrict__ roots_all, int64_t out_cap,
-                                                  T *__restrict__ dv_all, T *__restrict__ dx_all, int *__restrict__ cnt_all,
-                                                  long long *__restrict__ det_all, DevCounters *__restrict__ ctr_all) {
+__global__ __launch_bounds__(kCcdThreads, MODE == MODE_IMPULSE ? (DET ? 3 : 4) : 5) void k_ccd(CcdArgs<T> arg) {
     constexpr int NT = kCcdThreads;     // items per tile: the lanes of the one wavefront
     static_assert(NT == 64, "one wavefront per workgroup");
     constexpr int kRootCapT = 3 * NT;
@@ -1552,17 +1604,10 @@ __global__ __launch_bounds__(kCcdThreads, MODE == MODE_IMPULSE ? (DET ? 3 : 4) :
     __shared__ int64_t s_citem[NT];
     __shared__ T s_croot[NT];
     const int b = blockIdx.y, tid = threadIdx.x;
-    DevCounters *ctr = ctr_all + b;
-    const unsigned long long mc = ctr->items;
-    const int64_t M = (int64_t)(mc < (unsigned long long)capM ? mc : (unsigned long long)capM);
-    const uint32_t *items = items_all + (int64_t)b * capM;
-    const int2 *pairs = pairs_all + (int64_t)b * capK + c0;     // this chunk's candidate pairs
-    const T *tv = tv_all + (int64_t)b * n * 18;
-    const T *masses = MODE == MODE_IMPULSE ? masses_all + (int64_t)b * n * 3 : nullptr;
-    T *dv = MODE == MODE_IMPULSE ? dv_all + (int64_t)b * n * 9 : nullptr;
-    T *dx = MODE == MODE_IMPULSE ? dx_all + (int64_t)b * n * 9 : nullptr;
-    int *cnt = MODE == MODE_IMPULSE ? cnt_all + (int64_t)b * n * 3 : nullptr;
-    long long *det = DET ? det_all + (int64_t)b * n * 3 * kDetWords : nullptr;
+    const uint32_t *__restrict__ items = arg.items + (int64_t)b * arg.cap_items;
+    const uint32_t *__restrict__ tiles = arg.tiles + (int64_t)b * arg.cap_tiles;
+    const int2 *__restrict__ pairs = arg.pairs + (int64_t)b * arg.cap_pairs + arg.first_pair;     // this chunk's candidate pairs
+    const T *__restrict__ tv = arg.tv + (int64_t)b * arg.n * 18;
     // wave-uniform counts: roots found, collisions scattered, staged collisions, carried roots
     unsigned long long nroots = 0, ncoll = 0;
     int fill = 0, ncarry = 0;
@@ -1583,6 +1628,9 @@ __global__ __launch_bounds__(kCcdThreads, MODE == MODE_IMPULSE ? (DET ? 3 : 4) :
     auto flush = [&](int f) {
         for (int base = 0; base < f; base += kFlush) {
             const int nf = f - base < kFlush ? f - base : kFlush;
+            auto *late = late_args<T>();
+            const int64_t corner0 = (int64_t)blockIdx.y * late->n * 3;
+            const T *masses = late->masses + corner0;
             ImpulseParams<T> ip{};
             if (tid < nf) {
                 int64_t x, y;
@@ -1611,6 +1659,10 @@ __global__ __launch_bounds__(kCcdThreads, MODE == MODE_IMPULSE ? (DET ? 3 : 4) :
             const int j = tid & (kHalfFlush - 1), hi = tid >> 5;
             for (int h = 0; h * kHalfFlush < nf; ++h) {
                 const int nh = nf - h * kHalfFlush < kHalfFlush ? nf - h * kHalfFlush : kHalfFlush;
+                late = late_args<T>();
+                ImpulseOut<T> to{};
+                if (!DET) to = ImpulseOut<T>{late->dv + 3 * corner0, late->dx + 3 * corner0, late->cnt + corner0};
+                long long *det = DET ? late->det + corner0 * kDetWords : nullptr;
                 if (DET) dtab.clear(tid);
                 else tab.clear(tid);
                 wave_sync();
@@ -1639,15 +1691,15 @@ __global__ __launch_bounds__(kCcdThreads, MODE == MODE_IMPULSE ? (DET ? 3 : 4) :
                         corner_impulse(cp, type, k, dvk, imp, imd);
                         if (DET) {
                             const double v[6] = {(double)imp.x, (double)imp.y, (double)imp.z, (double)imd.x, (double)imd.y, (double)imd.z};
-                            dtab.add(c, v, det, cnt);
+                            dtab.add(c, v, det);
                         } else {
-                            tab.add(c, imp, imd, dv, dx, cnt);
+                            tab.add(c, imp, imd, to);
                         }
                     }
                 }
                 wave_sync();
-                if (DET) dtab.drain(tid, det, cnt);
-                else tab.drain(tid, dv, dx, cnt);
+                if (DET) dtab.drain(tid, det);
+                else tab.drain(tid, to);
                 wave_sync();
             }
         }
@@ -1657,9 +1709,12 @@ __global__ __launch_bounds__(kCcdThreads, MODE == MODE_IMPULSE ? (DET ? 3 : 4) :
     // counted, not written).
     auto write_rows = [&](int f) {
         unsigned long long ob = 0;
-        if (tid == 0 && f) ob = atomicAdd(&ctr->coll, (unsigned long long)f);
+        auto *late = late_args<T>();
+        const int64_t out_cap = late->out_cap;
+        if (tid == 0 && f) ob = atomicAdd(&late->ctr[blockIdx.y].coll, (unsigned long long)f);
         ob = readfirstlane_u64(ob);
-        int64_t *coll = coll_all + (int64_t)b * out_cap * 3;
+        int64_t *coll = late->coll + (int64_t)blockIdx.y * out_cap * 3;
+        T *roots = late->roots + (int64_t)blockIdx.y * out_cap;
         for (int j = tid; j < f; j += NT) {
             const unsigned long long slot = ob + (unsigned long long)j;
             if (slot < (unsigned long long)out_cap) {
@@ -1667,7 +1722,7 @@ __global__ __launch_bounds__(kCcdThreads, MODE == MODE_IMPULSE ? (DET ? 3 : 4) :
                 int type;
                 unpack_item(s_item[j], x, y, type);
                 coll[3 * slot] = x; coll[3 * slot + 1] = y; coll[3 * slot + 2] = type;
-                roots_all[(int64_t)b * out_cap + slot] = s_root[j];
+                roots[slot] = s_root[j];
             }
         }
         wave_sync();
@@ -1695,25 +1750,29 @@ __global__ __launch_bounds__(kCcdThreads, MODE == MODE_IMPULSE ? (DET ? 3 : 4) :
     // The tiles of CCC_FOR_TILES, walked by hand so that each lane's item of the next tile is
     // loaded one tile ahead (after this tile's gathers are issued) and its candidate pair
     // after phase B; kNoItem: no item.  An item is (pair index within the chunk) << 4 | type;
-    // the packed (x, y, type) form is made when the tile starts.  The moving items come in
-    // runs of one kind (edge-edge, then vertex-face, per k_subprim tile), so nearly every
-    // tile's roots and collisions take one branch of the filter and of the impulse in the
-    // whole wave.
-    constexpr uint32_t kNoItem = 0xffffffffu;   // type 15 does not exist
-    // tile counts in 32 bits (at most 15 * 2^28 / 64 tiles): the kernel's uniform values fill
-    // the scalar registers
-    const int ntiles = (int)((M + NT - 1) / NT);
+    // the packed (x, y, type) form is made when the tile starts.  A tile's items are of one
+    // kind (k_items), so its roots and collisions take one branch of the filter and of the
+    // impulse in the whole wave, but for the roots carried over a change.
+    // tile counts in 32 bits (at most 15 * 2^28 / 64 tiles and two per wave of k_items): the
+    // kernel's uniform values fill the scalar registers
+    const int ntiles = (int)arg.ctr[b].tiles;
     const int tper = (ntiles + kXcds - 1) / kXcds, tstep = (int)gridDim.x / kXcds;
     const int tbase = (int)(blockIdx.x % kXcds) * tper;
     // Each block takes one contiguous run of tiles: its collisions share corners, and the
     // blocks running beside it are far away in the list, so that their atomics fall on other
     // corners (tiles dealt out one by one: 129.6 instead of 104 ms per step of the 130k cloth,
     // 8.5 instead of 6.8 of the garment scene, in the order that k_pairs writes its pairs).
-    const int trun = (tper + tstep - 1) / tstep;
+    // With few tiles the runs are up to 8 tiles long, on fewer blocks, so that 8,192 blocks
+    // share them: a block's start and its last, partial rounds cost as much as several tiles
+    // (collect mode on 23k triangles, 93k tiles on 32,768 blocks: 375 us, on 8,192: 201).
+    const int tall = (tper + tstep - 1) / tstep, tfew = (ntiles + 8191) / 8192, tmin = tfew < 8 ? tfew : 8;
+    const int trun = tall > tmin ? tall : tmin;
     const int tfirst = (int)blockIdx.x / kXcds * trun, tlast = tfirst + trun < tper ? tfirst + trun : tper;
+    constexpr uint32_t kNoItem = 0xffffffffu;   // type 15 does not exist
     auto item_of = [&](int k) -> uint32_t {
-        const int64_t i = (int64_t)(tbase + k) * NT + tid;
-        return (k < tlast && tbase + k < ntiles && i < M) ? items[i] : kNoItem;
+        if (!(k < tlast && tbase + k < ntiles)) return kNoItem;
+        const uint32_t d = tiles[tbase + k];
+        return tid <= (int)(d & 63u) ? items[(d & ~63u) + (uint32_t)tid] : kNoItem;
     };
     // the next tile's item waits as its pair (registers) and its type (LDS, 15: no item), so
     // that it holds no more registers than the packed item through phases C and D
@@ -1818,8 +1877,9 @@ __global__ __launch_bounds__(kCcdThreads, MODE == MODE_IMPULSE ? (DET ? 3 : 4) :
         write_rows(fill);
     }
     if (tid == 0) {
-        if (nroots) atomicAdd(&ctr->roots, nroots);
-        if (MODE == MODE_IMPULSE && ncoll) atomicAdd(&ctr->coll, ncoll);
+        DevPartial *part = late_args<T>()->parts + (int64_t)b * kPartials + blockIdx.x % kPartials;
+        if (nroots) atomicAdd(&part->roots, nroots);
+        if (MODE == MODE_IMPULSE && ncoll) atomicAdd(&part->coll, ncoll);
     }
 }
 
@@ -2093,6 +2153,24 @@ __global__ void k_fold_items(DevCounters *__restrict__ ctr, int64_t B) {
     for (int64_t b = threadIdx.x; b < B; b += blockDim.x) {
         ctr[b].items_done += ctr[b].items;
         ctr[b].items = 0;
+        ctr[b].tiles = 0;
+    }
+}
+
+// End of the continuous narrow phase: the blocks' partial counts of every chunk to the
+// counters.  One wave per batch element.
+__global__ __launch_bounds__(64) void k_fold_partials(const DevPartial *__restrict__ part_all, bool coll, DevCounters *__restrict__ ctr) {
+    static_assert(kPartials == 64, "one lane per partial");
+    const DevPartial p = part_all[(int64_t)blockIdx.x * kPartials + threadIdx.x];
+    unsigned long long v[3] = {p.items, p.roots, p.coll};
+#pragma unroll
+    for (int d = 1; d < 64; d <<= 1)
+#pragma unroll
+        for (int k = 0; k < 3; ++k) v[k] += __shfl_xor(v[k], d, 64);
+    if (threadIdx.x == 0) {
+        ctr[blockIdx.x].items_done = v[0];
+        ctr[blockIdx.x].roots = v[1];
+        if (coll) ctr[blockIdx.x].coll = v[2];
     }
 }
 
@@ -2114,6 +2192,7 @@ static int64_t pair_chunk_of(const ccc_context *ctx, int64_t chunk_ext, int64_t 
     return std::max<int64_t>(std::min<int64_t>(std::min<int64_t>(pairs, budget / B), kMaxPairChunk), 1);
 }
 constexpr int kSubprimPairs = 2;   // pairs per thread of k_subprim
+constexpr int kItemWaves = 24;   // k_items: waves per CU (about two rounds of the resident ones)
 
 // Grid of the tile-looping kernels: one block per tile up to 128 blocks per CU, each block
 // then walking several tiles.  Measured on the 130k cloth (k_ccd per step): 4 blocks per CU
@@ -2209,6 +2288,28 @@ template <typename T> class GeneralTree {
     float *qbox_ = nullptr;
 };
 
+// The list of the continuous narrow phase for chunks of at most `chunk` pairs per batch
+// element: k_items' waves, the batches of 64 pairs that each takes at most, and the list
+// slots these can fill.
+struct ListPlan {
+    int64_t chunk, slots, tiles;
+    unsigned grid, run;
+    // the slots and the tiles' descriptors, each rounded as a workspace buffer is
+    size_t bytes(int64_t B) const {
+        auto r = [](size_t b) { return (b + 255) & ~(size_t)255; };
+        return r(sizeof(uint32_t) * B * slots) + r(sizeof(uint32_t) * B * tiles);
+    }
+};
+static ListPlan list_plan(const ccc_context *ctx, int64_t chunk, int64_t B) {
+    const int64_t batches = (chunk + kBatch - 1) / kBatch;
+    int64_t waves = std::max<int64_t>(std::min<int64_t>(batches, (int64_t)ctx->num_cus * kItemWaves / B), kXcds);
+    constexpr int kGroup = kXcds * kItemBlock;
+    waves = (waves + kGroup - 1) / kGroup * kGroup;
+    const int64_t per = (batches + kXcds - 1) / kXcds, run = (per + waves / kXcds - 1) / (waves / kXcds);
+    const int64_t slots = waves * run * (kSegEE + kSegVF) * kBatch;
+    return ListPlan{chunk, slots, slots / 64 + 2 * waves, (unsigned)(waves / kItemBlock), (unsigned)run};
+}
+
 template <typename T>
 static ccc_status run_query(const Query &q) {
     hipStream_t s = q.s;
@@ -2219,11 +2320,14 @@ static ccc_status run_query(const Query &q) {
     const bool moving = q.narrow == Narrow::CCD_COLLECT || q.narrow == Narrow::CCD_IMPULSE || q.narrow == Narrow::MINCOL;
     const int64_t nc = (n + kChunk - 1) >> kChunkBits;
     DevCounters *ctr = q.ctr_ext ? q.ctr_ext : ws.get_as<DevCounters>(B);
+    T *tv = moving ? ws.get_as<T>(B * n * 18) : nullptr;
+    const bool ccd_query = q.narrow == Narrow::CCD_COLLECT || q.narrow == Narrow::CCD_IMPULSE;
+    DevPartial *parts = ccd_query ? ws.get_as<DevPartial>(B * kPartials) : nullptr;
+    unsigned *foreign = q.nosync ? nullptr : ws.get_as<unsigned>(B * kForeignStep);
+    // from here on: what only the index tree's path uses, given back when the tree is another
     T *chunks = ws.get_as<T>(B * nc * 6);
     T *groups = ws.get_as<T>(B * nc * (kChunk / kPairQ) * 12);
     T *supers = nc > kSuperFrom ? ws.get_as<T>(B * ((nc + kChunk - 1) >> kChunkBits) * 6) : nullptr;
-    T *tv = moving ? ws.get_as<T>(B * n * 18) : nullptr;
-    unsigned *foreign = q.nosync ? nullptr : ws.get_as<unsigned>(B * kForeignStep);
     if (ws.failed()) return CCC_ERR_NO_MEMORY;
     ccc_status st;
 
@@ -2231,6 +2335,7 @@ static ccc_status run_query(const Query &q) {
     FillRegions fill;
     fill.add(ctr, B * (int64_t)sizeof(DevCounters), 0ull);
     if (foreign) fill.add(foreign, B * kForeignStep * 4, 0ull);
+    if (parts) fill.add(parts, B * kPartials * (int64_t)sizeof(DevPartial), 0ull);
     const uint64_t minus1 = sizeof(T) == 8 ? 0xBFF0000000000000ull : 0xBF800000BF800000ull;
     const int64_t cells = B * q.out_cap, tsz = (int64_t)sizeof(T);
     switch (q.narrow) {
@@ -2247,10 +2352,12 @@ static ccc_status run_query(const Query &q) {
             fill.add(q.out_roots, cells * tsz, minus1);
             break;
         case Narrow::CCD_IMPULSE:
-            fill.add(q.dv, B * n * 9 * tsz, 0ull);
-            fill.add(q.dx, B * n * 9 * tsz, 0ull);
-            fill.add(q.cnt, B * n * 12, 0ull);
             if (q.det_acc) fill.add(q.det_acc, B * n * 3 * kDetWords * 8, 0ull);
+            else {
+                fill.add(q.dv, B * n * 9 * tsz, 0ull);
+                fill.add(q.dx, B * n * 9 * tsz, 0ull);
+                fill.add(q.cnt, B * n * 12, 0ull);
+            }
             break;
     }
     if ((st = fill_regions(fill, s)) != CCC_OK) return st;
@@ -2321,7 +2428,11 @@ static ccc_status run_query(const Query &q) {
             CCC_HIP_TRY(hipMemcpyAsync(ctr, h.data(), sizeof(DevCounters) * B, hipMemcpyHostToDevice, s));
             if (flags & DEV_STACK) general.go_deep();
             else {
-                if (!q.pairs_ext) { ws.release(pairs); pairs = nullptr; }   // the list follows the tree's buffers
+                // the list follows the tree's buffers (last in, first out)
+                if (!q.pairs_ext) { ws.release(pairs); pairs = nullptr; }
+                if (supers) ws.release(supers);
+                ws.release(groups);
+                ws.release(chunks);
                 if ((st = general.prepare()) != CCC_OK) return st;
             }
             --attempt;
@@ -2370,17 +2481,27 @@ static ccc_status run_query(const Query &q) {
         // sub-primitive items and the narrow phase run over chunks of the pair list; the
         // chunk bounds the pairs of all batch elements together (the item buffer holds B
         // chunks), so the workspace does not grow with the batch
+        const bool ccd = q.narrow != Narrow::PROXIMITY;
         int64_t chunk = pair_chunk_of(q.ctx, q.chunk_ext, kmax, B, item_bytes(q.narrow));
+        ListPlan plan = list_plan(q.ctx, chunk, B);
         if (ws.arena()) {
             // the item list takes what the arena has left (results do not depend on the chunk)
-            const int64_t fit = (int64_t)(ws.arena_left() / ((size_t)B * 15 * item_bytes(q.narrow)));
-            if (fit < 1) {
+            if (ccd) {
+                while (plan.bytes(B) > ws.arena_left() && chunk > 1) {
+                    chunk = std::min(chunk / 2, std::max<int64_t>((int64_t)(ws.arena_left() / ((size_t)B * 15 * sizeof(uint32_t))), 1));
+                    plan = list_plan(q.ctx, chunk, B);
+                }
+                if (plan.bytes(B) > ws.arena_left()) chunk = 0;
+            } else {
+                chunk = std::min(chunk, (int64_t)(ws.arena_left() / ((size_t)B * 15 * item_bytes(q.narrow))));
+            }
+            if (chunk < 1) {
                 set_error("the scratch buffer has no room left for the sub-primitive items of one candidate pair");
                 return CCC_ERR_NO_MEMORY;
             }
-            chunk = std::min(chunk, fit);
         }
-        const int64_t capM = 15 * chunk;
+        const int64_t capM = ccd ? plan.slots : 15 * chunk;
+        uint32_t *tiles = ccd ? ws.get_as<uint32_t>(B * plan.tiles) : nullptr;
         void *items = ws.get_as<unsigned char>(B * capM * (int64_t)item_bytes(q.narrow));
         const unsigned gS = persistent_grid(q.ctx, (chunk + kSubprimPairs - 1) / kSubprimPairs, B);
         const unsigned gM = persistent_grid(q.ctx, capM, B);
@@ -2399,37 +2520,59 @@ static ccc_status run_query(const Query &q) {
                     hipLaunchKernelGGL((k_subprim<T, SUB_STATIC, kSubprimPairs>), dim3(gS, B), dim3(kThreads), 0, s, pairs, capK,
                                        c0, c1, (const T *)q.t0, n, thr, items, capM, ctr);
                 else
-                    hipLaunchKernelGGL((k_subprim<T, SUB_MOVING, kSubprimPairs>), dim3(gS, B), dim3(kThreads), 0, s, pairs, capK,
-                                       c0, c1, (const T *)tv, n, thr, items, capM, ctr);
+                    hipLaunchKernelGGL((k_items<T>), dim3(plan.grid, B), dim3(64 * kItemBlock), 0, s, pairs, capK, c0, c1, (const T *)tv, n,
+                                       (uint32_t *)items, capM, plan.run, tiles, plan.tiles, parts, ctr);
                 tm.end();
                 CCC_LAUNCH_CHECK("k_subprim");
                 tm.begin(q.narrow == Narrow::PROXIMITY ? "proximity" : q.narrow == Narrow::CCD_COLLECT ? "ccd_collect" : "ccd_impulse");
                 if (q.narrow == Narrow::PROXIMITY)
                     hipLaunchKernelGGL((k_proximity<T>), dim3(gM, B), dim3(kThreads), 0, s, (const int64_t *)items, capM, (const T *)q.t0, n, thr,
                                        q.out_rows, q.out_cap, ctr);
-                else if (q.narrow == Narrow::CCD_COLLECT)
-                    hipLaunchKernelGGL((k_ccd<T, MODE_COLLECT, false>), dim3(gCcdC, B), dim3(ccd_threads<MODE_COLLECT>()), 0, s, (const uint32_t *)items, capM, (const int2 *)pairs, capK, c0,
-                                       (const T *)tv, (const T *)nullptr, n, q.out_rows, (T *)q.out_roots, q.out_cap,
-                                       (T *)nullptr, (T *)nullptr, (int *)nullptr, (long long *)nullptr, ctr);
-                else if (q.det_acc)
-                    hipLaunchKernelGGL((k_ccd<T, MODE_IMPULSE, true>), dim3(gCcdI, B), dim3(ccd_threads<MODE_IMPULSE>()), 0, s, (const uint32_t *)items, capM, (const int2 *)pairs, capK, c0,
-                                       (const T *)tv, (const T *)q.masses, n, (int64_t *)nullptr, (T *)nullptr, (int64_t)0,
-                                       (T *)q.dv, (T *)q.dx, q.cnt, q.det_acc, ctr);
-                else
-                    hipLaunchKernelGGL((k_ccd<T, MODE_IMPULSE, false>), dim3(gCcdI, B), dim3(ccd_threads<MODE_IMPULSE>()), 0, s, (const uint32_t *)items, capM, (const int2 *)pairs, capK, c0,
-                                       (const T *)tv, (const T *)q.masses, n, (int64_t *)nullptr, (T *)nullptr, (int64_t)0,
-                                       (T *)q.dv, (T *)q.dx, q.cnt, (long long *)nullptr, ctr);
+                else {
+                    CcdArgs<T> ca{};
+                    ca.items = (const uint32_t *)items;
+                    ca.tiles = tiles;
+                    ca.pairs = pairs;
+                    ca.tv = tv;
+                    ca.ctr = ctr;
+                    ca.parts = parts;
+                    ca.cap_items = capM;
+                    ca.cap_tiles = plan.tiles;
+                    ca.cap_pairs = capK;
+                    ca.first_pair = c0;
+                    ca.n = n;
+                    ca.masses = (const T *)q.masses;
+                    ca.dv = (T *)q.dv;
+                    ca.dx = (T *)q.dx;
+                    ca.cnt = q.cnt;
+                    ca.det = q.det_acc;
+                    ca.coll = q.out_rows;
+                    ca.roots = (T *)q.out_roots;
+                    ca.out_cap = q.out_cap;
+                    if (q.narrow == Narrow::CCD_COLLECT)
+                        hipLaunchKernelGGL((k_ccd<T, MODE_COLLECT, false>), dim3(gCcdC, B), dim3(ccd_threads<MODE_COLLECT>()), 0, s, ca);
+                    else if (q.det_acc)
+                        hipLaunchKernelGGL((k_ccd<T, MODE_IMPULSE, true>), dim3(gCcdI, B), dim3(ccd_threads<MODE_IMPULSE>()), 0, s, ca);
+                    else
+                        hipLaunchKernelGGL((k_ccd<T, MODE_IMPULSE, false>), dim3(gCcdI, B), dim3(ccd_threads<MODE_IMPULSE>()), 0, s, ca);
+                }
                 tm.end();
                 CCC_LAUNCH_CHECK("narrow phase");
-                hipLaunchKernelGGL(k_fold_items, dim3(1), dim3(64), 0, s, ctr, B);
-                CCC_LAUNCH_CHECK("k_fold_items");
+                if (!ccd || c0 + chunk < kmax) {
+                    hipLaunchKernelGGL(k_fold_items, dim3(1), dim3(64), 0, s, ctr, B);
+                    CCC_LAUNCH_CHECK("k_fold_items");
+                }
+            }
+            if (ccd) {
+                hipLaunchKernelGGL(k_fold_partials, dim3(B), dim3(64), 0, s, parts, q.narrow == Narrow::CCD_IMPULSE, ctr);
+                CCC_LAUNCH_CHECK("k_fold_partials");
             }
             return CCC_OK;
         };
         if ((st = narrow_phase()) != CCC_OK) return st;
         if (q.det_acc) {
             hipLaunchKernelGGL((k_det_finalize<T>), dim3(grid_for(B * n * 3, 256)), dim3(256), 0, s, q.det_acc, B * n * 3,
-                               (T *)q.dv, (T *)q.dx);
+                               (T *)q.dv, (T *)q.dx, q.cnt);
             CCC_LAUNCH_CHECK("k_det_finalize");
         }
     }
@@ -2468,7 +2611,8 @@ static size_t resident_bytes(const Query &q) {
     const int64_t capK = q.cap_candidates > 0 ? q.cap_candidates : 1;
     if (!q.pairs_ext) tot += r(sizeof(int2) * B * capK);
     const int64_t chunk = pair_chunk_of(q.ctx, q.chunk_ext, capK, B, item_bytes(q.narrow));
-    tot += r(esz * B * n * 18) + r(item_bytes(q.narrow) * B * 15 * chunk);
+    const ListPlan plan = list_plan(q.ctx, chunk, B);
+    tot += r(esz * B * n * 18) + r(sizeof(DevPartial) * B * kPartials) + plan.bytes(B);
     return tot;
 }
 

@@ -6,7 +6,7 @@ import pytest
 
 from tests import cases
 from tests.conftest import sorted_rows, valid_rows
-from tests.test_gpu_parity import _np, _renumbered_internal_tree, _t
+from tests.test_gpu_parity import _check_close, _compare_collisions, _np, _renumbered_internal_tree, _t
 
 pytestmark = pytest.mark.gpu
 
@@ -75,3 +75,28 @@ def test_special_boxes(ccc, oracle):
     for bb, tree in ((rb, rt), _renumbered_internal_tree(rb, rt, 2)):
         _, k = _mincol(ccc, bb, tree, t0, t1, 200)
         assert k == total
+
+
+@pytest.mark.parametrize("chunk", [0, 1, 64, 65, 1000])
+@pytest.mark.parametrize("n", [2, 9, 70, 300])
+def test_items_at_batch_edges(ccc, oracle, n, chunk):
+    """The narrow phase's items in waves of 64 pairs and chunks of them: collisions, counts and
+    the two ways to impulses against the oracle."""
+    t0, t1, m = cases.random_soup(n, seed=n + 5, motion=0.2)
+    rb, rt, _, _ = oracle.bvh(t0, t1)
+    dv, dx, cnt, coll, roots, counts = oracle.compute_impulses(rb, rt, t0, t1, m)
+    args = (_t(rb[None]), _t(rt[None]), _t(t0[None]), _t(t1[None]))
+    want = [counts[k] for k in ("candidates", "subprims", "roots", "collisions")]
+    ccc.set_pair_chunk(chunk)
+    try:
+        gc, gr = ccc.find_collisions_continuous(*args, n, 4 * n)
+        assert ccc.last_counts()[0] == want
+        _compare_collisions(_np(gc)[0], _np(gr)[0], coll, roots)
+        direct = ccc.compute_impulses(*args, _t(m[None]), n, 16)
+        assert ccc.last_counts()[0] == want
+    finally:
+        ccc.set_pair_chunk(0)
+    for out in (direct, ccc.compute_impulses_from_collisions(gc, gr, args[2], args[3], _t(m[None]))):
+        np.testing.assert_array_equal(_np(out[2])[0], cnt)
+        _check_close(_np(out[0])[0], dv, "dv")
+        _check_close(_np(out[1])[0], dx, "dx")

@@ -1910,24 +1910,76 @@ __global__ void k_device_math(int what, const double *__restrict__ x, double *__
 }
 
 // compute_impulses_from_collisions (collisions_impulses.cu:1736-1880) over given rows;
-// rows with a negative or out-of-range index are skipped.
-template <typename T>
-__global__ __launch_bounds__(kThreads) void k_from_collisions(const int64_t *__restrict__ coll_all, const T *__restrict__ roots_all,
-                                                              int64_t m, const T *__restrict__ t0_all, const T *__restrict__ t1_all,
-                                                              const T *__restrict__ masses_all, int64_t n, T *__restrict__ dv_all,
-                                                              T *__restrict__ dx_all, int *__restrict__ cnt_all) {
-    const int b = blockIdx.y;
-    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= m) return;
-    const int64_t *row = coll_all + ((int64_t)b * m + i) * 3;
-    const int64_t x = row[0], y = row[1], type = row[2];
-    if (x < 0 || y < 0 || type < 0 || type > 14 || x >= n || y >= n) return;
-    const T root = roots_all[(int64_t)b * m + i];
-    const T *t0 = t0_all + (int64_t)b * n * 9;
-    const T *t1 = t1_all + (int64_t)b * n * 9;
-    const MTet<T> mt = gather_mtet(t0, t1, x, y, (int)type);
-    scatter_impulse(mt, (int)type, root, x, y, masses_all + (int64_t)b * n * 3, dv_all + (int64_t)b * n * 9,
-                    dx_all + (int64_t)b * n * 9, cnt_all + (int64_t)b * n * 3);
+// rows with a negative or out-of-range index are skipped.  Bound by its atomics: added one by
+// one they are 28 per row (450 us for 357k collisions of a 23k-triangle cloth, 22e9 atomics
+// per second).  So the corner sums of 32 rows at a time go through the same LDS table as
+// k_ccd's first, the collision lists being written in runs of neighbouring pairs: 105 us.
+// 64 rows in 128 slots take 143 us, 16 rows in 64 slots 120, tables kept over 128 rows 170 to
+// 190: more shares find their slots taken and probe on, or more slots are drained for the same
+// sums.  One wave per block, kRowRun rows in a row, every gridDim.x-th run, so that all waves
+// share the padding at a list's end (runs of 64, 128, 256: 105, 106, 110 us).  Meshes whose
+// corner numbers do not fit the table's 32-bit keys take the atomics one by one.
+constexpr int kRowRun = 128;
+template <typename T, bool TABLE>
+__global__ __launch_bounds__(kCcdThreads) void k_from_collisions(const int64_t *__restrict__ coll_all, const T *__restrict__ roots_all,
+                                                                 int64_t m, const T *__restrict__ t0_all, const T *__restrict__ t1_all,
+                                                                 const T *__restrict__ masses_all, int64_t n, T *__restrict__ dv_all,
+                                                                 T *__restrict__ dx_all, int *__restrict__ cnt_all) {
+    __shared__ __align__(16) unsigned char s_raw[TABLE ? ImpTable<T>::bytes() : 16];
+    const int b = blockIdx.y, lane = threadIdx.x;
+    const int64_t *coll = coll_all + (int64_t)b * m * 3;
+    const T *roots = roots_all + (int64_t)b * m;
+    const T *t0 = t0_all + (int64_t)b * n * 9, *t1 = t1_all + (int64_t)b * n * 9, *masses = masses_all + (int64_t)b * n * 3;
+    const ImpulseOut<T> to{dv_all + (int64_t)b * n * 9, dx_all + (int64_t)b * n * 9, cnt_all + (int64_t)b * n * 3};
+    ImpTable<T> tab = ImpTable<T>::over(s_raw);
+    for (int64_t run = (int64_t)blockIdx.x * kRowRun; run < m; run += (int64_t)gridDim.x * kRowRun) {
+        for (int64_t i = run + lane; i - lane < m && i - lane < run + kRowRun; i += kCcdThreads) {
+            int64_t x = -1, y = -1, type = -1;
+            if (i < m) { x = coll[3 * i]; y = coll[3 * i + 1]; type = coll[3 * i + 2]; }
+            const bool on = !(x < 0 || y < 0 || type < 0 || type > 14 || x >= n || y >= n);
+            if (!__any(on)) continue;
+            MTet<T> mt{};
+            T root = (T)0;
+            if (on) {
+                root = roots[i];
+                mt = gather_mtet(t0, t1, x, y, (int)type);
+            }
+            if (!TABLE) {
+                if (on) scatter_impulse(mt, (int)type, root, x, y, masses, to.dv, to.dx, to.cnt);
+                continue;
+            }
+            ImpulseParams<T> ip{};
+            if (on) {
+                T q[4];
+#pragma unroll
+                for (int k = 0; k < 4; ++k) {
+                    int side, idx;
+                    type_corner((int)type, k, side, idx);
+                    q[k] = masses[3 * (side ? y : x) + idx];
+                }
+                ip = collision_impulse(mt, (int)type, root, q);
+            }
+            for (int h = 0; h < 2; ++h) {
+                const bool mine = on && (lane >> 5) == h;
+                if (!__any(mine)) continue;
+                tab.clear(lane);
+                wave_sync();
+                if (mine) {
+#pragma unroll
+                    for (int k = 0; k < 4; ++k) {
+                        int side, idx;
+                        type_corner((int)type, k, side, idx);
+                        V3<T> imp, imd;
+                        corner_impulse(ip, (int)type, k, mt.dv[k], imp, imd);
+                        tab.add(3 * (side ? y : x) + idx, imp, imd, to);
+                    }
+                }
+                wave_sync();
+                tab.drain(lane, to);
+                wave_sync();
+            }
+        }
+    }
 }
 
 // Static proximity per item (proximity_static.cu:435-508): distance by type, kept when
@@ -2690,8 +2742,13 @@ static ccc_status from_collisions(ccc_context *ctx, const int64_t *coll, const v
     KernelTimer tm(ctx, s);
     if (m > 0) {
         tm.begin("from_collisions");
-        hipLaunchKernelGGL((k_from_collisions<T>), dim3(grid_for(m, kThreads), B), dim3(kThreads), 0, s, coll, (const T *)roots, m,
-                           (const T *)t0, (const T *)t1, (const T *)masses, n, (T *)dv, (T *)dx, cnt);
+        const unsigned g = (unsigned)std::min<int64_t>((m + kRowRun - 1) / kRowRun, 16384);
+        if (n < ((int64_t)1 << 28))
+            hipLaunchKernelGGL((k_from_collisions<T, true>), dim3(g, B), dim3(kCcdThreads), 0, s, coll, (const T *)roots, m,
+                               (const T *)t0, (const T *)t1, (const T *)masses, n, (T *)dv, (T *)dx, cnt);
+        else
+            hipLaunchKernelGGL((k_from_collisions<T, false>), dim3(g, B), dim3(kCcdThreads), 0, s, coll, (const T *)roots, m,
+                               (const T *)t0, (const T *)t1, (const T *)masses, n, (T *)dv, (T *)dx, cnt);
         tm.end();
         CCC_LAUNCH_CHECK("k_from_collisions");
     }

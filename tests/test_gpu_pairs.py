@@ -100,3 +100,32 @@ def test_items_at_batch_edges(ccc, oracle, n, chunk):
         np.testing.assert_array_equal(_np(out[2])[0], cnt)
         _check_close(_np(out[0])[0], dv, "dv")
         _check_close(_np(out[1])[0], dx, "dx")
+
+
+@pytest.mark.parametrize("dtype", [np.float64, np.float32])
+@pytest.mark.parametrize("m", [1, 31, 33, 64, 127, 129, 300])
+def test_impulses_of_given_rows(ccc, oracle, m, dtype):
+    """compute_impulses_from_collisions at the edges of its runs: two meshes' rows with padding
+    and out-of-range rows among them, shuffled, each row more than once, so that one corner
+    takes many shares.  Float sums of at most 4 m terms: within 8 m ulp of the largest."""
+    c = -np.ones((2, m, 3), np.int64)
+    r = np.zeros((2, m, 1), dtype)
+    t, want = [], []
+    for b in range(2):
+        t0, t1, mass = cases.random_soup(40, seed=3 * m + b, motion=0.2, dtype=dtype)
+        rb, rt, _, _ = oracle.bvh(t0, t1)
+        coll, roots, _ = oracle.find_collisions_continuous(rb, rt, t0, t1)
+        rng = np.random.default_rng(m + b)
+        pick = rng.integers(0, len(coll), m)
+        c[b], r[b, :, 0] = coll[pick], roots[pick]
+        keep = rng.random(m) < 0.8
+        c[b][~keep] = rng.permutation(np.array([[-1, -1, -1], [40, 0, 0], [0, 40, 3], [0, 1, 15], [1, -5, 2]]))[rng.integers(0, 5, (~keep).sum())]
+        t.append((t0, t1, mass))
+        want.append(oracle.impulses(t0, t1, mass, c[b][keep], r[b, keep, 0]))
+    t0, t1, mass = (np.stack(x) for x in zip(*t))
+    dv, dx, cnt = (_np(x) for x in ccc.compute_impulses_from_collisions(_t(c), _t(r), _t(t0), _t(t1), _t(mass)))
+    for b in range(2):
+        np.testing.assert_array_equal(cnt[b], want[b][2])
+        for got, ref in ((dv[b], want[b][0]), (dx[b], want[b][1])):
+            tol = 8 * m * np.finfo(dtype).eps * max(np.abs(ref).max(), np.finfo(dtype).tiny)
+            assert np.abs(got - ref).max() <= tol + 1e-12 * np.abs(ref).max()

@@ -245,36 +245,37 @@ template <typename T> __device__ __forceinline__ uint32_t moving_mask_axes(const
     return eq ? 0u : m;
 }
 
-// gather_mtet from vertex records (same values, so the same tetrahedron bit for bit).  The
-// record of each tetrahedron corner is picked as type_corner does, with the edge-edge and
-// the vertex-face types on separate paths: the narrow phase's waves hold one kind, so a wave
-// runs one of the two short address computations.
-template <typename T>
-__device__ __forceinline__ MTet<T> gather_mtet_rec(const T *tv, int64_t x, int64_t y, int type) {
-    // record indices (corner 3 * triangle + i, below 3 * 2^28 as meshes hold fewer than 2^28
-    // triangles); integers rather than pointers, so that the loads keep the records' global
-    // address space
-    const uint32_t rx = 3u * (uint32_t)x, ry = 3u * (uint32_t)y;
-    uint32_t c[4];
-    if (type < 9) {
-        // edge type / 3 of x, edge type % 3 of y
-        const int ea = type / 3, eb = type - 3 * ea;
-        c[0] = rx + edge_first(ea);
-        c[1] = rx + edge_second(ea);
-        c[2] = ry + edge_first(eb);
-        c[3] = ry + edge_second(eb);
-    } else {
-        // 9-11: face x, vertex type - 9 of y; 12-14: vertex type - 12 of x, face y
-        const bool inv = type >= 12;
-        const uint32_t j = (uint32_t)(inv ? type - 12 : type - 9);
-        c[0] = inv ? rx + j : rx;
-        c[1] = inv ? ry : rx + 1;
-        c[2] = inv ? ry + 1 : rx + 2;
-        c[3] = inv ? ry + 2 : ry + j;
+// The four corners of a type as type_corner gives them, one byte each: three times the corner's
+// index within its triangle (a record is three 16-byte or 8-byte units).
+__device__ __forceinline__ uint32_t corner_bytes(int type) {
+    uint32_t w = 0;
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+        int side, idx;
+        type_corner(type, k, side, idx);
+        w |= (uint32_t)(3 * idx) << (8 * k);
     }
+    return w;
+}
+
+// gather_mtet from vertex records (same values, so the same tetrahedron bit for bit), with
+// w = corner_bytes(type) from a table.  Corner 0 is always of x and corner 3 of y, corner 1 of
+// y for types 12-14 and corner 2 of x for types 9-11.  Addresses are counted in units of a
+// third of a record (9 per triangle, below 2^32 as meshes hold fewer than 2^28 triangles): a
+// shift-add per triangle, an add of a byte per corner and one 64-bit shift-add, no multiplies
+// (v_mad_u64_u32 is quarter rate).
+template <typename T>
+__device__ __forceinline__ MTet<T> gather_mtet_rec(const T *tv, int64_t x, int64_t y, int type, uint32_t w) {
+    const uint32_t ux = 9u * (uint32_t)x, uy = 9u * (uint32_t)y;
+    const uint32_t u[4] = {ux + (w & 255u), (type >= 12 ? uy : ux) + ((w >> 8) & 255u),
+                           ((unsigned)(type - 9) < 3u ? ux : uy) + ((w >> 16) & 255u), uy + (w >> 24)};
     MTet<T> m;
 #pragma unroll
-    for (int k = 0; k < 4; ++k) ld_vrec(tv, c[k], m.v[k], m.dv[k]);
+    for (int k = 0; k < 4; ++k) {
+        const VRec<T> r = *reinterpret_cast<const VRec<T> *>(tv + 2 * (uint64_t)u[k]);
+        m.v[k] = mk(r.a[0], r.a[1], r.a[2]);
+        m.dv[k] = mk(r.a[3], r.a[4], r.a[5]);
+    }
     return m;
 }
 
@@ -358,25 +359,74 @@ __device__ __forceinline__ double dd_cube_lead(double b) {
 // cubic_candidates and cubic_roots produce the roots.
 enum : int { CUBIC_NONE = 0, CUBIC_QUADRATIC = 1, CUBIC_TRIPLE = 2, CUBIC_TRIG = 3, CUBIC_CARDANO = 4 };
 
-struct CubicState { double a, b, c, d, f, g, h; };
+// What the branch needs, in the same three register pairs for all (a wave holding several
+// branches keeps one set): QUADRATIC b, c, d; TRIPLE d / a; TRIG and CARDANO b / (3 a), g, h.
+struct CubicState { double p, q, r; bool tame; };
+
+// The solver's divisions of a tame cubic share their reciprocals.  A division costs eleven
+// operations and a quarter-rate reciprocal: scaling of both operands, the reciprocal, two
+// Newton steps on it, then quotient, remainder and correction.  Without over- or underflow
+// the scaling changes nothing, and the refined reciprocals of a^2, a^3 and 3 a follow from
+// a's by one Newton step each, so that the six quotients by powers of a take 35 issue slots
+// instead of 84 (and the quotient under the arc cosine takes its reciprocal from the square
+// root).  One Newton step from a start within a few ulp leaves y within half an ulp (1 +
+// 2^-48) of the reciprocal, as the division's own steps do, and quotient_by's remainder step
+// then gives the rounded quotient (Markstein, IBM J. Res. Dev. 34(1), 1990): the division's
+// bits, but for the sign of a zero quotient.  With the gathers' addresses (gather_mtet_rec):
+// k_ccd per step of the 130k cloth 107.0 -> 103.4 ms, of the garment scene 4.58 -> 4.27.
+__device__ __forceinline__ double recip_step(double d, double y) { return fma(y, fma(-d, y, 1.0), y); }
+__device__ __forceinline__ double quotient_by(double n, double d, double y) {
+    const double q = n * y;
+    return fma(fma(-d, q, n), y, q);
+}
+
+// Tame: 1e-16 <= |a| <= 2^20, 2^-60 <= |b| <= 2^40, |c|, |d| <= 2^40 and d zero or at least
+// 2^-100.  Then every quotient, remainder and power below is far inside the normal range,
+// except that 3 c and b c may be zero or tiny, and those two quotients are then rounded away
+// against b^2 / a^2 >= 2^-160 and 2 b^3 / a^3 >= 2^-239.  f is 0 or at least 2^-216, g 0 or at
+// least 2^-298, so the square root's argument is at least 2^-706 (sqrt_no_rescale's range) and
+// nothing is infinite or NaN.  A zero's sign cannot matter: 3 c / a, p2 and p3 are summed with
+// other terms, the sign of a zero f or g changes no later value, and b is not zero.
+__device__ __forceinline__ bool cubic_tame(double a, double b, double c, double d) {
+    return fabs(a) <= 0x1p20 && fabs(b) >= 0x1p-60 && fabs(b) <= 0x1p40 && fabs(c) <= 0x1p40 &&
+           fabs(d) <= 0x1p40 && (d == 0 || fabs(d) >= 0x1p-100);
+}
 
 __device__ __forceinline__ int cubic_prepare(double a, double b, double c, double d, CubicState &st) {
-    st.a = a; st.b = b; st.c = c; st.d = d; st.f = 0; st.g = 0; st.h = 0;
+    st.p = b; st.q = c; st.r = d; st.tame = false;
     if (a == 0 && b == 0) return CUBIC_NONE;   // :532-536 linear root computed, never stored
     if (fabs(a) < 1e-16) return CUBIC_QUADRATIC;
-    // the divisions by 3 and 27 give the division's bits (div_exact)
-    const double f = div_exact<3>((3.0 * c / a) - ((b * b) / (a * a)));
+    st.tame = cubic_tame(a, b, c, d);
     const double b3 = 2 * dd_cube_lead(b);
     const double a2 = a * a;
     const double a3 = dd_cube_lead(a);
-    const double p1 = b3 / a3;
-    const double p2 = (b * c * 9) / a2;
-    const double p3 = 27.0 * d / a;
-    const double g = div_exact<27>(p1 - p2 + p3);
-    const double f3 = dd_cube_lead(f);
-    const double h = (g * g) / 4.0 + div_exact<27>(f3);
-    st.f = f; st.g = g; st.h = h;
-    if (f == 0 && g == 0 && h == 0) return CUBIC_TRIPLE;
+    const double d3 = 3.0 * a;
+    double f, g, h;
+    // the divisions by 3 and 27 give the division's bits (div_exact)
+    if (st.tame) {
+        const double y1 = recip_step(a, recip_step(a, __builtin_amdgcn_rcp(a)));
+        const double y2 = recip_step(a2, y1 * y1);
+        f = div_exact_finite<3>(quotient_by(3.0 * c, a, y1) - quotient_by(b * b, a2, y2));
+        const double p1 = quotient_by(b3, a3, recip_step(a3, y2 * y1));
+        const double p2 = quotient_by(b * c * 9, a2, y2);
+        const double p3 = quotient_by(27.0 * d, a, y1);
+        st.p = quotient_by(b, d3, recip_step(d3, y1 * CCC_THIRD));
+        g = div_exact_finite<27>(p1 - p2 + p3);
+        h = (g * g) / 4.0 + div_exact_finite<27>(dd_cube_lead(f));
+    } else {
+        f = div_exact<3>((3.0 * c / a) - ((b * b) / a2));
+        const double p1 = b3 / a3;
+        const double p2 = (b * c * 9) / a2;
+        const double p3 = 27.0 * d / a;
+        st.p = b / d3;
+        g = div_exact<27>(p1 - p2 + p3);
+        h = (g * g) / 4.0 + div_exact<27>(dd_cube_lead(f));
+    }
+    st.q = g; st.r = h;
+    if (f == 0 && g == 0 && h == 0) {
+        st.p = d / a;
+        return CUBIC_TRIPLE;
+    }
     return h <= 0 ? CUBIC_TRIG : CUBIC_CARDANO;
 }
 
@@ -387,9 +437,9 @@ __device__ __forceinline__ int cubic_prepare(double a, double b, double c, doubl
 // R >= 0 and -cbrt(-R) otherwise are +-cbrt(|R|)), so a wave holding both forms evaluates
 // them once.
 __device__ __forceinline__ int cubic_candidates(int code, const CubicState &st, double &x0, double &x1, double &x2) {
-    const double a = st.a, b = st.b, c = st.c, d = st.d, g = st.g, h = st.h;
     if (code == CUBIC_QUADRATIC) {
         // :537-547
+        const double b = st.p, c = st.q, d = st.r;
         double D = c * c - 4.0 * b * d;
         if (D >= 0) {
             D = sqrt(D);
@@ -400,19 +450,25 @@ __device__ __forceinline__ int cubic_candidates(int code, const CubicState &st, 
     } else if (code == CUBIC_TRIPLE) {
         // :564-575 triple root through a float k
         // k >= 0 ? -cbrtf(k) : cbrtf(-k), with one cube root
-        float k = (float)(d / a);
+        float k = (float)st.p;
         const float ck = pm_cbrtf(k >= 0 ? k : -k);
         x0 = k >= 0 ? (double)(ck * -1) : (double)ck;
         return 1;
     } else if (code == CUBIC_TRIG || code == CUBIC_CARDANO) {
         const bool trig = code == CUBIC_TRIG;
-        const double sq = sqrt(trig ? ((g * g) / 4.0) - h : h);
+        const double b3a = st.p, g = st.q, h = st.r;
+        const double sa = trig ? ((g * g) / 4.0) - h : h;
+        double sq, y = 0;      // y: about 1 / (2 sq)
+        if (st.tame) sq = sqrt_no_rescale(sa, y);
+        else sq = sqrt(sa);
         const double R = -(g / 2.0) + sq;
         const double cb = pm_cbrt(trig ? sq : fabs(R));
-        const double b3a = b / (3.0 * a);
         if (trig) {
             // :576-591 three real roots: i = sq, j = cb
-            const double k = pm_acos(-(g / (2 * sq)));
+            double r;
+            if (st.tame) r = quotient_by(g, 2 * sq, recip_step(2 * sq, y));
+            else r = g / (2 * sq);
+            const double k = pm_acos(-r);
             const double L = cb * -1;
             // cos(k / 3) appears twice in the formulas; evaluated once (the same value)
             const double k3 = div_exact_finite<3>(k);      // k in [0, pi] or NaN

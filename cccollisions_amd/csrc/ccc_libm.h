@@ -110,7 +110,8 @@ template <int D> __device__ __forceinline__ double div_exact(double x) {
 // emits for sqrt (reciprocal square root estimate, then Goldschmidt / Newton steps with fma,
 // x itself for +-0 and +inf), without its rescaling of arguments below 2^-767, which is the
 // identity on these inputs.  Gives sqrt's bits there.
-__device__ __forceinline__ double sqrt_no_rescale(double x) {
+// `half` becomes 1 / (2 sqrt(x)) to within 2^-40, what the sequence knows of it by then.
+__device__ __forceinline__ double sqrt_no_rescale(double x, double &half) {
     const double y = __builtin_amdgcn_rsq(x);
     double g = x * y, h = 0.5 * y;
     const double r = fma(-h, g, 0.5);
@@ -120,7 +121,12 @@ __device__ __forceinline__ double sqrt_no_rescale(double x) {
     g = fma(d, h, g);
     d = fma(-g, g, x);
     g = fma(d, h, g);
+    half = h;
     return (x == 0.0 || x == __builtin_huge_val()) ? x : g;
+}
+__device__ __forceinline__ double sqrt_no_rescale(double x) {
+    double half;
+    return sqrt_no_rescale(x, half);
 }
 
 // p <- fma(p, t, c[k]) for k = K, K-1, ..., 0
@@ -132,12 +138,13 @@ template <class TAB, int K> __device__ __forceinline__ double horner(double p, d
 // Written without branches (zero, infinities and NaN run through the same steps, whose
 // result is then replaced by x; the scale is a select of constants), so that a wave runs it
 // as one straight sequence.  e = 3q + r with r in {0, 1, 2} is split as an unsigned division
-// of e + 1200 (frexp exponents lie in [-1073, 1024]), the same q and r as the floor division.
+// of e + 1200 (frexp exponents lie in [-1073, 1024]), the same q and r as the floor division;
+// n / 3 = n * 43691 >> 17 below 2^17, a full-rate 24-bit product instead of a high half.
 __device__ __forceinline__ double pm_cbrt(double x) {
     const bool special = x == 0.0 || !isfinite(x);
     int e;
     const double m0 = frexp(fabs(x), &e);
-    const unsigned n = (unsigned)(e + 1200), qb = n / 3u;
+    const unsigned n = (unsigned)(e + 1200), qb = __umul24(n, 43691u) >> 17;
     const int r = (int)(n - 3u * qb), q = (int)qb - 400;
     double w = horner<RcbrtCoef, 3>(coef<RcbrtCoef, 4>(), m0);
     const double s1 = sgpr_const<__builtin_bit_cast(uint64_t, CCC_CBRT_SCALE1)>();

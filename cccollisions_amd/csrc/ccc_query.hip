@@ -1603,7 +1603,10 @@ __global__ __launch_bounds__(kCcdThreads, MODE == MODE_IMPULSE ? (DET ? 3 : 4) :
     // tile as (item, root) so that the filter runs full waves
     __shared__ int64_t s_citem[NT];
     __shared__ T s_croot[NT];
+    __shared__ uint32_t s_corner[16];
     const int b = blockIdx.y, tid = threadIdx.x;
+    if (tid < 15) s_corner[tid] = corner_bytes(tid);
+    wave_sync();
     const uint32_t *__restrict__ items = arg.items + (int64_t)b * arg.cap_items;
     const uint32_t *__restrict__ tiles = arg.tiles + (int64_t)b * arg.cap_tiles;
     const int2 *__restrict__ pairs = arg.pairs + (int64_t)b * arg.cap_pairs + arg.first_pair;     // this chunk's candidate pairs
@@ -1639,7 +1642,7 @@ __global__ __launch_bounds__(kCcdThreads, MODE == MODE_IMPULSE ? (DET ? 3 : 4) :
                 const T root = s_root[base + tid];
                 // the tetrahedron is gathered once per step (from L2) rather than held
                 // across both: that keeps this phase within the CCD phases' registers
-                const ImpulseWeights<T> w = impulse_weights(gather_mtet_rec(opaque_ptr(tv), x, y, type), type, root);
+                const ImpulseWeights<T> w = impulse_weights(gather_mtet_rec(opaque_ptr(tv), x, y, type, s_corner[type]), type, root);
                 T q[4];
 #pragma unroll
                 for (int k = 0; k < 4; ++k) {
@@ -1647,7 +1650,7 @@ __global__ __launch_bounds__(kCcdThreads, MODE == MODE_IMPULSE ? (DET ? 3 : 4) :
                     type_corner(type, k, side, idx);
                     q[k] = masses[3 * (side ? y : x) + idx];
                 }
-                ip = impulse_params(gather_mtet_rec(opaque_ptr(tv), x, y, type), type, root, w, q);
+                ip = impulse_params(gather_mtet_rec(opaque_ptr(tv), x, y, type, s_corner[type]), type, root, w, q);
             }
             ImpulseParams<T> pp;      // lane l ^ 32's parameters
             pp.nrm.x = __shfl_xor(ip.nrm.x, 32);
@@ -1736,7 +1739,7 @@ __global__ __launch_bounds__(kCcdThreads, MODE == MODE_IMPULSE ? (DET ? 3 : 4) :
             int64_t x, y;
             int type;
             unpack_item(rit, x, y, type);
-            acc = filter_collision(gather_mtet_rec(opaque_ptr(tv), x, y, type), type, root);
+            acc = filter_collision(gather_mtet_rec(opaque_ptr(tv), x, y, type, s_corner[type]), type, root);
         }
         const unsigned long long m = __ballot(acc);
         if (acc) {
@@ -1794,7 +1797,7 @@ __global__ __launch_bounds__(kCcdThreads, MODE == MODE_IMPULSE ? (DET ? 3 : 4) :
             unpack_item(it, x, y, type);
             T cf[4];
             {
-                const MTet<T> m = gather_mtet_rec(tv, x, y, type);
+                const MTet<T> m = gather_mtet_rec(tv, x, y, type, s_corner[type]);
                 cubic_coeffs(m, cf);
             }
             code = cubic_prepare(cf[0], cf[1], cf[2], cf[3], st);

@@ -48,6 +48,17 @@ class Workspace {
     ~Workspace();
     void *get(size_t bytes);
     template <typename P> P *get_as(size_t count) { return static_cast<P *>(get(count * sizeof(P))); }
+    // NULL when there is no room; the Workspace has not failed then.
+    template <typename P> P *try_get_as(size_t count) {
+        const bool failed = failed_;
+        P *p = get_as<P>(count);
+        if (!p) {
+            failed_ = failed;
+            if (!arena_) (void)hipGetLastError();
+            clear_error();
+        }
+        return p;
+    }
     // Returns a buffer obtained from get() before the Workspace ends (stream-ordered).  In
     // arena mode only the most recent buffer can be returned (its bytes become free again).
     void release(void *p);
@@ -219,6 +230,7 @@ struct ResidentPass {
     int ccd_blocks_per_cu;       // grid cap of k_ccd (0: 128)
     const int64_t *leaf_ids;     // the tree when its leaves are in another order than the triangles (fitted), else NULL
     long long *det_acc;
+    double *lines;               // non-NULL: the sums as lines, dv / dx / cnt not written (line_sums)
     void *dv, *dx;
     int32_t *cnt;
     DevCounters *ctr;
@@ -226,6 +238,9 @@ struct ResidentPass {
 ccc_status resident_pass(ccc_context *ctx, const ResidentPass &p, void *arena, size_t arena_bytes, hipStream_t s);
 size_t resident_pass_arena_bytes(ccc_context *ctx, const ResidentPass &p);
 constexpr int kDetWordsPerCorner = 24;
+constexpr int kLineWordsPerCorner = 8;     // dv xyz, dx xyz, count, 0
+// dv, dx and cnt of every corner from its line.
+ccc_status line_sums(const double *lines, int64_t corners, int32_t dtype, void *dv, void *dx, int32_t *cnt, hipStream_t s);
 
 // Buffers a call fills before it starts (a kernel instead of hipMemsetAsync, so that the
 // calls stay capturable): `words` 32-bit words of the repeated 64-bit `value`.

@@ -45,8 +45,10 @@ __global__ void k_gather_soup(const T *__restrict__ x, const int64_t *__restrict
 // x1[v] += (sum of the finite dx of v's corners) / (sum of their cnt), over v's corners in
 // ascending corner order starting from zero (the order numpy.add.at uses); a corner whose
 // correction has a non-finite component contributes neither.
+// The corner sums come from dx and cnt or, where there are lines, from the corner's line.
 template <typename T>
 __global__ void k_apply_corrections(T *__restrict__ x1, const T *__restrict__ dx, const int32_t *__restrict__ cnt,
+                                    const double *__restrict__ lines,
                                     const int32_t *__restrict__ off, const int32_t *__restrict__ corner, int64_t nv) {
     const int64_t v = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (v >= nv) return;
@@ -54,12 +56,13 @@ __global__ void k_apply_corrections(T *__restrict__ x1, const T *__restrict__ dx
     double k = 0.0;
     for (int32_t j = off[v]; j < off[v + 1]; ++j) {
         const int64_t c = corner[j];
-        const T a = dx[3 * c + 0], b = dx[3 * c + 1], d = dx[3 * c + 2];
+        const double *l = lines + kLineWordsPerCorner * c;
+        const T a = lines ? (T)l[3] : dx[3 * c + 0], b = lines ? (T)l[4] : dx[3 * c + 1], d = lines ? (T)l[5] : dx[3 * c + 2];
         if (!(isfinite(a) && isfinite(b) && isfinite(d))) continue;
         sx = sx + a;
         sy = sy + b;
         sz = sz + d;
-        k = k + (double)cnt[c];
+        k = k + (lines ? l[6] : (double)cnt[c]);
     }
     if (k > 0.0) {
         x1[3 * v + 0] = (T)((double)x1[3 * v + 0] + (double)sx / k);
@@ -121,6 +124,7 @@ struct ccc_sim {
     int2 *pairs = nullptr;
     int64_t cap_pairs = 0;
     long long *det_acc = nullptr;
+    double *lines = nullptr;
     DevCounters *ctr = nullptr;
     DevCounters *h_ctr = nullptr;         // pinned host copy of the per-pass counters
     void *arena = nullptr;                // own workspace (allocated at the first step that needs it)
@@ -159,6 +163,10 @@ static void drop_graphs(ccc_sim *s) {
     s->graphs.clear();
 }
 
+static bool fitted(const ccc_sim *s) { return s->meshes == 1 && s->o.morton != CCC_MORTON_COMPAT; }
+// A fitted tree is asked for where the faces are in no spatial order: the sums go to lines.
+static double *lines_of(const ccc_sim *s) { return fitted(s) ? s->lines : nullptr; }
+
 static ResidentPass pass_of(const ccc_sim *s, int it) {
     ResidentPass p{};
     p.bboxes = s->bboxes;
@@ -173,8 +181,9 @@ static ResidentPass pass_of(const ccc_sim *s, int it) {
     p.cap_pairs = s->cap_pairs;
     p.chunk = s->o.pair_chunk > 0 ? s->o.pair_chunk : 0;
     p.ccd_blocks_per_cu = s->o.ccd_blocks_per_cu;
-    p.leaf_ids = s->meshes == 1 && s->o.morton != CCC_MORTON_COMPAT ? s->tree : nullptr;
+    p.leaf_ids = fitted(s) ? s->tree : nullptr;
     p.det_acc = s->det_acc;
+    p.lines = lines_of(s);
     p.dv = s->dv;
     p.dx = s->dx;
     p.cnt = s->cnt;
@@ -206,9 +215,11 @@ static ccc_status enqueue_step(ccc_sim *s, void *arena, size_t bytes, hipStream_
         r = resident_pass(s->ctx, pass_of(s, it), arena, bytes, st);
         if (r != CCC_OK) return r;
         CCC_TIMED(tm, "sim_update", hipLaunchKernelGGL((k_apply_corrections<T>), dim3(grid_for(s->nv, 256)), dim3(256), 0, st,
-                                                       (T *)s->x1, (const T *)s->dx, s->cnt, s->csr_off, s->csr_corner, s->nv));
+                                                       (T *)s->x1, (const T *)s->dx, s->cnt, lines_of(s), s->csr_off, s->csr_corner, s->nv));
         CCC_LAUNCH_CHECK("k_apply_corrections");
     }
+    // the last pass's sums as the caller reads them
+    if (lines_of(s) && s->o.iters > 0) return line_sums(s->lines, corners, s->dtype, s->dv, s->dx, s->cnt, st);
     return CCC_OK;
 }
 
@@ -409,6 +420,8 @@ ccc_status ccc_sim_create(ccc_context *ctx, const void *x0, const void *x1, int6
     A((void **)&s->ctr, sizeof(DevCounters) * (size_t)o.iters);
     if (num_meshes > 1) A((void **)&s->mesh_end, sizeof(int32_t) * mend.size());
     if (o.deterministic) A((void **)&s->det_acc, sizeof(long long) * kDetWordsPerCorner * 3 * (size_t)num_faces);
+    else if (r == CCC_OK && fitted(s) && dmalloc((void **)&s->lines, sizeof(double) * kLineWordsPerCorner * 3 * (size_t)num_faces) != CCC_OK)
+        clear_error();     // without lines the passes add to dv, dx and cnt directly
     if (r == CCC_OK) r = grow_pairs(s, (int64_t)o.max_candidates * num_faces);
     if (r == CCC_OK && hipHostMalloc((void **)&s->h_ctr, sizeof(DevCounters) * (size_t)o.iters) != hipSuccess) {
         set_error("pinned host allocation failed");
@@ -451,7 +464,7 @@ void ccc_sim_destroy(ccc_sim *s) {
     drop_graphs(s);
     for (void *p : {s->x0, s->x1, s->x1_save, s->masses, s->t0, s->t1, s->bboxes, s->dv, s->dx, (void *)s->faces, (void *)s->tree,
                     (void *)s->cnt, (void *)s->csr_off, (void *)s->csr_corner, (void *)s->mesh_end, (void *)s->pairs,
-                    (void *)s->det_acc, (void *)s->ctr, s->arena})
+                    (void *)s->det_acc, (void *)s->lines, (void *)s->ctr, s->arena})
         dfree(p);
     if (s->h_ctr) (void)hipHostFree(s->h_ctr);
     if (s->cs) (void)hipStreamDestroy(s->cs);
@@ -590,6 +603,7 @@ size_t ccc_sim_footprint(const ccc_sim *s) {
                sizeof(DevCounters) * (size_t)s->o.iters + sizeof(int2) * (size_t)s->cap_pairs;
     if (s->mesh_end) b += sizeof(int32_t) * (size_t)s->nf;
     if (s->det_acc) b += sizeof(long long) * kDetWordsPerCorner * 3 * (size_t)s->nf;
+    if (s->lines) b += sizeof(double) * kLineWordsPerCorner * 3 * (size_t)s->nf;
     return b + s->arena_bytes;
 }
 

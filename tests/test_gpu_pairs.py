@@ -103,11 +103,11 @@ def test_items_at_batch_edges(ccc, oracle, n, chunk):
 
 
 @pytest.mark.parametrize("dtype", [np.float64, np.float32])
-@pytest.mark.parametrize("m", [1, 31, 33, 64, 127, 129, 300])
+@pytest.mark.parametrize("m", [1, 31, 33, 64, 127, 129, 300, 32767, 32768])
 def test_impulses_of_given_rows(ccc, oracle, m, dtype):
     """compute_impulses_from_collisions at the edges of its runs: two meshes' rows with padding
     and out-of-range rows among them, shuffled, each row more than once, so that one corner
-    takes many shares.  Float sums of at most 4 m terms: within 8 m ulp of the largest."""
+    takes many shares; from 65,536 rows on they are summed in lines.  Float sums of at most 4 m terms: within 8 m ulp of the largest."""
     c = -np.ones((2, m, 3), np.int64)
     r = np.zeros((2, m, 1), dtype)
     t, want = [], []

@@ -1602,7 +1602,7 @@ template <typename P> __device__ __forceinline__ P *opaque_ptr(P *p) {
 // current code 32 per lane and 40% slower again); at three 13% slower.  Staging each wave's
 // query triangle in LDS (so that half the corner reads leave the vector memory path) made
 // the impulse mode spill and took 196-209 ms per step instead of 177.
-constexpr int kCollectFlush = 64;
+constexpr int kCollectFlush = 128;
 
 // Waves per SIMD asked of the compiler: the deterministic table's LDS (12.3 KB) allows only
 // 3.25 waves, and at four its registers spilled (37.28 against 37.06 ms per pass at three).
@@ -1822,10 +1822,13 @@ __global__ __launch_bounds__(kCcdThreads, MODE == MODE_IMPULSE ? (SUMS == SUMS_D
     // blocks running beside it are far away in the list, so that their atomics fall on other
     // corners (tiles dealt out one by one: 129.6 instead of 104 ms per step of the 130k cloth,
     // 8.5 instead of 6.8 of the garment scene, in the order that k_pairs writes its pairs).
-    // With few tiles the runs are up to 8 tiles long, on fewer blocks, so that 8,192 blocks
-    // share them: a block's start and its last, partial rounds cost as much as several tiles
-    // (collect mode on 23k triangles, 93k tiles on 32,768 blocks: 375 us, on 8,192: 201).
-    const int tall = (tper + tstep - 1) / tstep, tfew = (ntiles + 8191) / 8192, tmin = tfew < 8 ? tfew : 8;
+    // With few tiles the runs are up to kLongRun tiles long, on fewer blocks, so that 8,192
+    // blocks share them: a block's start and its last, partial rounds cost as much as several
+    // tiles, and in collect mode one more reservation of rows (23k triangles, 93k tiles on
+    // 32,768 blocks: 375 us; runs of 8: 201; of 16 and rows written 128 at a time: 182.  Runs
+    // of 16 in impulse mode, pass of 33k triangles in fp32: 335 -> 351).
+    constexpr int kLongRun = MODE == MODE_COLLECT ? 16 : 8;
+    const int tall = (tper + tstep - 1) / tstep, tfew = (ntiles + 8191) / 8192, tmin = tfew < kLongRun ? tfew : kLongRun;
     const int trun = tall > tmin ? tall : tmin;
     const int tfirst = (int)blockIdx.x / kXcds * trun, tlast = tfirst + trun < tper ? tfirst + trun : tper;
     constexpr uint32_t kNoItem = 0xffffffffu;   // type 15 does not exist

@@ -18,7 +18,7 @@ struct ccc_context {
     ccc_free_fn free_fn;
     void *user;
     int num_cus;
-    // pairs per narrow-phase chunk over the whole batch (0: the default, 2^25)
+    // pairs per narrow-phase chunk over the whole batch (0: the default)
     int64_t pair_chunk = 0;
     // this device's copy of the allocation-free entry point's scratch array
     void *scratch = nullptr;

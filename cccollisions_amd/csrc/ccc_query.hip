@@ -1,14 +1,16 @@
-// Queries over the BVH wire format for gfx950: tree preparation, traversal, the 15-way
+// Queries over the BVH wire format for gfx950: preparation, candidate pairs, the 15-way
 // sub-primitive box filter, the fused CCD (coefficients -> cubic -> filter -> collision or
 // impulse) kernel, static proximity, static triangle-triangle SAT and impulses from
 // collision lists.
 //
 // Pipeline of one query call (all batch elements at once, batch index = blockIdx.y):
-//   check tree -> rightmost leaf per internal node -> 64-byte traversal nodes (children's
-//   fp32 boxes rounded outward and grown by the threshold) -> traversal (one lane per
-//   query leaf, LDS stack, exact fp64 leaf test, wave-staged appends) -> candidate pairs
-//   -> per pair: 15-bit sub-primitive mask -> packed (x, y, type) items -> per item:
-//   narrow phase.
+//   k_prep: is the tree the index tree, boxes of the chunks of 64 leaf positions and of the
+//   groups of 16 queries, vertex records -> k_pairs: each group against the chunks behind it,
+//   exact leaf tests -> candidate pairs -> k_items: per pair the 15-bit sub-primitive mask and
+//   its items, by kind in tiles of 64 -> k_ccd: the narrow phase and the impulse sums.
+// Any other tree (another builder's, a fitted one given back to a stateless call) takes the
+// checked walk of GeneralTree instead of k_pairs; the static queries share the pairs and take
+// k_subprim / k_proximity / k_sat.
 #include <float.h>
 #include <limits.h>
 
@@ -28,8 +30,8 @@ constexpr int kTravThreads = 64;   // one wave per traversal block (128: 20.2 ms
 constexpr int kStackShort = 24;
 constexpr int kStackDeep = 32;
 constexpr int kStage = 512;       // staged pairs per wave before a flush
-// queries start from the subtrees this deep below the root (k_traverse per pass on the 130k
-// cloth: depth 6 2.85 ms, 7 2.02 ms, 8 2.60 ms)
+// queries start from the subtrees this deep below the root (measured when every query walked:
+// k_traverse per pass on the 130k cloth at depth 6 2.85 ms, 7 2.02 ms, 8 2.60 ms)
 constexpr int kFrontierDepth = 7;
 constexpr int kFrontier = 1 << kFrontierDepth;
 
@@ -1591,17 +1593,20 @@ template <typename P> __device__ __forceinline__ P *opaque_ptr(P *p) {
 //      CCD phases); lanes l and l ^ 32 exchange them, and each half of the chunk adds its
 //      corners' shares to the table and drains it.  The scatter stays in this
 //      kernel: run as a kernel of its own over per-workgroup collision lists it took 14 ms
-//      per pass on the 130k cloth against ~6 here, where other workgroups' fp64 work hides
-//      its atomic latency.
+//      per pass on the 130k cloth against ~6 here (both with one sum per word), where other
+//      workgroups' fp64 work hides its atomic latency.
 //      (collect mode) accepted rows are written kCollectFlush at a time with one
 //      reservation (the row counter is one contended device address).
 // Each lane's item of the next tile is loaded while this tile is solved.  The cubic's
 // branches diverge within the wave whatever the order of the items, so the items are not
 // grouped by branch.  Occupancy: the impulse mode four waves per SIMD (128 VGPRs).  At five
-// waves the impulse mode spilled (once about a hundred registers and 40% slower; with the
-// current code 32 per lane and 40% slower again); at three 13% slower.  Staging each wave's
-// query triangle in LDS (so that half the corner reads leave the vector memory path) made
-// the impulse mode spill and took 196-209 ms per step instead of 177.
+// waves the impulse mode spills 41 registers (155 ms per step of the 130k cloth instead of
+// 104); at three it was 13% slower.  What bounds it at four (10.4 ms per pass there, 6.2 M
+// tiles): vector instructions issue 77% of the time, 750 per tile of which 55% fp64, and each
+// CU's L1 takes 0.83 accesses per cycle with the corner gathers, 24.5 per gather instruction;
+// fewer of one alone buys a third of its share.  A single-precision test of the roots from the
+// registers of the item's lane, ahead of the filter's gather, took the gathers down by a fifth
+// but left 56% of the roots undecided and cost 16% more instructions: 110 ms; not kept.
 constexpr int kCollectFlush = 128;
 
 // Waves per SIMD asked of the compiler: the deterministic table's LDS (12.3 KB) allows only

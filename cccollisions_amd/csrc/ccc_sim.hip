@@ -272,8 +272,8 @@ static ccc_status grow_pairs(ccc_sim *s, int64_t cap) {
     return CCC_OK;
 }
 
-// One step with the given workspace; re-runs it (from the saved x1) after a capacity or
-// stack overflow.  Synchronises `st`.
+// One step with the given workspace; re-runs it (from the saved x1) after a capacity
+// overflow.  Synchronises `st`.
 static ccc_status run_step(ccc_sim *s, void *arena, size_t bytes, hipStream_t st) {
     for (int attempt = 0; attempt < 4; ++attempt) {
         const bool own = arena == nullptr;
@@ -507,8 +507,8 @@ ccc_status ccc_sim_autotune(ccc_sim *s, void *workspace, size_t workspace_bytes,
             return CCC_OK;
         }
     }
-    // a first step settles the candidate capacity and the stack; every timed step then starts
-    // from the same x1
+    // a first step settles the candidate capacity; every timed step then starts from the
+    // same x1
     const size_t vb = s->esz * 3 * (size_t)s->nv;
     void *x1_start = nullptr;
     ccc_status r = dmalloc(&x1_start, vb);

@@ -663,7 +663,7 @@ PYBIND11_MODULE(_cccollisions, m) {
     m.def("set_fixed_capacity", &set_fixed_capacity,
           "Keep the reference candidate capacity (max_candidates_per_triangle * N) instead of growing it", py::arg("on"));
     m.def("set_pair_chunk", &set_pair_chunk,
-          "Candidate pairs per narrow-phase chunk over a call's batch (0: default 2^25); results do not depend on it",
+          "Candidate pairs per narrow-phase chunk over a call's batch (0: default 2^26, 2^25 for the static queries); results do not depend on it",
           py::arg("pairs"));
     m.def("set_morton_mode", &set_morton_mode,
           "Morton codes of the trees bvh / bvh_motion build: 0 the reference's (default), 1 fitted scene box with "

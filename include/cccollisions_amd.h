@@ -277,8 +277,7 @@ ccc_status ccc_compute_impulses_noalloc(ccc_context *ctx, const void *bboxes, co
  * them all.  A step neither allocates nor waits on the host until its end: it is captured
  * once as a HIP graph (opts.graph) per workspace arena and replayed.  At the end of a step
  * the per-pass counters are read; a pass that found more candidate pairs than the list
- * holds, or whose traversal needed the deep stack, grows the list and the step runs again
- * from the saved x1.  All calls on one simulation must be serialised by the caller. */
+ * holds grows the list and the step runs again from the saved x1.  All calls on one simulation must be serialised by the caller. */
 typedef struct ccc_sim ccc_sim;
 typedef struct {
     int32_t iters;              /* impulse passes per step (default 10)                          */

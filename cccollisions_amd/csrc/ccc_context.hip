@@ -13,6 +13,29 @@ static thread_local std::string g_last_error;
 void set_error(const std::string &msg) { g_last_error = msg; }
 void clear_error() { g_last_error.clear(); }
 
+HostBlock::HostBlock(ccc_context *ctx, hipStream_t s, bool on) : ctx_(ctx), s_(s) {
+    if (!on) return;
+    {
+        std::lock_guard<std::mutex> lock(ctx->host_mu);
+        if (!ctx->host_free.empty()) {
+            p_ = ctx->host_free.back();
+            ctx->host_free.pop_back();
+            return;
+        }
+    }
+    if (hipHostMalloc(&p_, kBytes) != hipSuccess) {
+        (void)hipGetLastError();
+        p_ = nullptr;
+    }
+}
+
+HostBlock::~HostBlock() {
+    if (!p_) return;
+    if (!settled_) (void)hipStreamSynchronize(s_);
+    std::lock_guard<std::mutex> lock(ctx_->host_mu);
+    ctx_->host_free.push_back(p_);
+}
+
 Workspace::~Workspace() {
     if (arena_) return;
     for (void *p : ptrs_) {
@@ -123,7 +146,11 @@ ccc_status ccc_context_create(ccc_context **out, int device, ccc_alloc_fn alloc,
     return CCC_OK;
 }
 
-void ccc_context_destroy(ccc_context *ctx) { delete ctx; }
+void ccc_context_destroy(ccc_context *ctx) {
+    if (ctx)
+        for (void *p : ctx->host_free) (void)hipHostFree(p);
+    delete ctx;
+}
 
 const char *ccc_status_string(ccc_status status) {
     switch (status & CCC_ERR_MASK) {

@@ -28,12 +28,35 @@ struct ccc_context {
     bool profiling = false;
     std::mutex prof_mu;
     std::map<std::string, std::pair<double, int64_t>> prof;
+    // pinned blocks that calls read their counters from (HostBlock), free ones; the context
+    // keeps as many as it ever had calls at once and frees them with itself
+    std::mutex host_mu;
+    std::vector<void *> host_free;
 };
 
 namespace ccc {
 
 void set_error(const std::string &msg);
 void clear_error();
+
+// A pinned host block of kBytes for the time of one call, from the context's free ones.  NULL
+// when `on` is false or none can be had.  Kernels of `s` may write to it: settled() says that
+// the stream was waited for since; without it the destructor waits.
+class HostBlock {
+  public:
+    static constexpr size_t kBytes = 16384;
+    HostBlock(ccc_context *ctx, hipStream_t s, bool on);
+    ~HostBlock();
+    template <typename P> P *as() const { return static_cast<P *>(p_); }
+    void written() { settled_ = false; }
+    void settled() { settled_ = true; }
+
+  private:
+    ccc_context *ctx_;
+    hipStream_t s_;
+    void *p_ = nullptr;
+    bool settled_ = true;
+};
 
 // Per-call device workspace.  Buffers come from the context's allocator (or
 // hipMallocAsync on the call's stream) and are released when the Workspace goes out of

@@ -1136,8 +1136,8 @@ __global__ __launch_bounds__(kThreads) void k_subprim(const int2 *__restrict__ p
 // behind them, so that k_ccd's 64-item tiles hold one kind and nothing is reserved while it
 // runs; at the end the block reserves its tiles' descriptors (first slot, a multiple of 64,
 // plus the number of items less one), which is all that k_ccd needs to find them.  A batch's
-// entries are assembled in LDS and written as whole lines.  Bound by VALU issue (about 600
-// instructions per 64 pairs, most of them comparisons): 1.11 ms per pass of the 130k cloth
+// entries are assembled in LDS and written as whole lines.  Bound by its record reads (0.95 L1
+// accesses per cycle and CU: 18 of 16 bytes per lane and pair; vector issue 65%): 1.10 ms per pass of the 130k cloth
 // (1.20 with blocks of 512 pairs and one reservation each), 33k f32 pass 56 -> 42 us.
 constexpr int kBatch = 64;       // pairs per wave at a time
 constexpr int kSegEE = 9, kSegVF = 6;
@@ -2281,7 +2281,8 @@ __global__ void k_fold_items(DevCounters *__restrict__ ctr, int64_t B) {
 
 // End of the continuous narrow phase: the blocks' partial counts of every chunk to the
 // counters.  One wave per batch element.
-__global__ __launch_bounds__(64) void k_fold_partials(const DevPartial *__restrict__ part_all, bool coll, DevCounters *__restrict__ ctr) {
+__global__ __launch_bounds__(64) void k_fold_partials(const DevPartial *__restrict__ part_all, bool coll, DevCounters *__restrict__ ctr,
+                                                      DevCounters *__restrict__ host) {
     static_assert(kPartials == 64, "one lane per partial");
     const DevPartial p = part_all[(int64_t)blockIdx.x * kPartials + threadIdx.x];
     unsigned long long v[3] = {p.items, p.roots, p.coll};
@@ -2293,7 +2294,17 @@ __global__ __launch_bounds__(64) void k_fold_partials(const DevPartial *__restri
         ctr[blockIdx.x].items_done = v[0];
         ctr[blockIdx.x].roots = v[1];
         if (coll) ctr[blockIdx.x].coll = v[2];
+        if (host) host[blockIdx.x] = ctr[blockIdx.x];
     }
+}
+
+// The counters to pinned host memory, which the calls' waits then find written (k_fold_partials
+// does it itself).  A copy into pageable memory goes through the runtime's staging and its own
+// waits, twice per call: pass of 450 triangles 84 -> 68 us, of 20k with a tenth checked
+// 132 -> 114, static proximity on 8k 309 -> 284.
+__global__ void k_report(const DevCounters *__restrict__ ctr, int64_t B, DevCounters *__restrict__ host) {
+    const int64_t b = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (b < B) host[b] = ctr[b];
 }
 
 // Pairs per narrow-phase chunk over all batch elements of a call (the context may set
@@ -2499,6 +2510,24 @@ static ccc_status run_query(const Query &q) {
 
     // traversal, re-run once with the exact size if the capacity was exceeded
     std::vector<DevCounters> h(B);
+    HostBlock block(q.ctx, s, !q.nosync && !q.arena && B * sizeof(DevCounters) <= HostBlock::kBytes);
+    DevCounters *hp = block.as<DevCounters>();
+    // the counters on the host; `reported`: the last kernel has written them to the block
+    auto read_counters = [&](bool reported) -> ccc_status {
+        if (hp) {
+            if (!reported) {
+                block.written();
+                hipLaunchKernelGGL(k_report, dim3((unsigned)((B + 255) / 256)), dim3(256), 0, s, ctr, B, hp);
+                CCC_LAUNCH_CHECK("k_report");
+            }
+        } else {
+            CCC_HIP_TRY(hipMemcpyAsync(h.data(), ctr, sizeof(DevCounters) * B, hipMemcpyDeviceToHost, s));
+        }
+        CCC_HIP_TRY(hipStreamSynchronize(s));
+        block.settled();
+        if (hp) std::copy(hp, hp + B, h.begin());
+        return CCC_OK;
+    };
     int64_t capK = q.cap_candidates > 0 ? q.cap_candidates : 1;
     bool warn_cand = false;
     int2 *pairs = nullptr;
@@ -2532,8 +2561,7 @@ static ccc_status run_query(const Query &q) {
             CCC_LAUNCH_CHECK("k_pairs");
         }
         if (q.nosync) break;          // the caller checks the counters after its step
-        CCC_HIP_TRY(hipMemcpyAsync(h.data(), ctr, sizeof(DevCounters) * B, hipMemcpyDeviceToHost, s));
-        CCC_HIP_TRY(hipStreamSynchronize(s));
+        if ((st = read_counters(false)) != CCC_OK) return st;
         unsigned flags = 0;
         unsigned long long kmax = 0;
         for (int64_t b = 0; b < B; ++b) {
@@ -2688,7 +2716,8 @@ static ccc_status run_query(const Query &q) {
                 }
             }
             if (ccd) {
-                hipLaunchKernelGGL(k_fold_partials, dim3(B), dim3(64), 0, s, parts, q.narrow == Narrow::CCD_IMPULSE, ctr);
+                block.written();
+                hipLaunchKernelGGL(k_fold_partials, dim3(B), dim3(64), 0, s, parts, q.narrow == Narrow::CCD_IMPULSE, ctr, hp);
                 CCC_LAUNCH_CHECK("k_fold_partials");
             }
             return CCC_OK;
@@ -2701,8 +2730,7 @@ static ccc_status run_query(const Query &q) {
         }
     }
     if (q.nosync) return CCC_OK;
-    CCC_HIP_TRY(hipMemcpyAsync(h.data(), ctr, sizeof(DevCounters) * B, hipMemcpyDeviceToHost, s));
-    CCC_HIP_TRY(hipStreamSynchronize(s));
+    if ((st = read_counters(hp && ccd_query)) != CCC_OK) return st;
     bool truncated = false;
     for (int64_t b = 0; b < B; ++b) {
         const int64_t K = std::min<int64_t>((int64_t)h[b].cand, capK);

@@ -129,3 +129,44 @@ def test_impulses_of_given_rows(ccc, oracle, m, dtype):
         for got, ref in ((dv[b], want[b][0]), (dx[b], want[b][1])):
             tol = 8 * m * np.finfo(dtype).eps * max(np.abs(ref).max(), np.finfo(dtype).tiny)
             assert np.abs(got - ref).max() <= tol + 1e-12 * np.abs(ref).max()
+
+
+@pytest.mark.parametrize("batch", [1, 256, 257])
+def test_counts_of_many_elements(ccc, oracle, batch):
+    """Counters of every batch element, up to and past what a pinned block holds (256)."""
+    t0, t1, m = cases.random_soup(24, seed=4, motion=0.2)
+    rb, rt, _, _ = oracle.bvh(t0, t1)
+    _, _, cnt, _, _, counts = oracle.compute_impulses(rb, rt, t0, t1, m)
+    one = [_t(np.ascontiguousarray(np.broadcast_to(a, (batch, *a.shape)))) for a in (rb, rt, t0, t1, m)]
+    out = ccc.compute_impulses(*one, 24, 16)
+    assert ccc.last_counts() == [[counts[k] for k in ("candidates", "subprims", "roots", "collisions")]] * batch
+    np.testing.assert_array_equal(_np(out[2]), np.broadcast_to(cnt, (batch, *cnt.shape)))
+
+
+def test_counts_from_several_threads(ccc, oracle):
+    """Calls of four threads on their own streams, each reading its own counters."""
+    import threading
+
+    import torch
+    args, want, bad = [], [], []
+    for k in range(4):
+        t0, t1, m = cases.random_soup(40 + 30 * k, seed=k, motion=0.2)
+        rb, rt, _, _ = oracle.bvh(t0, t1)
+        counts = oracle.compute_impulses(rb, rt, t0, t1, m)[5]
+        args.append([_t(a[None]) for a in (rb, rt, t0, t1, m)])
+        want.append([[counts[c] for c in ("candidates", "subprims", "roots", "collisions")]])
+    torch.cuda.synchronize()
+
+    def work(k):
+        with torch.cuda.stream(torch.cuda.Stream()):
+            for _ in range(30):
+                ccc.compute_impulses(*args[k], 200, 16)
+                if ccc.last_counts() != want[k]:
+                    bad.append(k)
+
+    ts = [threading.Thread(target=work, args=(k,)) for k in range(4)]
+    for t in ts:
+        t.start()
+    for t in ts:
+        t.join()
+    assert not bad

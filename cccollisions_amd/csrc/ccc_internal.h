@@ -274,6 +274,7 @@ struct FillRegion {
 };
 struct FillRegions {
     FillRegion r[8];
+    unsigned blocks[8] = {};     // of each region's, in one launch
     int count = 0;
     void add(void *p, int64_t bytes, uint64_t value) { r[count++] = FillRegion{p, bytes / 4, value}; }
 };

@@ -2556,6 +2556,15 @@ static ccc_status run_query(const Query &q) {
     const int64_t nq = (n + kPairQ - 1) / kPairQ, groups_all = nq * B;
     const int splits = (int)std::max<int64_t>(1, std::min<int64_t>(nc, std::max<int64_t>(16384 / groups_all, groups_all < 16384 ? 3 : 1)));
     GeneralTree<T> general(q, ws, bb, ctr, s, tm);
+    // A context that fits its trees gets them back here: straight to the walk, without a first
+    // attempt that only finds out (static query on 10k triangles 208 us with it, 172 without).
+    // Packed meshes always have the index tree.
+    if (!q.nosync && !q.mesh_end && q.ctx->morton != CCC_MORTON_COMPAT) {
+        if (supers) ws.release(supers);
+        ws.release(groups);
+        ws.release(chunks);
+        if ((st = general.prepare()) != CCC_OK) return st;
+    }
     for (int attempt = 0; attempt < 2; ++attempt) {
         if (q.pairs_ext) {
             pairs = q.pairs_ext;

@@ -170,3 +170,18 @@ def test_counts_from_several_threads(ccc, oracle):
     for t in ts:
         t.join()
     assert not bad
+
+
+@pytest.mark.parametrize("n", [2, 65, 300])
+def test_index_tree_in_a_fitted_context(ccc, oracle, n):
+    """A context that fits its trees walks every tree: the index tree's pairs are the same."""
+    t0, t1, _ = cases.random_soup(n, seed=n + 9)
+    rb, rt, _, _ = oracle.bvh(t0, t1)
+    pairs, total = oracle.traverse(rb, rt, 0.0)
+    ccc.set_morton_mode(1)
+    try:
+        rows, k = _mincol(ccc, rb, rt, t0, t1, total // n + 2)
+    finally:
+        ccc.set_morton_mode(0)
+    assert k == total
+    np.testing.assert_array_equal(rows, sorted_rows(oracle.mincol(t0, t1, pairs)))

@@ -99,13 +99,14 @@ void *Workspace::get(size_t bytes) {
 // 6.4 to 6.9 TB/s on 1 to 6 GiB, where a loop over 8,192 blocks reached 4.3 to 5.0 and 8-byte
 // stores over 65,536 blocks 5.7; up to 50 MB they are alike.
 constexpr int64_t kFillWords = 4 * 256;     // per block
-__global__ __launch_bounds__(256) void k_fill_regions(FillRegions r) {
+__global__ __launch_bounds__(256) void k_fill_regions(FillRegions r, unsigned base) {
+    const unsigned block = base + blockIdx.x;
     unsigned first = 0;
     int k = 0;
-    while (k + 1 < r.count && blockIdx.x >= first + r.blocks[k]) first += r.blocks[k++];
+    while (k + 1 < r.count && block >= first + r.blocks[k]) first += r.blocks[k++];
     const FillRegion f = r.r[k];
     const uint32_t lo = (uint32_t)f.value, hi = (uint32_t)(f.value >> 32);
-    const int64_t i = (int64_t)(blockIdx.x - first) * kFillWords + 4 * threadIdx.x;
+    const int64_t i = (int64_t)(block - first) * kFillWords + 4 * threadIdx.x;
     uint32_t *p = reinterpret_cast<uint32_t *>(f.p);
     if (i + 4 <= f.words && ((uintptr_t)f.p & 15) == 0) {
         *reinterpret_cast<uint4 *>(p + i) = make_uint4(lo, hi, lo, hi);
@@ -114,17 +115,33 @@ __global__ __launch_bounds__(256) void k_fill_regions(FillRegions r) {
     for (int64_t j = i; j < i + 4 && j < f.words; ++j) p[j] = (j & 1) ? hi : lo;
 }
 
-ccc_status fill_regions(const FillRegions &regions, hipStream_t s) {
-    FillRegions r = regions;
+// A launch holds fewer than 2^32 work items (hip_runtime_api.h), which is 64 GiB here: larger
+// fills take one launch per 32 GiB.
+constexpr int64_t kFillLaunchBlocks = (int64_t)1 << 23;
+
+// Blocks of each region, and of all of them.
+static int64_t count_fill_blocks(FillRegions &r) {
     int64_t total = 0;
     for (int k = 0; k < r.count; ++k) {
         const int64_t blocks = r.r[k].words > 0 ? (r.r[k].words + kFillWords - 1) / kFillWords : 0;
         r.blocks[k] = (unsigned)blocks;
         total += blocks;
     }
-    if (total <= 0) return CCC_OK;
+    return total;
+}
+// launch(first block, blocks) for every launch of a fill of `total` blocks.
+template <typename F> static void each_fill_launch(int64_t total, F launch) {
+    for (int64_t base = 0; base < total; base += kFillLaunchBlocks)
+        launch((unsigned)base, (unsigned)std::min(total - base, kFillLaunchBlocks));
+}
+
+ccc_status fill_regions(const FillRegions &regions, hipStream_t s) {
+    FillRegions r = regions;
+    const int64_t total = count_fill_blocks(r);
     if (total > INT_MAX) return bad_arg("an output of more than 8 TiB");
-    hipLaunchKernelGGL(k_fill_regions, dim3((unsigned)total), dim3(256), 0, s, r);
+    each_fill_launch(total, [&](unsigned base, unsigned blocks) {
+        hipLaunchKernelGGL(k_fill_regions, dim3(blocks), dim3(256), 0, s, r, base);
+    });
     CCC_LAUNCH_CHECK("fill_regions");
     return CCC_OK;
 }
@@ -225,6 +242,23 @@ int ccc_context_kernel_names(ccc_context *ctx, char *buf, size_t len) {
         buf[n] = 0;
     }
     return (int)all.size();
+}
+
+int ccc_debug_fill_launches(const int64_t *bytes, int count, int64_t *blocks, int capacity) {
+    ccc::FillRegions r;
+    if (!bytes || !blocks || count < 0 || count > (int)(sizeof(r.r) / sizeof(r.r[0]))) return -1;
+    for (int k = 0; k < count; ++k) r.add(nullptr, bytes[k], 0ull);
+    const int64_t total = ccc::count_fill_blocks(r);
+    if (total > INT_MAX) return -1;
+    int launches = 0;
+    ccc::each_fill_launch(total, [&](unsigned base, unsigned n) {
+        if (launches < capacity) {
+            blocks[2 * launches] = base;
+            blocks[2 * launches + 1] = n;
+        }
+        ++launches;
+    });
+    return launches;
 }
 
 }  // extern "C"

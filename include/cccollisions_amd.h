@@ -117,6 +117,12 @@ ccc_status ccc_context_set_morton(ccc_context *ctx, int mode);
  * float (x holds 2 n values), else 0. */
 ccc_status ccc_debug_device_math(ccc_context *ctx, int what, const double *x, double *y, int64_t n, void *stream);
 
+/* Test hook (no counterpart in the reference): the launches by which a call clears `count`
+ * buffers of the given sizes: their number, and in blocks[2i], blocks[2i + 1] the first block
+ * and the number of blocks (256 work items, 4 KiB each) of launch i < capacity; -1 for what
+ * the calls refuse.  Host arithmetic only. */
+int ccc_debug_fill_launches(const int64_t *bytes, int count, int64_t *blocks, int capacity);
+
 /* Opt-in kernel timing (no counterpart in the reference; used by the benchmark).  While on,
  * every kernel launch of a call is bracketed by HIP events on the call's stream and the
  * elapsed times are accumulated per kernel name.  Enabling or disabling clears the totals. */

@@ -10,9 +10,11 @@
 #include <c10/hip/HIPStream.h>
 #include <torch/extension.h>
 
+#include <exception>
 #include <map>
 #include <mutex>
 #include <string>
+#include <utility>
 #include <vector>
 
 #include "../../include/cccollisions_amd.h"
@@ -26,8 +28,17 @@ namespace {
     CHECK_CUDA(x);     \
     CHECK_CONTIGUOUS(x)
 
+// The allocator of the contexts.  Exceptions do not pass through the C ABI: a failed allocation
+// is NULL there, which a call either does without or reports as CCC_ERR_NO_MEMORY; finish()
+// then raises what torch raised.
+thread_local std::exception_ptr g_alloc_error;
 void *torch_alloc(void *, size_t bytes, void *stream) {
-    return c10::hip::HIPCachingAllocator::raw_alloc_with_stream(bytes, (hipStream_t)stream);
+    try {
+        return c10::hip::HIPCachingAllocator::raw_alloc_with_stream(bytes, (hipStream_t)stream);
+    } catch (...) {
+        g_alloc_error = std::current_exception();
+        return nullptr;
+    }
 }
 void torch_free(void *, void *ptr, void *) { c10::hip::HIPCachingAllocator::raw_delete(ptr); }
 
@@ -84,6 +95,8 @@ void warn(const char *msg) {
 }
 
 void finish(ccc_status st, const char *what) {
+    const std::exception_ptr alloc_error = std::exchange(g_alloc_error, nullptr);
+    if ((st & CCC_ERR_MASK) == CCC_ERR_NO_MEMORY && alloc_error) std::rethrow_exception(alloc_error);
     TORCH_CHECK((st & CCC_ERR_MASK) == CCC_OK, "cccollisions.", what, " failed: ", ccc_status_string(st), ": ", ccc_last_error());
     if (st & CCC_WARN_CANDIDATES) {
         if (g_flags & CCC_FLAG_FIXED_CAPACITY)

@@ -64,7 +64,8 @@ typedef struct {
 } ccc_counts;
 
 /* Device workspace allocator (e.g. a framework's caching allocator).  Both callbacks are
- * optional; without them the library uses hipMallocAsync / hipFreeAsync on the stream. */
+ * optional; without them the library uses hipMallocAsync / hipFreeAsync on the stream.  A
+ * failed allocation is NULL (no exception passes through these functions). */
 typedef void *(*ccc_alloc_fn)(void *user, size_t bytes, void *stream);
 typedef void (*ccc_free_fn)(void *user, void *ptr, void *stream);
 

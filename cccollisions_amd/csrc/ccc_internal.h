@@ -218,7 +218,7 @@ struct alignas(64) DevCounters {
 static_assert(sizeof(DevCounters) == 64, "DevCounters is one 64-byte line");
 
 // Counts that nobody reads before the call ends: every block of the narrow phase adds its own
-// to one of kPartials lines, and k_fold_items sums them.  An atomic on one device address
+// to one of up to kPartials lines of its batch element, and k_fold_partials sums them.  An atomic on one device address
 // takes 6-13 ns however many waves issue them: on the shared counters the 32,768 blocks of
 // k_ccd spent 0.4-0.8 ms of a pass on two of them each (all of its time on the 33k f32 pass).
 struct alignas(128) DevPartial {

@@ -696,9 +696,8 @@ __global__ __launch_bounds__(kTravThreads) void k_traverse(const T *__restrict__
 // chunks: 130k cloth (5.9e7 pairs) 1,770 -> 390 us, packed 12 meshes (1.4e8 pairs) 9,300 ->
 // 1,000 us, shuffled 32k 500 -> 63 us, garment 122k 220 -> 130 us, 33k f32 144 -> 38 us.
 
-// The answer of k_prep's tree check, one 256-byte line per batch element: every wave of
+// The answer of k_prep's tree check is a word per batch element (`foreign`): every wave of
 // k_pairs reads it, so it lies apart from the counters that they reserve pairs on.
-constexpr int kForeignStep = 64;
 
 constexpr int kPairQ = 16;        // queries per wave of k_pairs, each held by 64 / kPairQ lanes
 
@@ -763,7 +762,7 @@ __global__ __launch_bounds__(256) void k_prep(const T *__restrict__ bb_all, cons
         } else {
             ok = ok && l == -1 && rr == -1 && tree[4 * r + 3] == r - (n - 1);
         }
-        if (!ok) foreign[kForeignStep * b] = 1u;
+        if (!ok) foreign[b] = 1u;
     } else if (blockIdx.x < row_blocks + leaf_blocks) {
         const int64_t p = (int64_t)(blockIdx.x - row_blocks) * 256 + threadIdx.x;
         if ((p & ~(int64_t)(kChunk - 1)) >= n) return;
@@ -862,7 +861,7 @@ __global__ __launch_bounds__(64 * kPairWaves) void k_pairs(const T *__restrict__
     int *s_leaf = s_leafs[w], *s_id = s_idss[w];
     uint32_t *s_ent = s_ents[w];
     DevCounters *ctr = ctr_all + b;
-    if (foreign_all && foreign_all[kForeignStep * b]) {
+    if (foreign_all && foreign_all[b]) {
         if (blockIdx.x == 0 && threadIdx.x == 0) atomicOr(&ctr->flags, DEV_FOREIGN);
         return;
     }
@@ -1132,10 +1131,11 @@ __global__ __launch_bounds__(kThreads) void k_subprim(const int2 *__restrict__ p
 // (collisions_continuous.cu:234-318, :340-396), as 32-bit items (pair index within the chunk)
 // << 4 | type for k_ccd.
 // Each wave takes a contiguous run of pairs, 64 at a time (lane = pair), and keeps its
-// edge-edge items in its own kSegEE slots per pair and its vertex-face items in the kSegVF
-// behind them, so that k_ccd's 64-item tiles hold one kind and nothing is reserved while it
-// runs; at the end the block reserves its tiles' descriptors (first slot, a multiple of 64,
-// plus the number of items less one), which is all that k_ccd needs to find them.  A batch's
+// edge-edge items in the kSegEE slots per pair that the run's place in the list gives it and
+// its vertex-face items in the kSegVF behind them, so that k_ccd's 64-item tiles hold one kind,
+// nothing is reserved while it runs and the list is as long as its pairs can make it; at the
+// end the block reserves its tiles' descriptors (first slot, a multiple of 64, plus the number
+// of items less one), which is all that k_ccd needs to find them.  A batch's
 // entries are assembled in LDS and written as whole lines.  Bound by its record reads (0.95 L1
 // accesses per cycle and CU: 18 of 16 bytes per lane and pair; vector issue 65%): 1.10 ms per pass of the 130k cloth
 // (1.20 with blocks of 512 pairs and one reservation each), 33k f32 pass 56 -> 42 us.
@@ -1146,8 +1146,8 @@ constexpr int kItemBlock = 4;    // waves per block
 template <typename T>
 __global__ __launch_bounds__(64 * kItemBlock) void k_items(const int2 *__restrict__ pairs_all, int64_t capK, int64_t c0, int64_t c1,
                                               const T *__restrict__ tv_all, int64_t n, uint32_t *__restrict__ list_all, int64_t capM,
-                                              unsigned slot_run, uint32_t *__restrict__ tile_all, int64_t capT,
-                                              DevPartial *__restrict__ part_all, DevCounters *__restrict__ ctr_all) {
+                                              uint32_t *__restrict__ tile_all, int64_t capT,
+                                              DevPartial *__restrict__ part_all, int nparts, DevCounters *__restrict__ ctr_all) {
     // (pair in batch) << 4 | type: edge-edge entries from the front, vertex-face ones from kSegEE kBatch on
     __shared__ unsigned short s_ents[kItemBlock][(kSegEE + kSegVF) * kBatch];
     __shared__ unsigned s_tiles[kItemBlock];
@@ -1161,11 +1161,10 @@ __global__ __launch_bounds__(64 * kItemBlock) void k_items(const int2 *__restric
     const int64_t per = (nbatch + kXcds - 1) / kXcds, step = (int64_t)gridDim.x / kXcds * kItemBlock, run = (per + step - 1) / step;
     const int64_t base = (int64_t)(blockIdx.x % kXcds) * per, k0 = ((int64_t)(blockIdx.x / kXcds) * kItemBlock + w) * run;
     const int64_t first = base + k0, last = base + (k0 + run < per ? k0 + run : per), stop = last < nbatch ? last : nbatch;
-    const unsigned wave = blockIdx.x * kItemBlock + w;
     const int2 *pairs = pairs_all + (int64_t)b * capK + c0;
     const T *tv = tv_all + (int64_t)b * n * 18;
-    // slot_run >= run: the batches per wave that the list was sized for
-    const uint32_t slot_ee = wave * ((kSegEE + kSegVF) * kBatch * slot_run), slot_vf = slot_ee + kSegEE * kBatch * slot_run;
+    const uint32_t mine = first < stop ? (uint32_t)(stop - first) : 0u;       // this wave's batches
+    const uint32_t slot_ee = (uint32_t)first * ((kSegEE + kSegVF) * kBatch), slot_vf = slot_ee + mine * (kSegEE * kBatch);
     uint32_t *list_ee = list_all + (int64_t)b * capM + slot_ee, *list_vf = list_all + (int64_t)b * capM + slot_vf;
     unsigned nee = 0, nvf = 0;      // items in the two segments
     int2 pr = make_int2(0, 0);
@@ -1228,7 +1227,7 @@ __global__ __launch_bounds__(64 * kItemBlock) void k_items(const int2 *__restric
     for (unsigned k = lane; k < tee; k += 64) tiles[k] = slot_ee + 64 * k + (nee - 64 * k < 64u ? nee - 64 * k - 1u : 63u);
     for (unsigned k = lane; k < tvf; k += 64) tiles[tee + k] = slot_vf + 64 * k + (nvf - 64 * k < 64u ? nvf - 64 * k - 1u : 63u);
     if (lane == 0 && nee + nvf > 0)
-        atomicAdd(&part_all[(int64_t)b * kPartials + blockIdx.x % kPartials].items, (unsigned long long)(nee + nvf));
+        atomicAdd(&part_all[(int64_t)b * nparts + (blockIdx.x & (nparts - 1))].items, (unsigned long long)(nee + nvf));
 }
 
 // ---- fused narrow phase --------------------------------------------------------------------
@@ -1619,7 +1618,7 @@ template <typename T> struct CcdArgs {
     const int2 *pairs;          // [B][cap_pairs], this chunk's from first_pair on
     const T *tv;                // vertex records
     DevCounters *ctr;
-    DevPartial *parts;
+    DevPartial *parts;          // [B][nparts]
     int64_t cap_items, cap_tiles, cap_pairs, first_pair, n;
     // impulse mode
     const T *masses;
@@ -1631,6 +1630,7 @@ template <typename T> struct CcdArgs {
     int64_t *coll;
     T *roots;
     int64_t out_cap;
+    int nparts;
 };
 // The arguments read again where they are used: what only the scatter or the output needs
 // would otherwise sit in scalar registers, or in lanes of vector registers, through the solver
@@ -1818,7 +1818,7 @@ __global__ __launch_bounds__(kCcdThreads, MODE == MODE_IMPULSE ? (SUMS == SUMS_D
     // the packed (x, y, type) form is made when the tile starts.  A tile's items are of one
     // kind (k_items), so its roots and collisions take one branch of the filter and of the
     // impulse in the whole wave, but for the roots carried over a change.
-    // tile counts in 32 bits (at most 15 * 2^28 / 64 tiles and two per wave of k_items): the
+    // tile counts in 32 bits (at most 15 * 2^28 / 64 tiles): the
     // kernel's uniform values fill the scalar registers
     const int ntiles = (int)arg.ctr[b].tiles;
     const int tper = (ntiles + kXcds - 1) / kXcds, tstep = (int)gridDim.x / kXcds;
@@ -1945,7 +1945,8 @@ __global__ __launch_bounds__(kCcdThreads, MODE == MODE_IMPULSE ? (SUMS == SUMS_D
         write_rows(fill);
     }
     if (tid == 0) {
-        DevPartial *part = late_args<T>()->parts + (int64_t)b * kPartials + blockIdx.x % kPartials;
+        auto *late = late_args<T>();
+        DevPartial *part = late->parts + (int64_t)b * late->nparts + (blockIdx.x & (late->nparts - 1));
         if (nroots) atomicAdd(&part->roots, nroots);
         if (MODE == MODE_IMPULSE && ncoll) atomicAdd(&part->coll, ncoll);
     }
@@ -2299,10 +2300,11 @@ __global__ void k_fold_items(DevCounters *__restrict__ ctr, int64_t B) {
 
 // End of the continuous narrow phase: the blocks' partial counts of every chunk to the
 // counters.  One wave per batch element.
-__global__ __launch_bounds__(64) void k_fold_partials(const DevPartial *__restrict__ part_all, bool coll, DevCounters *__restrict__ ctr,
-                                                      DevCounters *__restrict__ host) {
+__global__ __launch_bounds__(64) void k_fold_partials(const DevPartial *__restrict__ part_all, int nparts, bool coll,
+                                                      DevCounters *__restrict__ ctr, DevCounters *__restrict__ host) {
     static_assert(kPartials == 64, "one lane per partial");
-    const DevPartial p = part_all[(int64_t)blockIdx.x * kPartials + threadIdx.x];
+    DevPartial p{};
+    if ((int)threadIdx.x < nparts) p = part_all[(int64_t)blockIdx.x * nparts + threadIdx.x];
     unsigned long long v[3] = {p.items, p.roots, p.coll};
 #pragma unroll
     for (int d = 1; d < 64; d <<= 1)
@@ -2368,14 +2370,22 @@ template <typename T> class GeneralTree {
         : q_(q), ws_(ws), bb_(bb), ctr_(ctr), s_(s), tm_(tm) {}
     bool used() const { return used_; }
     bool deep() const { return deep_; }
+    void use() { used_ = true; }
     void go_deep() { deep_ = true; }
+    bool prepared() const { return prepared_; }
+    // The buffers, last in, first out.
+    void release() {
+        for (void *p : {(void *)qbox_, (void *)frontier_, (void *)recs_, (void *)qnodes_, (void *)nodes_, (void *)lo_, (void *)rm_, (void *)claims_})
+            ws_.release(p);
+        prepared_ = false;
+    }
     ccc_status prepare() {
-        used_ = true;
+        prepared_ = true;
         const int64_t B = q_.B, n = q_.n, rows = 2 * n - 1, nint = n > 1 ? n - 1 : 1;
-        int *claims = ws_.get_as<int>(B * n);
-        int *rm = ws_.get_as<int>(B * nint);
-        int *lo = ws_.get_as<int>(B * nint);
-        TNode *nodes = ws_.get_as<TNode>(B * nint);
+        int *claims = claims_ = ws_.get_as<int>(B * n);
+        int *rm = rm_ = ws_.get_as<int>(B * nint);
+        int *lo = lo_ = ws_.get_as<int>(B * nint);
+        TNode *nodes = nodes_ = ws_.get_as<TNode>(B * nint);
         qnodes_ = ws_.get_as<QNode>(B * nint);
         recs_ = ws_.get_as<LeafRec>(B * n);
         frontier_ = ws_.get_as<Frontier>(B);
@@ -2431,7 +2441,9 @@ template <typename T> class GeneralTree {
     DevCounters *ctr_;
     hipStream_t s_;
     KernelTimer &tm_;
-    bool used_ = false, deep_ = false;
+    bool used_ = false, deep_ = false, prepared_ = false;
+    int *claims_ = nullptr, *rm_ = nullptr, *lo_ = nullptr;
+    TNode *nodes_ = nullptr;
     QNode *qnodes_ = nullptr;
     LeafRec *recs_ = nullptr;
     Frontier *frontier_ = nullptr;
@@ -2440,11 +2452,12 @@ template <typename T> class GeneralTree {
 };
 
 // The list of the continuous narrow phase for chunks of at most `chunk` pairs per batch
-// element: k_items' waves, the batches of 64 pairs that each takes at most, and the list
-// slots these can fill.
+// element, in whole batches of 64 pairs: 15 slots per pair, a descriptor per 64 of them (a
+// wave's items of one kind start at a multiple of 64 and fill at most its slots), and the
+// blocks of k_items.
 struct ListPlan {
     int64_t chunk, slots, tiles;
-    unsigned grid, run;
+    unsigned grid;
     // the slots and the tiles' descriptors, each rounded as a workspace buffer is
     size_t bytes(int64_t B) const {
         auto r = [](size_t b) { return (b + 255) & ~(size_t)255; };
@@ -2452,13 +2465,19 @@ struct ListPlan {
     }
 };
 static ListPlan list_plan(const ccc_context *ctx, int64_t chunk, int64_t B) {
-    const int64_t batches = (chunk + kBatch - 1) / kBatch;
-    int64_t waves = std::max<int64_t>(std::min<int64_t>(batches, (int64_t)ctx->num_cus * kItemWaves / B), kXcds);
+    const int64_t batches = (chunk + kBatch - 1) / kBatch, slots = batches * (kSegEE + kSegVF) * kBatch;
+    static_assert(kSegEE * kBatch % 64 == 0 && kSegVF * kBatch % 64 == 0, "segments start at multiples of a tile");
+    const int64_t waves = std::max<int64_t>(std::min<int64_t>(batches, (int64_t)ctx->num_cus * kItemWaves / B), 1);
     constexpr int kGroup = kXcds * kItemBlock;
-    waves = (waves + kGroup - 1) / kGroup * kGroup;
-    const int64_t per = (batches + kXcds - 1) / kXcds, run = (per + waves / kXcds - 1) / (waves / kXcds);
-    const int64_t slots = waves * run * (kSegEE + kSegVF) * kBatch;
-    return ListPlan{chunk, slots, slots / 64 + 2 * waves, (unsigned)(waves / kItemBlock), (unsigned)run};
+    return ListPlan{chunk, slots, slots / 64, (unsigned)((waves + kGroup - 1) / kGroup * kXcds)};
+}
+// Partial counts per batch element, a power of two: kPartials lines each, and at most sixteen
+// times as many over the whole batch (the blocks that add to them are spread over its
+// elements; 8 lines on each of six 5,000-triangle meshes instead of 64: 273 -> 282 us).
+static int partials_of(int64_t B) {
+    int k = kPartials;
+    while (k > 1 && k * B > 16 * kPartials) k >>= 1;
+    return k;
 }
 
 template <typename T>
@@ -2473,8 +2492,11 @@ static ccc_status run_query(const Query &q) {
     DevCounters *ctr = q.ctr_ext ? q.ctr_ext : ws.get_as<DevCounters>(B);
     T *tv = moving ? ws.get_as<T>(B * n * 18) : nullptr;
     const bool ccd_query = q.narrow == Narrow::CCD_COLLECT || q.narrow == Narrow::CCD_IMPULSE;
-    DevPartial *parts = ccd_query ? ws.get_as<DevPartial>(B * kPartials) : nullptr;
-    unsigned *foreign = q.nosync ? nullptr : ws.get_as<unsigned>(B * kForeignStep);
+    // with a scratch block that may be tight the partial counts wait until the traversal's buffers are gone
+    int nparts = partials_of(B);
+    const bool late_parts = ws.arena() && !q.nosync;
+    DevPartial *parts = ccd_query && !late_parts ? ws.get_as<DevPartial>(B * nparts) : nullptr;
+    unsigned *foreign = q.nosync ? nullptr : ws.get_as<unsigned>(B);
     // from here on: what only the index tree's path uses, given back when the tree is another
     T *chunks = ws.get_as<T>(B * nc * 6);
     T *groups = ws.get_as<T>(B * nc * (kChunk / kPairQ) * 12);
@@ -2485,8 +2507,8 @@ static ccc_status run_query(const Query &q) {
     // outputs start at -1 (index rows, roots) or 0 (impulses)
     FillRegions fill;
     fill.add(ctr, B * (int64_t)sizeof(DevCounters), 0ull);
-    if (foreign) fill.add(foreign, B * kForeignStep * 4, 0ull);
-    if (parts) fill.add(parts, B * kPartials * (int64_t)sizeof(DevPartial), 0ull);
+    if (foreign) fill.add(foreign, B * 4, 0ull);
+    if (parts) fill.add(parts, B * nparts * (int64_t)sizeof(DevPartial), 0ull);
     const uint64_t minus1 = sizeof(T) == 8 ? 0xBFF0000000000000ull : 0xBF800000BF800000ull;
     const int64_t cells = B * q.out_cap, tsz = (int64_t)sizeof(T);
     switch (q.narrow) {
@@ -2563,16 +2585,20 @@ static ccc_status run_query(const Query &q) {
         if (supers) ws.release(supers);
         ws.release(groups);
         ws.release(chunks);
-        if ((st = general.prepare()) != CCC_OK) return st;
+        general.use();
     }
     for (int attempt = 0; attempt < 2; ++attempt) {
         if (q.pairs_ext) {
             pairs = q.pairs_ext;
         } else {
-            if (pairs) ws.release(pairs);     // a re-run: the first attempt's pairs are not kept
+            // a re-run: the first attempt's pairs are not kept (in an arena the walk's buffers
+            // lie behind them and go first)
+            if (general.prepared() && ws.arena()) general.release();
+            if (pairs) ws.release(pairs);
             pairs = ws.get_as<int2>(B * capK);
             if (ws.failed()) return CCC_ERR_NO_MEMORY;
         }
+        if (general.used() && !general.prepared() && (st = general.prepare()) != CCC_OK) return st;
         if (general.used()) {
             if ((st = general.traverse(pairs, capK)) != CCC_OK) return st;
         } else {
@@ -2606,12 +2632,14 @@ static ccc_status run_query(const Query &q) {
             CCC_HIP_TRY(hipMemcpyAsync(ctr, h.data(), sizeof(DevCounters) * B, hipMemcpyHostToDevice, s));
             if (flags & DEV_STACK) general.go_deep();
             else {
-                // the list follows the tree's buffers (last in, first out)
+                // last in, first out
                 if (!q.pairs_ext) { ws.release(pairs); pairs = nullptr; }
                 if (supers) ws.release(supers);
                 ws.release(groups);
                 ws.release(chunks);
-                if ((st = general.prepare()) != CCC_OK) return st;
+                ws.release(foreign);
+                foreign = nullptr;
+                general.use();
             }
             --attempt;
             continue;
@@ -2624,6 +2652,7 @@ static ccc_status run_query(const Query &q) {
         for (int64_t b = 0; b < B; ++b) h[b].cand = 0;
         CCC_HIP_TRY(hipMemcpyAsync(ctr, h.data(), sizeof(DevCounters) * B, hipMemcpyHostToDevice, s));
     }
+    if (general.prepared() && ws.arena()) general.release();      // room for the narrow phase
     int64_t kmax = 0;
     if (q.nosync) kmax = capK;        // sizes must not depend on the counts
     else
@@ -2662,6 +2691,14 @@ static ccc_status run_query(const Query &q) {
         const bool ccd = q.narrow != Narrow::PROXIMITY;
         int64_t chunk = pair_chunk_of(q.ctx, q.chunk_ext, kmax, B, item_bytes(q.narrow));
         ListPlan plan = list_plan(q.ctx, chunk, B);
+        if (ccd && late_parts) {
+            while (nparts > 1 && nparts * (int64_t)kBatch > chunk) nparts >>= 1;
+            parts = ws.get_as<DevPartial>(B * nparts);
+            if (ws.failed()) return CCC_ERR_NO_MEMORY;
+            FillRegions zero;
+            zero.add(parts, B * nparts * (int64_t)sizeof(DevPartial), 0ull);
+            if ((st = fill_regions(zero, s)) != CCC_OK) return st;
+        }
         if (ws.arena()) {
             // the item list takes what the arena has left (results do not depend on the chunk)
             if (ccd) {
@@ -2699,7 +2736,7 @@ static ccc_status run_query(const Query &q) {
                                        c0, c1, (const T *)q.t0, n, thr, items, capM, ctr);
                 else
                     hipLaunchKernelGGL((k_items<T>), dim3(plan.grid, B), dim3(64 * kItemBlock), 0, s, pairs, capK, c0, c1, (const T *)tv, n,
-                                       (uint32_t *)items, capM, plan.run, tiles, plan.tiles, parts, ctr);
+                                       (uint32_t *)items, capM, tiles, plan.tiles, parts, nparts, ctr);
                 tm.end();
                 CCC_LAUNCH_CHECK("k_subprim");
                 tm.begin(q.narrow == Narrow::PROXIMITY ? "proximity" : q.narrow == Narrow::CCD_COLLECT ? "ccd_collect" : "ccd_impulse");
@@ -2714,6 +2751,7 @@ static ccc_status run_query(const Query &q) {
                     ca.tv = tv;
                     ca.ctr = ctr;
                     ca.parts = parts;
+                    ca.nparts = nparts;
                     ca.cap_items = capM;
                     ca.cap_tiles = plan.tiles;
                     ca.cap_pairs = capK;
@@ -2744,7 +2782,7 @@ static ccc_status run_query(const Query &q) {
             }
             if (ccd) {
                 block.written();
-                hipLaunchKernelGGL(k_fold_partials, dim3(B), dim3(64), 0, s, parts, q.narrow == Narrow::CCD_IMPULSE, ctr, hp);
+                hipLaunchKernelGGL(k_fold_partials, dim3(B), dim3(64), 0, s, parts, nparts, q.narrow == Narrow::CCD_IMPULSE, ctr, hp);
                 CCC_LAUNCH_CHECK("k_fold_partials");
             }
             return CCC_OK;
@@ -2791,7 +2829,7 @@ static size_t resident_bytes(const Query &q) {
     if (!q.pairs_ext) tot += r(sizeof(int2) * B * capK);
     const int64_t chunk = pair_chunk_of(q.ctx, q.chunk_ext, capK, B, item_bytes(q.narrow));
     const ListPlan plan = list_plan(q.ctx, chunk, B);
-    tot += r(esz * B * n * 18) + r(sizeof(DevPartial) * B * kPartials) + plan.bytes(B);
+    tot += r(esz * B * n * 18) + r(sizeof(DevPartial) * B * partials_of(B)) + plan.bytes(B);
     return tot;
 }
 

@@ -729,7 +729,9 @@ template <typename T> __device__ __forceinline__ void split_union(const BoxReg<T
     float best = cost;
 #pragma unroll
     for (int d = 1; d < kPairQ; d <<= 1) best = fminf(best, __shfl_xor(best, d, kPairQ));
-    const int at = best < 0.75f * whole ? __ffsll((long long)__ballot(cost == best)) - 1 : kPairQ - 1;
+    // the wave holds 64 / kPairQ groups: of the ballot only the lane's own group's bits
+    const unsigned lowest = (unsigned)(__ballot(cost == best) >> (threadIdx.x & 63 & ~(kPairQ - 1))) & ((1u << kPairQ) - 1u);
+    const int at = best < 0.75f * whole ? __ffs(lowest) - 1 : kPairQ - 1;
     const int from = at == kPairQ - 1 ? 0 : at + 1;
 #pragma unroll
     for (int k = 0; k < 6; ++k) {
@@ -825,6 +827,8 @@ template <typename T> __device__ __forceinline__ void box_grow(BoxReg<T> &o, T t
         o.v[k + 3] = o.v[k + 3] + thr;
     }
 }
+
+static_assert(kPairQ < 32, "a group's lanes as bits of a word");
 
 // One wave per (group of kPairQ queries, split): split s of `splits` takes every splits-th
 // chunk, so that small meshes fill the chip too.  The chunks that the group's union box meets
@@ -3286,5 +3290,23 @@ extern "C" ccc_status ccc_debug_device_math(ccc_context *ctx, int what, const do
     CCC_HIP_TRY(hipSetDevice(ctx->device));
     hipLaunchKernelGGL(ccc::k_device_math, dim3(ccc::grid_for(n, 256)), dim3(256), 0, (hipStream_t)stream, what, x, y, n);
     CCC_LAUNCH_CHECK("k_device_math");
+    return CCC_OK;
+}
+
+extern "C" ccc_status ccc_debug_query_groups(ccc_context *ctx, const void *bboxes, int64_t n, int32_t dtype, void *chunks, void *groups,
+                                             void *stream) {
+    ccc::clear_error();
+    if (!ctx) return ccc::bad_arg("context is NULL");
+    if (n < 1 || n >= ((int64_t)1 << 28) || !bboxes || !chunks || !groups) return ccc::bad_arg("need n in [1, 2^28) and device arrays");
+    CCC_HIP_TRY(hipSetDevice(ctx->device));
+    const unsigned g = ccc::grid_for(n, 256);
+    if (dtype == CCC_FLOAT64)
+        hipLaunchKernelGGL((ccc::k_prep<double>), dim3(g), dim3(256), 0, (hipStream_t)stream, (const double *)bboxes, (const int64_t *)nullptr, n, 0u, g,
+                           (double *)chunks, (double *)groups, (const double *)nullptr, (const double *)nullptr, (double *)nullptr, (unsigned *)nullptr);
+    else if (dtype == CCC_FLOAT32)
+        hipLaunchKernelGGL((ccc::k_prep<float>), dim3(g), dim3(256), 0, (hipStream_t)stream, (const float *)bboxes, (const int64_t *)nullptr, n, 0u, g,
+                           (float *)chunks, (float *)groups, (const float *)nullptr, (const float *)nullptr, (float *)nullptr, (unsigned *)nullptr);
+    else return ccc::bad_arg("dtype must be CCC_FLOAT32 or CCC_FLOAT64");
+    CCC_LAUNCH_CHECK("k_prep");
     return CCC_OK;
 }

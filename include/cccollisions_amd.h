@@ -118,6 +118,12 @@ ccc_status ccc_context_set_morton(ccc_context *ctx, int mode);
  * float (x holds 2 n values), else 0. */
 ccc_status ccc_debug_device_math(ccc_context *ctx, int what, const double *x, double *y, int64_t n, void *stream);
 
+/* Test hook (no counterpart in the reference): the boxes that the candidate search groups the
+ * leaves of one mesh by.  chunks [ceil(n / 64), 6]: the union of each 64 leaf boxes;
+ * groups [4 ceil(n / 64), 2, 6]: of each 16 leaves (past the last one: copies of it), as one
+ * box twice or as the two boxes on either side of a split. */
+ccc_status ccc_debug_query_groups(ccc_context *ctx, const void *bboxes, int64_t n, int32_t dtype, void *chunks, void *groups, void *stream);
+
 /* Test hook (no counterpart in the reference): the launches by which a call clears `count`
  * buffers of the given sizes: their number, and in blocks[2i], blocks[2i + 1] the first block
  * and the number of blocks (256 work items, 4 KiB each) of launch i < capacity; -1 for what

@@ -121,8 +121,10 @@ ccc_status ccc_debug_device_math(ccc_context *ctx, int what, const double *x, do
 /* Test hook (no counterpart in the reference): the boxes that the candidate search groups the
  * leaves of one mesh by.  chunks [ceil(n / 64), 6]: the union of each 64 leaf boxes;
  * groups [4 ceil(n / 64), 2, 6]: of each 16 leaves (past the last one: copies of it), as one
- * box twice or as the two boxes on either side of a split. */
-ccc_status ccc_debug_query_groups(ccc_context *ctx, const void *bboxes, int64_t n, int32_t dtype, void *chunks, void *groups, void *stream);
+ * box twice or as the two boxes on either side of a split; with to_check [n] (or NULL) only
+ * of the leaves whose byte is set (none: an empty box). */
+ccc_status ccc_debug_query_groups(ccc_context *ctx, const void *bboxes, const uint8_t *to_check, int64_t n, int32_t dtype, void *chunks,
+                                  void *groups, void *stream);
 
 /* Test hook (no counterpart in the reference): the launches by which a call clears `count`
  * buffers of the given sizes: their number, and in blocks[2i], blocks[2i + 1] the first block

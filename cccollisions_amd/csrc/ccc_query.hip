@@ -1996,15 +1996,19 @@ __global__ void k_device_math(int what, const double *__restrict__ x, double *__
 // k_ccd's first, the collision lists being written in runs of neighbouring pairs: 105 us.
 // 64 rows in 128 slots take 143 us, 16 rows in 64 slots 120, tables kept over 128 rows 170 to
 // 190: more shares find their slots taken and probe on, or more slots are drained for the same
-// sums.  One wave per block, kRowRun rows in a row, every gridDim.x-th run, so that all waves
-// share the padding at a list's end (runs of 64, 128, 256: 105, 106, 110 us).  Meshes whose
-// corner numbers do not fit the table's 32-bit keys take the atomics one by one.
-constexpr int kRowRun = 128;
+// sums.  One wave per block takes 64 rows, and then every gridDim.x-th 64 so that all waves
+// share the padding at a list's end; the next ones are read meanwhile.  A short list is bound
+// by what one wave does in series: with 128 rows in a row 5,000 rows on 10k triangles took
+// 42 us (by single atomics 37.5), with 64 32, and lists of up to kShortRows take 32 per wave
+// (30).  Meshes whose corner numbers do not fit the table's 32-bit keys take the atomics one
+// by one.
+constexpr int64_t kShortRows = 32768;
 template <typename T, bool TABLE, bool LINES>
 __global__ __launch_bounds__(kCcdThreads) void k_from_collisions(const int64_t *__restrict__ coll_all, const T *__restrict__ roots_all,
                                                                  int64_t m, const T *__restrict__ t0_all, const T *__restrict__ t1_all,
                                                                  const T *__restrict__ masses_all, int64_t n, T *__restrict__ dv_all,
-                                                                 T *__restrict__ dx_all, int *__restrict__ cnt_all, double *__restrict__ lines_all) {
+                                                                 T *__restrict__ dx_all, int *__restrict__ cnt_all, double *__restrict__ lines_all,
+                                                                 int per_wave) {
     __shared__ __align__(16) unsigned char s_raw[TABLE ? ImpTable<T, LINES>::bytes() : 16];
     const int b = blockIdx.y, lane = threadIdx.x;
     const int64_t *coll = coll_all + (int64_t)b * m * 3;
@@ -2013,52 +2017,54 @@ __global__ __launch_bounds__(kCcdThreads) void k_from_collisions(const int64_t *
     const ImpulseOut<T> to{dv_all + (int64_t)b * n * 9, dx_all + (int64_t)b * n * 9, cnt_all + (int64_t)b * n * 3,
                            LINES ? lines_all + (int64_t)b * n * 3 * kLineWords : nullptr};
     ImpTable<T, LINES> tab = ImpTable<T, LINES>::over(s_raw);
-    for (int64_t run = (int64_t)blockIdx.x * kRowRun; run < m; run += (int64_t)gridDim.x * kRowRun) {
-        for (int64_t i = run + lane; i - lane < m && i - lane < run + kRowRun; i += kCcdThreads) {
-            int64_t x = -1, y = -1, type = -1;
-            if (i < m) { x = coll[3 * i]; y = coll[3 * i + 1]; type = coll[3 * i + 2]; }
-            const bool on = !(x < 0 || y < 0 || type < 0 || type > 14 || x >= n || y >= n);
-            if (!__any(on)) continue;
-            MTet<T> mt{};
-            T root = (T)0;
-            if (on) {
-                root = roots[i];
-                mt = gather_mtet(t0, t1, x, y, (int)type);
+    const int64_t step = (int64_t)gridDim.x * per_wave, end = lane < per_wave ? m : 0;
+    int64_t i = (int64_t)blockIdx.x * per_wave + lane, nx = -1, ny = -1, ntype = -1;   // the next row, read while one is worked on
+    if (i < end) { nx = coll[3 * i]; ny = coll[3 * i + 1]; ntype = coll[3 * i + 2]; }
+    for (; i - lane < m; i += step) {
+        const int64_t x = nx, y = ny, type = ntype;
+        nx = ny = ntype = -1;
+        if (i + step < end) { nx = coll[3 * (i + step)]; ny = coll[3 * (i + step) + 1]; ntype = coll[3 * (i + step) + 2]; }
+        const bool on = !(x < 0 || y < 0 || type < 0 || type > 14 || x >= n || y >= n);
+        if (!__any(on)) continue;
+        MTet<T> mt{};
+        T root = (T)0;
+        if (on) {
+            root = roots[i];
+            mt = gather_mtet(t0, t1, x, y, (int)type);
+        }
+        if (!TABLE) {
+            if (on) scatter_impulse(mt, (int)type, root, x, y, masses, to.dv, to.dx, to.cnt);
+            continue;
+        }
+        ImpulseParams<T> ip{};
+        if (on) {
+            T q[4];
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {
+                int side, idx;
+                type_corner((int)type, k, side, idx);
+                q[k] = masses[3 * (side ? y : x) + idx];
             }
-            if (!TABLE) {
-                if (on) scatter_impulse(mt, (int)type, root, x, y, masses, to.dv, to.dx, to.cnt);
-                continue;
-            }
-            ImpulseParams<T> ip{};
-            if (on) {
-                T q[4];
+            ip = collision_impulse(mt, (int)type, root, q);
+        }
+        for (int h = 0; h < 2; ++h) {
+            const bool mine = on && (lane >> 5) == h;
+            if (!__any(mine)) continue;
+            tab.clear(lane);
+            wave_sync();
+            if (mine) {
 #pragma unroll
                 for (int k = 0; k < 4; ++k) {
                     int side, idx;
                     type_corner((int)type, k, side, idx);
-                    q[k] = masses[3 * (side ? y : x) + idx];
+                    V3<T> imp, imd;
+                    corner_impulse(ip, (int)type, k, mt.dv[k], imp, imd);
+                    tab.add(3 * (side ? y : x) + idx, imp, imd, to);
                 }
-                ip = collision_impulse(mt, (int)type, root, q);
             }
-            for (int h = 0; h < 2; ++h) {
-                const bool mine = on && (lane >> 5) == h;
-                if (!__any(mine)) continue;
-                tab.clear(lane);
-                wave_sync();
-                if (mine) {
-#pragma unroll
-                    for (int k = 0; k < 4; ++k) {
-                        int side, idx;
-                        type_corner((int)type, k, side, idx);
-                        V3<T> imp, imd;
-                        corner_impulse(ip, (int)type, k, mt.dv[k], imp, imd);
-                        tab.add(3 * (side ? y : x) + idx, imp, imd, to);
-                    }
-                }
-                wave_sync();
-                tab.drain(lane, to);
-                wave_sync();
-            }
+            wave_sync();
+            tab.drain(lane, to);
+            wave_sync();
         }
     }
 }
@@ -2938,10 +2944,11 @@ static ccc_status from_collisions(ccc_context *ctx, const int64_t *coll, const v
     KernelTimer tm(ctx, s);
     if (m > 0) {
         tm.begin("from_collisions");
-        const unsigned g = (unsigned)std::min<int64_t>((m + kRowRun - 1) / kRowRun, 16384);
+        const int per_wave = m * B <= kShortRows ? kCcdThreads / 2 : kCcdThreads;
+        const unsigned g = (unsigned)std::min<int64_t>((m + per_wave - 1) / per_wave, 16384);
 #define CCC_ROWS(TABLE, LINES)                                                                                            \
     hipLaunchKernelGGL((k_from_collisions<T, TABLE, LINES>), dim3(g, B), dim3(kCcdThreads), 0, s, coll, (const T *)roots, \
-                       m, (const T *)t0, (const T *)t1, (const T *)masses, n, (T *)dv, (T *)dx, cnt, lines)
+                       m, (const T *)t0, (const T *)t1, (const T *)masses, n, (T *)dv, (T *)dx, cnt, lines, per_wave)
         if (lines) CCC_ROWS(true, true);
         else if (n < ((int64_t)1 << 28)) CCC_ROWS(true, false);
         else CCC_ROWS(false, false);

@@ -99,8 +99,7 @@ void *Workspace::get(size_t bytes) {
 // 6.4 to 6.9 TB/s on 1 to 6 GiB, where a loop over 8,192 blocks reached 4.3 to 5.0 and 8-byte
 // stores over 65,536 blocks 5.7; up to 50 MB they are alike.
 constexpr int64_t kFillWords = 4 * 256;     // per block
-__global__ __launch_bounds__(256) void k_fill_regions(FillRegions r, unsigned base) {
-    const unsigned block = base + blockIdx.x;
+__device__ __forceinline__ void fill_block(const FillRegions &r, unsigned block) {
     unsigned first = 0;
     int k = 0;
     while (k + 1 < r.count && block >= first + r.blocks[k]) first += r.blocks[k++];
@@ -113,6 +112,18 @@ __global__ __launch_bounds__(256) void k_fill_regions(FillRegions r, unsigned ba
         return;
     }
     for (int64_t j = i; j < i + 4 && j < f.words; ++j) p[j] = (j & 1) ? hi : lo;
+}
+__global__ __launch_bounds__(256) void k_fill_regions(FillRegions r, unsigned base) { fill_block(r, base + blockIdx.x); }
+// Every gridDim.x-th block's worth, as a block starts with a wait for its four rows: 156 MB on
+// 4,096 blocks in 30 us (8 blocks' worth in a row each: 33; 38,000 blocks of one: about 60).  What
+// lies past the chosen regions finds no words left in the last of them.
+constexpr int64_t kRowsFillBlocks = 4096;
+__global__ __launch_bounds__(256) void k_fill_by_rows(FillRegions many, FillRegions few, GivenRows g, unsigned total) {
+    const bool all = many_rows(g);
+    for (unsigned j = blockIdx.x; j < total; j += gridDim.x) {
+        if (all) fill_block(many, j);
+        else fill_block(few, j);
+    }
 }
 
 // A launch holds fewer than 2^32 work items (hip_runtime_api.h), which is 64 GiB here: larger
@@ -143,6 +154,16 @@ ccc_status fill_regions(const FillRegions &regions, hipStream_t s) {
         hipLaunchKernelGGL(k_fill_regions, dim3(blocks), dim3(256), 0, s, r, base);
     });
     CCC_LAUNCH_CHECK("fill_regions");
+    return CCC_OK;
+}
+
+ccc_status fill_by_rows(const FillRegions &many, const FillRegions &few, const GivenRows &g, hipStream_t s) {
+    FillRegions a = many, b = few;
+    const int64_t total = std::max(count_fill_blocks(a), count_fill_blocks(b));
+    if (total > INT_MAX) return bad_arg("an output of more than 8 TiB");
+    const int64_t blocks = std::min<int64_t>(total, std::max<int64_t>(kRowsFillBlocks, total / 64));
+    if (total > 0) hipLaunchKernelGGL(k_fill_by_rows, dim3((unsigned)blocks), dim3(256), 0, s, a, b, g, (unsigned)total);
+    CCC_LAUNCH_CHECK("fill_by_rows");
     return CCC_OK;
 }
 

@@ -280,6 +280,25 @@ struct FillRegions {
 };
 ccc_status fill_regions(const FillRegions &r, hipStream_t s);
 
+// Lists of given rows, -1 from each list's end on.  Whether they hold a row per triangle is only
+// known on the device: the kernels that depend on it look at the same four places.  (Rows in
+// another order than that may be taken for fewer or more than they are; both ways are right.)
+struct GivenRows {
+    const int64_t *at[4];       // all NULL: nothing depends on the rows
+};
+// B lists of m rows on meshes of n <= m triangles: at quarters of the first n, each in a quarter
+// of the lists.
+inline GivenRows given_rows(const int64_t *rows, int64_t m, int64_t n, int64_t B) {
+    GivenRows g;
+    for (int q = 0; q < 4; ++q) g.at[q] = rows + 3 * (q * B / 4 * m + ((q + 1) * n + 3) / 4 - 1);
+    return g;
+}
+__device__ __forceinline__ bool many_rows(const GivenRows &g) {
+    return (*g.at[0] >= 0) & (*g.at[1] >= 0) & (*g.at[2] >= 0) & (*g.at[3] >= 0);
+}
+// Fills `many` or `few`, as many_rows says.
+ccc_status fill_by_rows(const FillRegions &many, const FillRegions &few, const GivenRows &g, hipStream_t s);
+
 // BVH over B soups of n triangles each (t1 = NULL: static boxes) into the wire format, with
 // Morton mode `morton` (CCC_MORTON_*); arguments already validated, the device already
 // current.

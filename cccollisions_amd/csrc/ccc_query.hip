@@ -1393,13 +1393,15 @@ template <typename T> struct ImpulseOut {
 // bound by its instructions and L1 accesses, and the wider buffer costs more to clear and read
 // (122k garment scene 4.31 direct, 4.36 by lines, its updates 115 and 143 us; 130k cloth 103.7
 // and 103.9 ms).
-enum : int { SUMS_DIRECT = 0, SUMS_LINES = 1, SUMS_DET = 2 };
+enum : int { SUMS_DIRECT = 0, SUMS_LINES = 1, SUMS_DET = 2, SUMS_BY_ROWS = 3 };
 constexpr int kLineWords = kLineWordsPerCorner;
 
-template <typename T, bool LINES> struct ImpTable {
+// SUMS_BY_ROWS: in lines where the call has some (ImpulseOut::lines), else direct.
+template <typename T, int SUMS> struct ImpTable {
     int *key;
     int *count;
     T *acc;     // [slot][dv.xyz, dx.xyz]
+    __device__ static bool by_lines(const ImpulseOut<T> &to) { return SUMS == SUMS_LINES || (SUMS == SUMS_BY_ROWS && to.lines); }
 
     static constexpr size_t bytes() { return (size_t)kImpSlots * (2 * sizeof(int) + 6 * sizeof(T)); }
     __device__ static ImpTable over(unsigned char *raw) {
@@ -1439,7 +1441,7 @@ template <typename T, bool LINES> struct ImpTable {
             atomicAdd(&acc[6 * s + 4], imd.y);
             atomicAdd(&acc[6 * s + 5], imd.z);
             atomicAdd(&count[s], 1);
-        } else if (LINES) {
+        } else if (by_lines(to)) {
             double *l = to.lines + kLineWords * c;
             atomicAdd(l + 0, (double)imp.x);
             atomicAdd(l + 1, (double)imp.y);
@@ -1459,7 +1461,7 @@ template <typename T, bool LINES> struct ImpTable {
         }
     }
     __device__ void drain(int tid, const ImpulseOut<T> &to) {
-        if (LINES) {
+        if (by_lines(to)) {
             // eight lanes per slot, one line per slot
             const int word = tid & 7;
 #pragma unroll 2
@@ -1486,21 +1488,23 @@ template <typename T, bool LINES> struct ImpTable {
 };
 static_assert(kImpSlots == 1 << kImpBits, "the slot count is a power of two");
 
-// Lines -> dv, dx and cnt of every corner.
+// Lines -> dv, dx and cnt of every corner; with given rows (or none: NULL) if they were summed
+// in lines.
 template <typename T>
 __global__ void k_line_sums(const double *__restrict__ lines, int64_t corners, T *__restrict__ dv, T *__restrict__ dx,
-                            int *__restrict__ cnt) {
-    const int64_t c = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (c >= corners) return;
-    const double2 *l = reinterpret_cast<const double2 *>(lines + kLineWords * c);
-    const double2 a = l[0], b = l[1], d = l[2], e = l[3];
-    dv[3 * c + 0] = (T)a.x;
-    dv[3 * c + 1] = (T)a.y;
-    dv[3 * c + 2] = (T)b.x;
-    dx[3 * c + 0] = (T)b.y;
-    dx[3 * c + 1] = (T)d.x;
-    dx[3 * c + 2] = (T)d.y;
-    cnt[c] = (int)e.x;
+                            int *__restrict__ cnt, GivenRows given) {
+    if (given.at[0] && !many_rows(given)) return;
+    for (int64_t c = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; c < corners; c += (int64_t)gridDim.x * blockDim.x) {
+        const double2 *l = reinterpret_cast<const double2 *>(lines + kLineWords * c);
+        const double2 a = l[0], b = l[1], d = l[2], e = l[3];
+        dv[3 * c + 0] = (T)a.x;
+        dv[3 * c + 1] = (T)a.y;
+        dv[3 * c + 2] = (T)b.x;
+        dx[3 * c + 0] = (T)b.y;
+        dx[3 * c + 1] = (T)d.x;
+        dx[3 * c + 2] = (T)d.y;
+        cnt[c] = (int)e.x;
+    }
 }
 
 // The deterministic mode's per-block table: the same slots and probing as ImpTable, holding
@@ -1656,7 +1660,7 @@ template <typename T, int MODE, int SUMS>
 __global__ __launch_bounds__(kCcdThreads, MODE == MODE_IMPULSE ? (SUMS == SUMS_DET ? 3 : 4) : 5) void k_ccd(CcdArgs<T> arg) {
     constexpr int NT = kCcdThreads;     // items per tile: the lanes of the one wavefront
     constexpr bool DET = SUMS == SUMS_DET;
-    using Table = ImpTable<T, SUMS == SUMS_LINES>;
+    using Table = ImpTable<T, SUMS == SUMS_LINES ? SUMS_LINES : SUMS_DIRECT>;
     static_assert(NT == 64, "one wavefront per workgroup");
     constexpr int kRootCapT = 3 * NT;
     // the root list (phases B-C) shares its LDS with the impulse table of phase D
@@ -1997,33 +2001,51 @@ __global__ void k_device_math(int what, const double *__restrict__ x, double *__
 // 64 rows in 128 slots take 143 us, 16 rows in 64 slots 120, tables kept over 128 rows 170 to
 // 190: more shares find their slots taken and probe on, or more slots are drained for the same
 // sums.  One wave per block takes 64 rows, and then every gridDim.x-th 64 so that all waves
-// share the padding at a list's end; the next ones are read meanwhile.  A short list is bound
+// share the padding at a list's end, read up to four steps ahead.  A short list is bound
 // by what one wave does in series: with 128 rows in a row 5,000 rows on 10k triangles took
 // 42 us (by single atomics 37.5), with 64 32, and lists of up to kShortRows take 32 per wave
 // (30).  Meshes whose corner numbers do not fit the table's 32-bit keys take the atomics one
 // by one.
 constexpr int64_t kShortRows = 32768;
-template <typename T, bool TABLE, bool LINES>
+template <typename T, bool TABLE, int SUMS>
 __global__ __launch_bounds__(kCcdThreads) void k_from_collisions(const int64_t *__restrict__ coll_all, const T *__restrict__ roots_all,
                                                                  int64_t m, const T *__restrict__ t0_all, const T *__restrict__ t1_all,
                                                                  const T *__restrict__ masses_all, int64_t n, T *__restrict__ dv_all,
                                                                  T *__restrict__ dx_all, int *__restrict__ cnt_all, double *__restrict__ lines_all,
-                                                                 int per_wave) {
-    __shared__ __align__(16) unsigned char s_raw[TABLE ? ImpTable<T, LINES>::bytes() : 16];
+                                                                 int per_wave, GivenRows given) {
+    __shared__ __align__(16) unsigned char s_raw[TABLE ? ImpTable<T, SUMS>::bytes() : 16];
     const int b = blockIdx.y, lane = threadIdx.x;
     const int64_t *coll = coll_all + (int64_t)b * m * 3;
     const T *roots = roots_all + (int64_t)b * m;
     const T *t0 = t0_all + (int64_t)b * n * 9, *t1 = t1_all + (int64_t)b * n * 9, *masses = masses_all + (int64_t)b * n * 3;
-    const ImpulseOut<T> to{dv_all + (int64_t)b * n * 9, dx_all + (int64_t)b * n * 9, cnt_all + (int64_t)b * n * 3,
-                           LINES ? lines_all + (int64_t)b * n * 3 * kLineWords : nullptr};
-    ImpTable<T, LINES> tab = ImpTable<T, LINES>::over(s_raw);
+    ImpulseOut<T> to{dv_all + (int64_t)b * n * 9, dx_all + (int64_t)b * n * 9, cnt_all + (int64_t)b * n * 3,
+                     nullptr};
+    bool asked = SUMS != SUMS_BY_ROWS;      // where the sums go, looked up at the first row
+    ImpTable<T, SUMS> tab = ImpTable<T, SUMS>::over(s_raw);
+    // four rows' first columns are on their way together, so that padding is passed over at the
+    // memory's rate
     const int64_t step = (int64_t)gridDim.x * per_wave, end = lane < per_wave ? m : 0;
-    int64_t i = (int64_t)blockIdx.x * per_wave + lane, nx = -1, ny = -1, ntype = -1;   // the next row, read while one is worked on
-    if (i < end) { nx = coll[3 * i]; ny = coll[3 * i + 1]; ntype = coll[3 * i + 2]; }
-    for (; i - lane < m; i += step) {
-        const int64_t x = nx, y = ny, type = ntype;
-        nx = ny = ntype = -1;
-        if (i + step < end) { nx = coll[3 * (i + step)]; ny = coll[3 * (i + step) + 1]; ntype = coll[3 * (i + step) + 2]; }
+    int64_t x1 = -1, x2 = -1, x3 = -1, y1 = -1, type1 = -1;
+    int left = 0;
+    for (int64_t i = (int64_t)blockIdx.x * per_wave + lane; i - lane < m; i += step) {
+        int64_t x = x1, y = y1, type = type1;
+        if (left == 0) {
+            x = x1 = x2 = x3 = -1;
+            if (i < end) { x = coll[3 * i]; y = coll[3 * i + 1]; type = coll[3 * i + 2]; }
+            if (i + step < end) x1 = coll[3 * (i + step)];
+            if (i + 2 * step < end) x2 = coll[3 * (i + 2 * step)];
+            if (i + 3 * step < end) x3 = coll[3 * (i + 3 * step)];
+            left = 4;
+        } else {
+            x1 = x2;
+            x2 = x3;
+        }
+        if (--left > 0 && x1 >= 0) { y1 = coll[3 * (i + step) + 1]; type1 = coll[3 * (i + step) + 2]; }
+        if (!__any(x >= 0)) continue;
+        if (!asked) {
+            asked = true;
+            if (many_rows(given)) to.lines = lines_all + (int64_t)b * n * 3 * kLineWords;
+        }
         const bool on = !(x < 0 || y < 0 || type < 0 || type > 14 || x >= n || y >= n);
         if (!__any(on)) continue;
         MTet<T> mt{};
@@ -2885,9 +2907,9 @@ size_t resident_pass_arena_bytes(ccc_context *ctx, const ResidentPass &p) { retu
 
 ccc_status line_sums(const double *lines, int64_t corners, int32_t dtype, void *dv, void *dx, int32_t *cnt, hipStream_t s) {
     if (dtype == CCC_FLOAT64)
-        hipLaunchKernelGGL((k_line_sums<double>), dim3(grid_for(corners, 256)), dim3(256), 0, s, lines, corners, (double *)dv, (double *)dx, cnt);
+        hipLaunchKernelGGL((k_line_sums<double>), dim3(grid_for(corners, 256)), dim3(256), 0, s, lines, corners, (double *)dv, (double *)dx, cnt, GivenRows{});
     else
-        hipLaunchKernelGGL((k_line_sums<float>), dim3(grid_for(corners, 256)), dim3(256), 0, s, lines, corners, (float *)dv, (float *)dx, cnt);
+        hipLaunchKernelGGL((k_line_sums<float>), dim3(grid_for(corners, 256)), dim3(256), 0, s, lines, corners, (float *)dv, (float *)dx, cnt, GivenRows{});
     CCC_LAUNCH_CHECK("k_line_sums");
     return CCC_OK;
 }
@@ -2921,42 +2943,51 @@ static ccc_status run(const Query &q) {
     return bad_arg("dtype must be CCC_FLOAT32 or CCC_FLOAT64");
 }
 
-// Whether `rows` given rows of meshes of `n` triangles in all are summed in lines: a launch and
-// about 400 bytes of traffic per triangle more, six atomic requests per table slot less.  357k
-// rows of 2.2M (the rest padding) on 23k triangles: 104 us direct, 54 by lines.
-static bool use_lines(int64_t rows, int64_t n) { return rows >= 65536 && rows >= n; }
+// Whether `m` given rows on each of B meshes of n triangles may be summed in lines.  Lines take a
+// launch and 420 bytes of traffic per triangle more and up to six atomic requests per table
+// slot less: on 130k triangles with 16 rows each 113 us against 148 direct, with 4 84 and 102,
+// with one 82 and 87, with half of one 80 and 74; collections of a folded cloth (23k triangles,
+// 15 rows each) 48 us less.  How many rows there are the device finds out (many_rows): an empty
+// list of 8 rows per triangle takes 32 us on 130k triangles (41 when capacity alone chose
+// lines, 28 without the choice) and 93 on 1M (164, 84).
+static bool lines_pay(int64_t m, int64_t B, int64_t n) { return m * B >= 65536 && m >= n && n < ((int64_t)1 << 28); }
 
 template <typename T>
 static ccc_status from_collisions(ccc_context *ctx, const int64_t *coll, const void *roots, int64_t m, const void *t0,
                                   const void *t1, const void *masses, int64_t B, int64_t n, void *dv, void *dx, int32_t *cnt,
                                   hipStream_t s) {
     Workspace ws(ctx, s);
-    double *lines = use_lines(m * B, B * n) && n < ((int64_t)1 << 28) ? ws.try_get_as<double>(B * n * 3 * kLineWords) : nullptr;
-    FillRegions fill;
-    if (lines) fill.add(lines, B * n * 3 * kLineWords * 8, 0ull);
-    else {
-        fill.add(dv, B * n * 9 * (int64_t)sizeof(T), 0ull);
-        fill.add(dx, B * n * 9 * (int64_t)sizeof(T), 0ull);
-        fill.add(cnt, B * n * 12, 0ull);
+    double *lines = lines_pay(m, B, n) ? ws.try_get_as<double>(B * n * 3 * kLineWords) : nullptr;
+    const GivenRows given = lines ? given_rows(coll, m, n, B) : GivenRows{};
+    FillRegions direct;
+    direct.add(dv, B * n * 9 * (int64_t)sizeof(T), 0ull);
+    direct.add(dx, B * n * 9 * (int64_t)sizeof(T), 0ull);
+    direct.add(cnt, B * n * 12, 0ull);
+    ccc_status st;
+    if (lines) {
+        FillRegions many;
+        many.add(lines, B * n * 3 * kLineWords * 8, 0ull);
+        st = fill_by_rows(many, direct, given, s);
+    } else {
+        st = fill_regions(direct, s);
     }
-    const ccc_status st = fill_regions(fill, s);
     if (st != CCC_OK) return st;
     KernelTimer tm(ctx, s);
     if (m > 0) {
         tm.begin("from_collisions");
         const int per_wave = m * B <= kShortRows ? kCcdThreads / 2 : kCcdThreads;
         const unsigned g = (unsigned)std::min<int64_t>((m + per_wave - 1) / per_wave, 16384);
-#define CCC_ROWS(TABLE, LINES)                                                                                            \
-    hipLaunchKernelGGL((k_from_collisions<T, TABLE, LINES>), dim3(g, B), dim3(kCcdThreads), 0, s, coll, (const T *)roots, \
-                       m, (const T *)t0, (const T *)t1, (const T *)masses, n, (T *)dv, (T *)dx, cnt, lines, per_wave)
-        if (lines) CCC_ROWS(true, true);
-        else if (n < ((int64_t)1 << 28)) CCC_ROWS(true, false);
-        else CCC_ROWS(false, false);
+#define CCC_ROWS(TABLE, SUMS)                                                                                             \
+    hipLaunchKernelGGL((k_from_collisions<T, TABLE, SUMS>), dim3(g, B), dim3(kCcdThreads), 0, s, coll, (const T *)roots, \
+                       m, (const T *)t0, (const T *)t1, (const T *)masses, n, (T *)dv, (T *)dx, cnt, lines, per_wave, given)
+        if (lines) CCC_ROWS(true, SUMS_BY_ROWS);
+        else if (n < ((int64_t)1 << 28)) CCC_ROWS(true, SUMS_DIRECT);
+        else CCC_ROWS(false, SUMS_DIRECT);
 #undef CCC_ROWS
         tm.end();
         CCC_LAUNCH_CHECK("k_from_collisions");
         if (lines) {
-            hipLaunchKernelGGL((k_line_sums<T>), dim3(grid_for(B * n * 3, 256)), dim3(256), 0, s, lines, B * n * 3, (T *)dv, (T *)dx, cnt);
+            hipLaunchKernelGGL((k_line_sums<T>), dim3(std::min(grid_for(B * n * 3, 256), 1024u)), dim3(256), 0, s, lines, B * n * 3, (T *)dv, (T *)dx, cnt, given);
             CCC_LAUNCH_CHECK("k_line_sums");
         }
     }

@@ -251,9 +251,7 @@ __global__ void k_nodes(const T *__restrict__ bb_all, const int64_t *__restrict_
 // Four-wide view of the binary tree for the traversal.  For internal row i: the up to four
 // grandchildren of i, left to right (a child that is a leaf stands for itself), with their
 // TNode fp32 boxes as structure of arrays, refs and rightmost leaf positions; unused entries
-// (at the end) have a NaN box and rightmost INT_MIN.  Entry k > 0 starts at the leaf after
-// entry k-1's rightmost one (trees built here cover contiguous position ranges).  Testing a
-// grandchild's box without its parent's prunes nothing that matters when boxes contain their
+// (at the end) have a NaN box and rightmost INT_MIN.  Testing a grandchild's box without its parent's prunes nothing that matters when boxes contain their
 // children's (the traversal's assumption throughout: it starts below the root, and its node
 // tests are conservative fp32): a pair needs the leaf's exact box to overlap the query.  One
 // node is 128 bytes, one cache line.
@@ -361,24 +359,22 @@ template <typename T> __device__ __forceinline__ bool overlap_inward(const Box<T
 }
 
 // Start points of the traversal: the subtrees kFrontierDepth levels below the root, each
-// with its fp32 box grown outward by the threshold (as in TNode), its rightmost leaf and
-// its first leaf position.  Slot i follows the path of the bits of i from the root (1 =
-// right); a leaf reached above that depth stands for itself in the slot of its leftmost
-// path, and the other slots below it are empty (first = INT_MAX: no query enters them).
+// with its fp32 box grown outward by the threshold (as in TNode) and its rightmost leaf.  Slot
+// i follows the path of the bits of i from the root (1 = right); a leaf reached above that
+// depth stands for itself in the slot of its leftmost path, and the other slots below it are
+// empty (a NaN box: no query enters them).
 // A query runs one traversal per start point, so the launch has kFrontier times as many
 // lanes.
 struct Frontier {
     int count;               // slots in use: kFrontier, or 0 (no traversal)
     int ref[kFrontier];      // internal node index, or ~leaf position
     int rightmost[kFrontier];
-    int first[kFrontier];    // first leaf position (in-order trees; 0 otherwise); INT_MAX: empty
     float box[kFrontier][6];
 };
 
 template <typename T>
 __global__ __launch_bounds__(kFrontier) void k_frontier(const T *__restrict__ bb_all, const int64_t *__restrict__ tree_all,
-                                                      const int *__restrict__ rm_all, const int *__restrict__ lo_all, int64_t n,
-                                                      double thr, Frontier *__restrict__ fr_all, const DevCounters *__restrict__ ctr) {
+                                                      const int *__restrict__ rm_all, int64_t n, double thr, Frontier *__restrict__ fr_all, const DevCounters *__restrict__ ctr) {
     const int b = blockIdx.x, i = threadIdx.x;     // one thread per slot
     Frontier &f = fr_all[b];
     if (n < 2 || (ctr[b].flags & DEV_BAD_TREE)) {
@@ -390,8 +386,6 @@ __global__ __launch_bounds__(kFrontier) void k_frontier(const T *__restrict__ bb
     const T *bb = bb_all + (int64_t)b * rows * 6;
     const int64_t *tree = tree_all + (int64_t)b * rows * 4;
     const int *rm = rm_all + (int64_t)b * (n - 1);
-    const int *lo = lo_all + (int64_t)b * (n - 1);
-    const bool ordered = !(ctr[b].flags & DEV_UNORDERED);
     int ref = 0;            // the root row
     bool used = true;
     for (int level = 0; level < kFrontierDepth; ++level) {
@@ -405,13 +399,11 @@ __global__ __launch_bounds__(kFrontier) void k_frontier(const T *__restrict__ bb
     f.ref[i] = ref;
     if (!used) {
         f.rightmost[i] = 0;
-        f.first[i] = INT_MAX;
-        for (int k = 0; k < 3; ++k) { f.box[i][k] = INFINITY; f.box[i][k + 3] = -INFINITY; }
+        for (int k = 0; k < 6; ++k) f.box[i][k] = NAN;
         return;
     }
     const int64_t row = ref >= 0 ? ref : n - 1 + (int64_t)(~ref);
     f.rightmost[i] = ref >= 0 ? rm[ref] : ~ref;
-    f.first[i] = ref >= 0 ? (ordered ? lo[ref] : 0) : ~ref;
     for (int k = 0; k < 3; ++k) {
         f.box[i][k] = f32_down((double)bb[6 * row + k] - thr);
         f.box[i][k + 3] = f32_up((double)bb[6 * row + k + 3] + thr);
@@ -463,7 +455,6 @@ __global__ __launch_bounds__(kTravThreads) void k_traverse(const T *__restrict__
                                                            const QNode *__restrict__ qnodes_all,
                                                            const LeafRec *__restrict__ recs_all, int64_t n, T thr,
                                                            const uint8_t *__restrict__ to_check_all,
-                                                           const int32_t *__restrict__ mesh_end,
                                                            int2 *__restrict__ pairs_all, int64_t cap,
                                                            DevCounters *__restrict__ ctr_all, const Frontier *__restrict__ fr_all,
                                                            const float *__restrict__ qbox_all) {
@@ -514,7 +505,7 @@ __global__ __launch_bounds__(kTravThreads) void k_traverse(const T *__restrict__
 
     // Query setup (inactive lanes: no query; they stay in the loop below as idle lanes).
     Box<T> q{};
-    int qid = 0, lim = INT_MAX;
+    int qid = 0;
     float qx0 = 0, qy0 = 0, qz0 = 0, qx1 = 0, qy1 = 0, qz1 = 0;
     bool alive = false;
     if (active) {
@@ -523,13 +514,10 @@ __global__ __launch_bounds__(kTravThreads) void k_traverse(const T *__restrict__
         qid = recs[p].id;
         qx0 = f32_down((double)q.mn.x); qy0 = f32_down((double)q.mn.y); qz0 = f32_down((double)q.mn.z);
         qx1 = f32_up((double)q.mx.x); qy1 = f32_up((double)q.mx.y); qz1 = f32_up((double)q.mx.z);
-        // packed meshes: leaves at positions >= lim belong to later meshes
-        lim = mesh_end ? mesh_end[p] : INT_MAX;
-        // the start point itself: box, rightmost and first-leaf tests as for a child
+        // the start point itself: box and rightmost tests as for a child
         const float *fb = fr.box[s];
         alive = qx0 <= fb[3] && qx1 >= fb[0] && qy0 <= fb[4] && qy1 >= fb[1] && qz0 <= fb[5] && qz1 >= fb[2];
         if (!PARTIAL) alive = alive && fr.rightmost[s] > (int)p;
-        alive = alive && fr.first[s] < lim;
     }
     const int lane = tid & 63;
     const int sbase = fr.ref[s];
@@ -594,9 +582,6 @@ __global__ __launch_bounds__(kTravThreads) void k_traverse(const T *__restrict__
                 for (int k = 0; k < 4; ++k) {
                     bool hit = qx0 <= mxx[k] && qx1 >= mnx[k] && qy0 <= mxy[k] && qy1 >= mny[k] && qz0 <= mxz[k] && qz1 >= mnz[k];
                     if (!PARTIAL) hit = hit && rmv[k] > (int)p;
-                    // entry k starts after entry k-1's last leaf; the node itself (so entry 0)
-                    // is only entered when its first leaf is below lim
-                    if (k > 0) hit = hit && rmv[k - 1] + 1 < lim;
                     leaf[k] = hit && rf[k] < 0;
                     if (hit && rf[k] >= 0) im |= 1u << k;
                 }
@@ -2448,7 +2433,7 @@ template <typename T> class GeneralTree {
             hipLaunchKernelGGL(k_qnodes, dim3(grid_for(n - 1, 256), B), dim3(256), 0, s_, nodes, n, qnodes_, ctr_);
         }
         hipLaunchKernelGGL((k_leaf_recs<T>), dim3(grid_for(n, 256), B), dim3(256), 0, s_, bb_, q_.tree, n, recs_, ctr_);
-        hipLaunchKernelGGL((k_frontier<T>), dim3(B), dim3(kFrontier), 0, s_, bb_, q_.tree, rm, lo, n, q_.thr, frontier_, ctr_);
+        hipLaunchKernelGGL((k_frontier<T>), dim3(B), dim3(kFrontier), 0, s_, bb_, q_.tree, rm, n, q_.thr, frontier_, ctr_);
         hipLaunchKernelGGL((k_qblock_boxes<T>), dim3(nqb_, B), dim3(kTravThreads), 0, s_, bb_, n, nqb_, qbox_, ctr_);
         tm_.end();
         CCC_LAUNCH_CHECK("tree preparation");
@@ -2459,7 +2444,7 @@ template <typename T> class GeneralTree {
         tm_.begin("traverse");
 #define CCC_TRAVERSE(P, D)                                                                                                  \
     hipLaunchKernelGGL((k_traverse<T, P, D>), g, dim3(kTravThreads), 0, s_, bb_, q_.tree, qnodes_, recs_, q_.n, (T)q_.thr, \
-                       q_.to_check, q_.mesh_end, pairs, capK, ctr_, frontier_, qbox_)
+                       q_.to_check, pairs, capK, ctr_, frontier_, qbox_)
         if (q_.to_check) {
             if (deep_) CCC_TRAVERSE(true, kStackDeep);
             else CCC_TRAVERSE(true, kStackShort);
@@ -2666,7 +2651,11 @@ static ccc_status run_query(const Query &q) {
             }
             CCC_HIP_TRY(hipMemcpyAsync(ctr, h.data(), sizeof(DevCounters) * B, hipMemcpyHostToDevice, s));
             if (flags & DEV_STACK) general.go_deep();
-            else {
+            else if (q.mesh_end) {
+                // (a packed call builds its tree itself, and the walk knows of one mesh)
+                set_error("internal error: a packed batch's tree is not the index tree");
+                return CCC_ERR_BAD_TREE;
+            } else {
                 // last in, first out
                 if (!q.pairs_ext) { ws.release(pairs); pairs = nullptr; }
                 if (supers) ws.release(supers);

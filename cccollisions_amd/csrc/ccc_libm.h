@@ -139,7 +139,8 @@ template <class TAB, int K> __device__ __forceinline__ double horner(double p, d
 // result is then replaced by x; the scale is a select of constants), so that a wave runs it
 // as one straight sequence.  e = 3q + r with r in {0, 1, 2} is split as an unsigned division
 // of e + 1200 (frexp exponents lie in [-1073, 1024]), the same q and r as the floor division;
-// n / 3 = n * 43691 >> 17 below 2^17, a full-rate 24-bit product instead of a high half.
+// n / 3 = n * 43691 >> 17 as long as the product fits 32 bits (below 98,304; n is at most
+// 2,224), a full-rate 24-bit product instead of a high half.
 __device__ __forceinline__ double pm_cbrt(double x) {
     const bool special = x == 0.0 || !isfinite(x);
     int e;

@@ -251,10 +251,11 @@ __global__ void k_nodes(const T *__restrict__ bb_all, const int64_t *__restrict_
 // Four-wide view of the binary tree for the traversal.  For internal row i: the up to four
 // grandchildren of i, left to right (a child that is a leaf stands for itself), with their
 // TNode fp32 boxes as structure of arrays, refs and rightmost leaf positions; unused entries
-// (at the end) have a NaN box and rightmost INT_MIN.  Testing a grandchild's box without its parent's prunes nothing that matters when boxes contain their
-// children's (the traversal's assumption throughout: it starts below the root, and its node
-// tests are conservative fp32): a pair needs the leaf's exact box to overlap the query.  One
-// node is 128 bytes, one cache line.
+// (at the end) have a NaN box and rightmost INT_MIN.  Testing a grandchild's box without its
+// parent's prunes nothing that matters when boxes contain their children's (the traversal's
+// assumption throughout: it starts below the root, and its node tests are conservative fp32):
+// a pair needs the leaf's exact box to overlap the query.  One node is 128 bytes, one cache
+// line.
 struct alignas(16) QNode {
     float4 mnx, mny, mnz, mxx, mxy, mxz;
     int4 ref;   // >= 0 internal row, < 0 leaf at position ~ref
@@ -1608,8 +1609,6 @@ template <typename P> __device__ __forceinline__ P *opaque_ptr(P *p) {
 // but left 56% of the roots undecided and cost 16% more instructions: 110 ms; not kept.
 constexpr int kCollectFlush = 128;
 
-// Waves per SIMD asked of the compiler: the deterministic table's LDS (12.3 KB) allows only
-// 3.25 waves, and at four its registers spilled (37.28 against 37.06 ms per pass at three).
 // k_ccd's arguments, all of them, so that late_args finds them at the start of the kernel's
 // argument memory.
 template <typename T> struct CcdArgs {
@@ -1641,6 +1640,8 @@ template <typename T> __device__ __forceinline__ const __attribute__((address_sp
     return p;
 }
 
+// Waves per SIMD asked of the compiler: the deterministic table's LDS (12.3 KB) allows only
+// 3.25 waves, and at four its registers spilled (37.28 against 37.06 ms per pass at three).
 template <typename T, int MODE, int SUMS>
 __global__ __launch_bounds__(kCcdThreads, MODE == MODE_IMPULSE ? (SUMS == SUMS_DET ? 3 : 4) : 5) void k_ccd(CcdArgs<T> arg) {
     constexpr int NT = kCcdThreads;     // items per tile: the lanes of the one wavefront
@@ -1818,8 +1819,8 @@ __global__ __launch_bounds__(kCcdThreads, MODE == MODE_IMPULSE ? (SUMS == SUMS_D
     // the packed (x, y, type) form is made when the tile starts.  A tile's items are of one
     // kind (k_items), so its roots and collisions take one branch of the filter and of the
     // impulse in the whole wave, but for the roots carried over a change.
-    // tile counts in 32 bits (at most 15 * 2^28 / 64 tiles): the
-    // kernel's uniform values fill the scalar registers
+    // tile counts in 32 bits (at most 15 * 2^28 / 64 tiles): the kernel's uniform values fill
+    // the scalar registers
     const int ntiles = (int)arg.ctr[b].tiles;
     const int tper = (ntiles + kXcds - 1) / kXcds, tstep = (int)gridDim.x / kXcds;
     const int tbase = (int)(blockIdx.x % kXcds) * tper;
@@ -2762,7 +2763,7 @@ static ccc_status run_query(const Query &q) {
                     hipLaunchKernelGGL((k_items<T>), dim3(plan.grid, B), dim3(64 * kItemBlock), 0, s, pairs, capK, c0, c1, (const T *)tv, n,
                                        (uint32_t *)items, capM, tiles, plan.tiles, parts, nparts, ctr);
                 tm.end();
-                CCC_LAUNCH_CHECK("k_subprim");
+                CCC_LAUNCH_CHECK(ccd ? "k_items" : "k_subprim");
                 tm.begin(q.narrow == Narrow::PROXIMITY ? "proximity" : q.narrow == Narrow::CCD_COLLECT ? "ccd_collect" : "ccd_impulse");
                 if (q.narrow == Narrow::PROXIMITY)
                     hipLaunchKernelGGL((k_proximity<T>), dim3(gM, B), dim3(kThreads), 0, s, (const int64_t *)items, capM, (const T *)q.t0, n, thr,

@@ -75,3 +75,28 @@ def test_noalloc_with_a_list_in_pieces(ccc, oracle, capi):  # noqa: F811
             assert counts == [k]
             np.testing.assert_array_equal(_np(cnt)[0], want[2])
         assert seen == {0, CCC_ERR_NO_MEMORY}
+
+
+def test_noalloc_with_the_deep_stack(ccc, oracle, capi):  # noqa: F811
+    """A tree whose rows are numbered at random needs the walk's deep stack: in the scratch array
+    its buffers and the list are then laid out again."""
+    n = 40000
+    rng = np.random.default_rng(31)
+    c = rng.random((n, 3))
+    key = np.zeros(n, np.int64)
+    for bit in range(10):
+        for a in range(3):
+            key |= ((c[:, a] * 1024).astype(np.int64) >> bit & 1) << (3 * bit + a)
+    c = c[np.argsort(key)][:, None]
+    t0 = c + 0.01 * rng.standard_normal((n, 3, 3))
+    t1 = t0 + 0.01 * rng.standard_normal((n, 3, 3))
+    m = rng.uniform(0.5, 2.0, (n, 3))
+    bb, tree, _, _ = oracle.bvh(t0, t1)
+    args = [_t(a[None]) for a in (t0, t1, m)]
+    ref = _call(capi, capi[2], _t(bb[None]), _t(tree[None]), *args, 64)
+    bb, tree = (_t(a[None]) for a in _renumbered_internal_tree(bb, tree, 4))
+    for fn in (capi[2], capi[3]):
+        got = _call(capi, fn, bb, tree, *args, 64)
+        assert got[0] & 0xff == 0, got[5]
+        assert got[4] == ref[4] and ref[4][0][3] > 0
+        np.testing.assert_array_equal(_np(got[3]), _np(ref[3]))
